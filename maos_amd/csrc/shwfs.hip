@@ -317,6 +317,12 @@ struct OpdArgs {
     int nllt, llt_tiles;
     double llt_origx, llt_origy, llt_ox, llt_oy;
     float *llt_opd; // [nwfs][side^2]
+    // static surface [nwfs][nsa][nxsa^2] (WFS stride opdadd_ws: 0 where every
+    // WFS has the same one) and piston/tip/tilt [nwfs][3] added to the traced
+    // OPD of the subaperture points; either may be null
+    const float *opdadd;
+    long opdadd_ws;
+    const double *ptt;
     int tiles;      // a subaperture grid is tiles x tiles blocks of the kernel's NXSA
     int tworow;     // interpolate every layer from two tile rows a point (verification)
 };
@@ -423,6 +429,30 @@ __device__ __forceinline__ void screen_coord(const DevLayer &L, bool isx, int i,
     screen_wrap(L, isx, i, dout, oout, ii, ff);
 }
 
+// Static surface OPD (powfs.opdadd, maos/wfsgrad.c:228-230) and per-step
+// piston/tip/tilt (loc_add_ptt, maos/wfsgrad.c:243-256: TTM/FSM commands) of
+// one subaperture grid with origin (x0, y0):
+// opd += opdadd + ptt0 + ptt1 x + ptt2 y, x = x0 + ix dx.  Added by the
+// kernel that writes the OPD last (the ray trace, or the DM surfaces'): as a
+// pass of its own over the OPD it took 72 us of a 6 x 2820 x 32^2-point
+// step, a third of it for reading and writing the OPD again.
+struct OpdIn {
+    const float *add;  // the grid's first point, or null
+    const double *ptt; // the WFS's three values, or null
+    double x0, y0, dx;
+};
+__device__ __forceinline__ OpdIn opd_in(const float *add, long ws, const double *ptt, int iwfs, long first, double x0,
+                                        double y0, double dx) {
+    return OpdIn{add ? add + ws * iwfs + first : nullptr, ptt ? ptt + 3 * iwfs : nullptr, x0, y0, dx};
+}
+// point (ix, iy), element e of the grid's storage
+__device__ __forceinline__ float opd_add(const OpdIn &in, float v, int ix, int iy, long e) {
+    if (in.add) v += in.add[e];
+    if (in.ptt)
+        v += (float)(in.ptt[0] + in.ptt[1] * (in.x0 + in.dx * (double)ix) + in.ptt[2] * (in.y0 + in.dx * (double)iy));
+    return v;
+}
+
 // four floats at 4-byte (a screen row) and 16-byte (an LDS tile row)
 // alignment
 typedef float float4_a4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -462,7 +492,7 @@ __device__ __forceinline__ void ray_trace(const DevLayer *layers, int nps, doubl
                                           long isim, double dt, double atmscale, double ptsdx,
                                           double origx, double origy, int line, float *opd,
                                           int *cidx, float *cfrac, float *tile, double *ctab,
-                                          bool tworow, int ostride = NXSA) {
+                                          bool tworow, int ostride = NXSA, const OpdIn &in = {}) {
     static_assert(N == 64 && 2 * NXSA <= N, "one wave holds the coordinate lanes");
     constexpr int PPT = NXSA * NXSA / N;
     constexpr int TW = NXSA + 2, TS = rt_tile_stride(NXSA);
@@ -671,7 +701,22 @@ __device__ __forceinline__ void ray_trace(const DevLayer *layers, int nps, doubl
         }
     }
 #pragma unroll
-    for (int j = 0; j < PPT; j++) opd[(jb + j) * ostride + ix] = (float)atmscale * acc[j];
+    for (int j = 0; j < PPT; j++) acc[j] *= (float)atmscale;
+    // (uniform branches, so that the surface's loads are issued together)
+    if (in.add) {
+#pragma unroll
+        for (int j = 0; j < PPT; j++) {
+            if (j % 8 == 0) __builtin_amdgcn_sched_barrier(0); // (8 loads in flight: no register spills)
+            acc[j] += in.add[(jb + j) * ostride + ix];
+        }
+    }
+    if (in.ptt) {
+        const double t1 = in.ptt[1] * (in.x0 + in.dx * (double)ix), t2 = in.ptt[2];
+#pragma unroll
+        for (int j = 0; j < PPT; j++) acc[j] += (float)(in.ptt[0] + t1 + t2 * (in.y0 + in.dx * (double)(jb + j)));
+    }
+#pragma unroll
+    for (int j = 0; j < PPT; j++) opd[(jb + j) * ostride + ix] = acc[j];
 }
 
 // XCD-aware unit index: consecutive units (the WFS of one subaperture
@@ -945,7 +990,9 @@ __global__ __launch_bounds__(MX_OPD_THREADS) __attribute__((amdgpu_waves_per_eu(
         ray_trace<MX_OPD_THREADS, NXSA, DIRECT>(a.layers + W.ireal * MX_MAXLAYER, a.nps, W.hs, W.thetax, W.thetay,
                                                 W.misregx, W.misregy, 0., 0., a.isim, a.dt, a.atmscale[W.ireal],
                                                 a.ptsdx, a.ptsx[isa], a.ptsy[isa], threadIdx.x,
-                                                a.opd + ((long)iwfs * a.nsa + isa) * NXSA * NXSA, cidx, cfrac, tile, ctab, a.tworow);
+                                                a.opd + ((long)iwfs * a.nsa + isa) * NXSA * NXSA, cidx, cfrac, tile, ctab, a.tworow,
+                                                NXSA, opd_in(a.opdadd, a.opdadd_ws, a.ptt, iwfs, (long)isa * NXSA * NXSA,
+                                                             a.ptsx[isa], a.ptsy[isa], a.ptsdx));
         return;
     }
     // unit: (WFS, subaperture, tile); a subaperture grid of side NXSA * tiles
@@ -961,37 +1008,11 @@ __global__ __launch_bounds__(MX_OPD_THREADS) __attribute__((amdgpu_waves_per_eu(
                                     a.ptsx[isa] + a.ptsdx * (double)(NXSA * tx), a.ptsy[isa] + a.ptsdx * (double)(NXSA * ty),
                                     threadIdx.x,
                                     a.opd + ((long)iwfs * a.nsa + isa) * side * side + (long)ty * NXSA * side + tx * NXSA,
-                                    cidx, cfrac, tile, ctab, a.tworow, side);
-}
-
-// ------------------------------------------------------------ OPD inputs
-// Static surface OPD (powfs.opdadd, maos/wfsgrad.c:228-230) and per-step
-// piston/tip/tilt (loc_add_ptt, maos/wfsgrad.c:243-256: TTM/FSM commands)
-// added to the traced OPD of every subaperture point:
-// opd += opdadd + ptt0 + ptt1 x + ptt2 y, x = origx + ix dx.
-struct OpdAddArgs {
-    int nsa, nxsa, nwfs;
-    double dx;
-    const double *ptsx, *ptsy;
-    const float *opdadd; // [nwfs][nsa][nxsa^2] or null
-    const double *ptt;   // [nwfs][3] or null
-    float *opd;
-};
-__global__ __launch_bounds__(256) void k_opd_add(OpdAddArgs a) {
-    const long np = (long)a.nxsa * a.nxsa, total = np * a.nsa * a.nwfs;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
-        const int pt = (int)(i % np);
-        const long sw = i / np;
-        const int isa = (int)(sw % a.nsa), iwfs = (int)(sw / a.nsa);
-        float v = a.opd[i];
-        if (a.opdadd) v += a.opdadd[i];
-        if (a.ptt) {
-            const double *t = a.ptt + 3 * iwfs;
-            const double x = a.ptsx[isa] + a.dx * (double)(pt % a.nxsa), y = a.ptsy[isa] + a.dx * (double)(pt / a.nxsa);
-            v += (float)(t[0] + t[1] * x + t[2] * y);
-        }
-        a.opd[i] = v;
-    }
+                                    cidx, cfrac, tile, ctab, a.tworow, side,
+                                    opd_in(a.opdadd, a.opdadd_ws, a.ptt, iwfs,
+                                           (long)isa * side * side + (long)ty * NXSA * side + tx * NXSA,
+                                           a.ptsx[isa] + a.ptsdx * (double)(NXSA * tx),
+                                           a.ptsy[isa] + a.ptsdx * (double)(NXSA * ty), a.ptsdx));
 }
 
 // ------------------------------------------------------------ dither fold
@@ -1264,6 +1285,9 @@ struct DmArgs {
     const DevLayer *dms; // [MX_MAXREAL][MX_MAXDM]
     const DevWfs *wfs;
     float *opd;
+    const float *opdadd; // as in OpdArgs, added after the surfaces
+    long opdadd_ws;
+    const double *ptt;
 };
 __global__ __launch_bounds__(64) void k_dm_opd(DmArgs a) {
     const int unit = xcd_unit((int)blockIdx.x, a.nsa * a.nwfs);
@@ -1298,6 +1322,10 @@ __global__ __launch_bounds__(64) void k_dm_opd(DmArgs a) {
             const float v1 = fmaf(fx, r1[nx0 + 1] - r1[nx0], r1[nx0]);
             op[pt] -= fmaf(fy, v1 - v0, v0);
         }
+    }
+    if (a.opdadd || a.ptt) { // (each lane adds to the points it traced)
+        const OpdIn in = opd_in(a.opdadd, a.opdadd_ws, a.ptt, iwfs, (long)isa * n * n, a.ptsx[isa], a.ptsy[isa], a.ptsdx);
+        for (int pt = threadIdx.x; pt < n * n; pt += 64) op[pt] = opd_add(in, op[pt], pt % n, pt / n, pt);
     }
 }
 
@@ -2963,10 +2991,10 @@ struct mx_wfsgrad_s {
     GtiltArgs arg_gtilt{};
     float *d_opdadd = nullptr;        // [nwfs][nsa][nxsa^2] static surface OPD
     bool opdadd_set = false;
+    bool opdadd_same = false;         // set for all WFS together: all read the first one's
     double *d_ptt = nullptr;          // [nwfs][3] piston, tip, tilt per step
     std::vector<double> h_ptt;
     bool ptt_set = false, ptt_dirty = false;
-    OpdAddArgs arg_opdadd{};
     ZtiltArgs arg_ztilt{};
     DmArgs arg_dm{};
     // TT-dither statistics and the on-GPU matched-filter update
@@ -4056,6 +4084,26 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
         const char *e = getenv("MX_RT_TWOROW");
         o.tworow = e && atoi(e) != 0;
     }
+    // the DM surfaces (every realisation of the engine has the same count)
+    const int ndm = g_dm[0].ndm;
+    for (int r = 1; r < h->nreal; r++)
+        if (g_dm[r].ndm != ndm)
+            return set_err(MX_EINVAL, "realisation %d has %d DMs, realisation 0 %d", r, g_dm[r].ndm, ndm);
+    // static surface and tip/tilt inputs of the WFS OPD, added by the last
+    // kernel that writes it
+    if (h->ptt_set && h->ptt_dirty) {
+        HIPCHK(hipMemcpyAsync(h->d_ptt, h->h_ptt.data(), sizeof(double) * h->h_ptt.size(), hipMemcpyHostToDevice,
+                              h->stream));
+        h->ptt_dirty = false;
+    }
+    const float *opdadd = h->opdadd_set ? h->d_opdadd : nullptr;
+    const long opdadd_ws = h->opdadd_same ? 0 : h->nsa * h->nxsa * h->nxsa;
+    const double *ptt = h->ptt_set ? h->d_ptt : nullptr;
+    if (ndm == 0) {
+        o.opdadd = opdadd;
+        o.opdadd_ws = opdadd_ws;
+        o.ptt = ptt;
+    }
     // the ray trace covers a subaperture grid with tiles of 32 or 16 points
     // a side (an LLT grid is one tile of nxsa)
     const int opd_nx = h->opd_tile ? h->opd_tile : ((h->lf && h->nxsa % 32 == 0) || h->nxsa == 32 ? 32 : 16);
@@ -4247,11 +4295,6 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
         L[nl++] = {kopd,
                    dim3((unsigned)(h->nsa * h->nwfs * o.tiles * o.tiles + o.nllt)), dim3(MX_OPD_THREADS), &o};
     }
-    // the DM surfaces (every realisation of the engine has the same count)
-    const int ndm = g_dm[0].ndm;
-    for (int r = 1; r < h->nreal; r++)
-        if (g_dm[r].ndm != ndm)
-            return set_err(MX_EINVAL, "realisation %d has %d DMs, realisation 0 %d", r, g_dm[r].ndm, ndm);
     if (ndm > 0) {
         DmArgs &dm = h->arg_dm;
         dm = DmArgs{};
@@ -4265,30 +4308,10 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
         dm.dms = g_ddms;
         dm.wfs = h->d_wfs;
         dm.opd = h->d_opd;
+        dm.opdadd = opdadd;
+        dm.opdadd_ws = opdadd_ws;
+        dm.ptt = ptt;
         L[nl++] = {reinterpret_cast<const void *>(&k_dm_opd), dim3((unsigned)(h->nsa * h->nwfs)), dim3(64), &dm};
-    }
-    // static surface and tip/tilt inputs of the WFS OPD
-    const bool opdin = h->opdadd_set || h->ptt_set;
-    if (opdin) {
-        if (h->ptt_dirty) {
-            HIPCHK(hipMemcpyAsync(h->d_ptt, h->h_ptt.data(), sizeof(double) * h->h_ptt.size(), hipMemcpyHostToDevice,
-                                  h->stream));
-            h->ptt_dirty = false;
-        }
-        OpdAddArgs &q = h->arg_opdadd;
-        q = OpdAddArgs{};
-        q.nsa = (int)h->nsa;
-        q.nxsa = (int)h->nxsa;
-        q.nwfs = h->nwfs;
-        q.dx = h->cfg.dx;
-        q.ptsx = h->d_ptsx;
-        q.ptsy = h->d_ptsy;
-        q.opdadd = h->opdadd_set ? h->d_opdadd : nullptr;
-        q.ptt = h->ptt_set ? h->d_ptt : nullptr;
-        q.opd = h->d_opd;
-        const long tot = h->nsa * h->nwfs * h->nxsa * h->nxsa;
-        L[nl++] = {reinterpret_cast<const void *>(&k_opd_add), dim3((unsigned)std::min<long>((tot + 255) / 256, 65536)),
-                   dim3(256), &q};
     }
     sp.slot_opd_last = nl - 1;
     if (h->geom == 2) {
@@ -4306,7 +4329,7 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
         sp.slot_img = nl;
         L[nl++] = {reinterpret_cast<const void *>(&k_gtilt), dim3((unsigned)(2 * h->nsa)), dim3(64), &q};
         sp.nl = sp.nmain = nl;
-        sp.key = (1 << 30) | (1 << 29) | (1 << 26) | (opdin ? 1 << 28 : 0) | (ndm ? 1 << 27 : 0) | (direct ? 8 : 0) |
+        sp.key = (1 << 30) | (1 << 29) | (1 << 26) | (ndm ? 1 << 27 : 0) | (direct ? 8 : 0) |
                  (o.tiles > 1 ? 1 << 7 : 0) | (opd_nx << 8);
         sp.slot_llt = -1;
         sp.llt = false;
@@ -4330,7 +4353,7 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
         sp.slot_img = nl;
         L[nl++] = {reinterpret_cast<const void *>(&k_ztilt), dim3((unsigned)(h->nsa * h->nwfs)), dim3(64), &z};
         sp.nl = sp.nmain = nl;
-        sp.key = (1 << 30) | (1 << 29) | (opdin ? 1 << 28 : 0) | (ndm ? 1 << 27 : 0) | (direct ? 8 : 0) |
+        sp.key = (1 << 30) | (1 << 29) | (ndm ? 1 << 27 : 0) | (direct ? 8 : 0) |
                  (o.tiles > 1 ? 1 << 7 : 0) | (opd_nx << 8);
         sp.slot_llt = -1;
         sp.llt = false;
@@ -4653,7 +4676,7 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
     h->lotf_last = cur;
     if (nl > MX_MAXLAUNCH) return set_err(MX_EINVAL, "internal: %d kernels in a step", nl);
     sp.nl = nl;
-    sp.key = (1 << 30) | (opdin ? 1 << 28 : 0) | (ndm ? 1 << 27 : 0) | (N == 64 ? 1 : 0) | (llt ? 2 : 0) | (h->lf ? 4 : 0) |
+    sp.key = (1 << 30) | (ndm ? 1 << 27 : 0) | (N == 64 ? 1 : 0) | (llt ? 2 : 0) | (h->lf ? 4 : 0) |
              (direct ? 8 : 0) | (variant << 4) | (o.tiles > 1 ? 1 << 7 : 0) | (opd_nx << 8) |
              (h->lf ? h->lf_threads << 14 : 0) | (h->cfg.sigmatch == 2 ? 1 << 25 : 0) |
              ((mf || fftform) && h->d_etf2_t[0] ? 1 << 24 : 0) | (fftform ? 1 << 6 : 0) |
@@ -5348,6 +5371,7 @@ int mx_wfsgrad_set_opdadd(mx_wfsgrad_t *h, int iwfs, const double *opd) {
     for (int w = w0; w < w1; w++)
         HIPCHK(hipMemcpy(h->d_opdadd + (long)w * n, t.data(), sizeof(float) * n, hipMemcpyHostToDevice));
     h->opdadd_set = true;
+    h->opdadd_same = iwfs < 0; // the copies of the others stay current
     return MX_OK;
 }
 
