@@ -314,7 +314,7 @@ struct OpdArgs {
     // origin and launch offset; WFS w's grid is llt_tiles x llt_tiles blocks
     // of the kernel's NXSA, stored with side llt_tiles NXSA (its first llt_nx
     // rows and columns are the LLT's points)
-    int nllt, llt_tiles;
+    int nllt, llt_tiles, llt_side;
     double llt_origx, llt_origy, llt_ox, llt_oy;
     float *llt_opd; // [nwfs][side^2]
     // static surface [nwfs][nsa][nxsa^2] (WFS stride opdadd_ws: 0 where every
@@ -323,6 +323,8 @@ struct OpdArgs {
     const float *opdadd;
     long opdadd_ws;
     const double *ptt;
+    int nxsa, ndm;       // k_wfs_opd_pt: the grid's side; DM surfaces (as DmArgs.dms)
+    const DevLayer *dms;
     int tiles;      // a subaperture grid is tiles x tiles blocks of the kernel's NXSA
     int tworow;     // interpolate every layer from two tile rows a point (verification)
 };
@@ -482,10 +484,10 @@ constexpr int rt_tile_rows(int nxsa) {
 // tile-relative offsets (column, row * tile width) with the periodic wrap
 // already applied.  A tile that crosses the screen edge wraps periodically;
 // the common case that does not (a uniform test) skips the wrap arithmetic.
-// DIRECT (a grid coarser than some screen, whose footprint exceeds the
-// tile) reads the four neighbours of each point from the screen itself.
+// (A grid coarser than some screen, whose footprint exceeds the tile, takes
+// k_wfs_opd_pt instead.)
 // cidx, cfrac hold 4 NXSA entries (two layers' coordinates).
-template <int N, int NXSA, bool DIRECT>
+template <int N, int NXSA>
 __device__ __forceinline__ void ray_trace(const DevLayer *layers, int nps, double hs,
                                           double thetax, double thetay, double misregx,
                                           double misregy, double shift0x, double shift0y,
@@ -511,194 +513,159 @@ __device__ __forceinline__ void ray_trace(const DevLayer *layers, int nps, doubl
     const int ci = isx ? line : line - NXSA;
     // this lane's points: column ix of the PPT consecutive rows from jb
     const int ix = line % NXSA, jb = line / NXSA * PPT;
-    // FP64 coordinates of layer L, as (ii, ff) on the lanes [0, 2 NXSA)
-    auto coords = [&](const DevLayer &L, int &ii, float &ff) {
-        ii = 0;
-        ff = 0.f;
-        if (line < 2 * NXSA)
-            screen_coord(L, isx, ci, ihs, isx ? thetax : thetay, isx ? misregx : misregy,
-                         isx ? shift0x : shift0y, isim, dt, ptsdx, isx ? origx : origy, ii, ff);
+    // The tile is TH = KM RPI >= TW rows of TS = TW rounded up to 4
+    // floats (the padding rows and columns are loaded, never read).
+    // Lane line loads 16 bytes: row k RPI + line / LPR, columns
+    // 4 (line % LPR) .. +3, LPR lanes a row; the row step lives in the
+    // 32-bit offset and the LDS offset immediates.  Lanes past RPI LPR
+    // repeat lane 0's slot (the same value to the same address), so no
+    // load is masked.  The screen rows are 4-byte aligned only: the
+    // 16-byte loads are unaligned, which this target performs (the
+    // compiler splits them where it cannot).
+    constexpr int LPR = TS / 4, RPI = N / LPR, KM = (TW + RPI - 1) / RPI, TH = KM * RPI;
+    static_assert(TH <= rt_tile_rows(NXSA), "tile rows");
+    const bool lane_on = line < RPI * LPR;
+    const int mrow = lane_on ? line / LPR : 0, mcol = lane_on ? 4 * (line % LPR) : 0;
+    float4_a4 v[KM];
+    // Screen and tile origin of a staged layer.  A tile inside the screen
+    // is prefetched into v (its loads stay in flight until the tile is
+    // stored); one that crosses the screen edge (rare) is loaded with
+    // the periodic wrap when it is stored, so that v has one producer
+    // and the compiler need not wait for the prefetch to merge values.
+    struct Staged {
+        const float *p;
+        int nx, ny, tx0, ty0;
+        bool inside;
     };
-    if constexpr (DIRECT) {
-        for (int l = next_layer(-1); l < nps; l = next_layer(l)) {
-            const DevLayer L = layers[l];
-            __syncthreads(); // the previous layer's coordinates fully read
-            int ii;
-            float ff;
-            coords(L, ii, ff);
-            if (line < 2 * NXSA) {
-                cidx[line] = ii;
-                cfrac[line] = ff;
+    auto fetch = [&](const DevLayer &L, int tx0, int ty0) {
+        Staged t{L.p, L.nx, L.ny, tx0, ty0, tx0 <= L.nx - TS && ty0 <= L.ny - TH};
+        if (t.inside) {
+            const char *base = (const char *)(L.p + (long)ty0 * L.nx + tx0);
+            const unsigned moff = (unsigned)(mrow * L.nx + mcol) * 4u, rstep = (unsigned)(RPI * L.nx) * 4u;
+#pragma unroll
+            for (int k = 0; k < KM; k++)
+                v[k] = *(const float4_a4 *)(base + (size_t)(moff + (unsigned)k * rstep));
+        }
+        return t;
+    };
+    auto store = [&](const Staged &t) {
+        if (t.inside) {
+#pragma unroll
+            for (int k = 0; k < KM; k++) *(float4_a16 *)(tile + (k * RPI + mrow) * TS + mcol) = v[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < KM; k++)
+                if (k * RPI + mrow < TW) {
+                    int gy = t.ty0 + k * RPI + mrow;
+                    gy -= gy >= t.ny ? t.ny : 0;
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        if (mcol + q < TW) {
+                            int gx = t.tx0 + mcol + q;
+                            gx -= gx >= t.nx ? t.nx : 0;
+                            tile[(k * RPI + mrow) * TS + mcol + q] = t.p[(long)gy * t.nx + gx];
+                        }
+                }
+        }
+    };
+    // tile-relative coordinates of layer L into slot s; returns its
+    // tile origin through tx0, ty0
+    // jump: some row step of the grid is not 0 or 1 tile row (a step
+    // of one pixel rounding over a row): that layer interpolates each
+    // point from two tile rows instead of carrying the upper one
+    auto publish = [&](const DevLayer &L, int lidx, int s, int &tx0, int &ty0, bool &jump) {
+        int ii = 0;
+        float ff = 0.f;
+        if (line < 2 * NXSA) {
+            const double *m = ctab + 2 * (2 * lidx + (isx ? 0 : 1));
+            screen_wrap(L, isx, ci, m[0], m[1], ii, ff);
+        }
+        tx0 = __builtin_amdgcn_readlane(ii, 0);
+        ty0 = __builtin_amdgcn_readlane(ii, NXSA);
+        int rel = ii - (isx ? tx0 : ty0);
+        rel += rel < 0 ? (isx ? L.nx : L.ny) : 0;
+        const int prev = __shfl_up(rel, 1);
+        jump = tworow || __any(line > NXSA && line < 2 * NXSA && (rel - prev > 1 || rel < prev));
+        if (line < 2 * NXSA) {
+            cidx[s * 2 * NXSA + line] = isx ? rel : rel * TS;
+            cfrac[s * 2 * NXSA + line] = ff;
+        }
+    };
+    // grid-uniform axis maps of every layer, lane 2 l + (y axis), once
+    if (line < 2 * nps) {
+        const bool ax = (line & 1) == 0;
+        double dout, oout;
+        axis_map(layers[line >> 1], ax, ihs, ax ? thetax : thetay, ax ? misregx : misregy,
+                 ax ? shift0x : shift0y, isim, dt, ptsdx, ax ? origx : origy, dout, oout);
+        ctab[2 * line] = dout;
+        ctab[2 * line + 1] = oout;
+    }
+    __syncthreads();
+    int l = next_layer(-1), s = 0;
+    Staged cur{};
+    bool jcur = false;
+    if (l < nps) {
+        int tx0, ty0;
+        const DevLayer L0 = layers[l];
+        publish(L0, l, 0, tx0, ty0, jcur);
+        cur = fetch(L0, tx0, ty0);
+    }
+    // (also keeps the layer table loads in the loop scalar: the compiler
+    // proves them unclobbered across a barrier, not across the stores
+    // above)
+    __syncthreads();
+    while (l < nps) {
+        const int ln = next_layer(l);
+        const DevLayer L1 = layers[ln < nps ? ln : l];
+        int tx1 = 0, ty1 = 0;
+        bool jnext = false;
+        if (ln < nps) publish(L1, ln, s ^ 1, tx1, ty1, jnext); // overlaps the loads of layer l
+        __syncthreads(); // layer l-1's interpolation done with the tile
+        store(cur);
+        __syncthreads();
+        if (ln < nps) cur = fetch(L1, tx1, ty1); // in flight during the interpolation
+        // The lane's rows jb .. jb + PPT - 1 are consecutive and their
+        // tile rows advance by 0 or 1 (a step <= 1 pixel; else jump):
+        // the x-interpolated upper row of one point is the lower row of
+        // the next one that advances, so each point reads one tile row.
+        // Scheduling barriers every 4 points bound the registers that
+        // preloaded coordinates take.
+        const int *cx = cidx + s * 2 * NXSA;
+        const float *cf = cfrac + s * 2 * NXSA;
+        const float *tc = tile + cx[ix];
+        const float fx = cf[ix];
+        auto xlerp = [&](int roff) {
+            const float *t = tc + roff;
+            return fmaf(fx, t[1] - t[0], t[0]);
+        };
+        if (!jcur) {
+            int rp = cx[NXSA + jb];
+            float lo = xlerp(rp), up = xlerp(rp + TS);
+            acc[0] += fmaf(cf[NXSA + jb], up - lo, lo);
+#pragma unroll
+            for (int j = 1; j < PPT; j++) {
+                if (j % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+                const int r = cx[NXSA + jb + j];
+                const float nu = xlerp(r + TS);
+                if (r != rp) {
+                    lo = up;
+                    up = nu;
+                }
+                rp = r;
+                acc[j] += fmaf(cf[NXSA + jb + j], up - lo, lo);
             }
-            __syncthreads();
-            const int nx = L.nx, ny = L.ny;
+        } else {
 #pragma unroll
             for (int j = 0; j < PPT; j++) {
-                const int iy = jb + j;
-                const int c0 = cidx[ix], r0i = cidx[NXSA + iy];
-                const int c1 = c0 + 1 == nx ? 0 : c0 + 1, r1i = r0i + 1 == ny ? 0 : r0i + 1;
-                const float *p0 = L.p + (long)r0i * nx, *p1 = L.p + (long)r1i * nx;
-                const float fx = cfrac[ix], fy = cfrac[NXSA + iy];
-                const float r0 = fmaf(fx, p0[c1] - p0[c0], p0[c0]);
-                const float r1 = fmaf(fx, p1[c1] - p1[c0], p1[c0]);
-                acc[j] += fmaf(fy, r1 - r0, r0);
+                if (j % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+                const int r = cx[NXSA + jb + j];
+                const float lo = xlerp(r), up = xlerp(r + TS);
+                acc[j] += fmaf(cf[NXSA + jb + j], up - lo, lo);
             }
         }
-    } else {
-        // The tile is TH = KM RPI >= TW rows of TS = TW rounded up to 4
-        // floats (the padding rows and columns are loaded, never read).
-        // Lane line loads 16 bytes: row k RPI + line / LPR, columns
-        // 4 (line % LPR) .. +3, LPR lanes a row; the row step lives in the
-        // 32-bit offset and the LDS offset immediates.  Lanes past RPI LPR
-        // repeat lane 0's slot (the same value to the same address), so no
-        // load is masked.  The screen rows are 4-byte aligned only: the
-        // 16-byte loads are unaligned, which this target performs (the
-        // compiler splits them where it cannot).
-        constexpr int LPR = TS / 4, RPI = N / LPR, KM = (TW + RPI - 1) / RPI, TH = KM * RPI;
-        static_assert(TH <= rt_tile_rows(NXSA), "tile rows");
-        const bool lane_on = line < RPI * LPR;
-        const int mrow = lane_on ? line / LPR : 0, mcol = lane_on ? 4 * (line % LPR) : 0;
-        float4_a4 v[KM];
-        // Screen and tile origin of a staged layer.  A tile inside the screen
-        // is prefetched into v (its loads stay in flight until the tile is
-        // stored); one that crosses the screen edge (rare) is loaded with
-        // the periodic wrap when it is stored, so that v has one producer
-        // and the compiler need not wait for the prefetch to merge values.
-        struct Staged {
-            const float *p;
-            int nx, ny, tx0, ty0;
-            bool inside;
-        };
-        auto fetch = [&](const DevLayer &L, int tx0, int ty0) {
-            Staged t{L.p, L.nx, L.ny, tx0, ty0, tx0 <= L.nx - TS && ty0 <= L.ny - TH};
-            if (t.inside) {
-                const char *base = (const char *)(L.p + (long)ty0 * L.nx + tx0);
-                const unsigned moff = (unsigned)(mrow * L.nx + mcol) * 4u, rstep = (unsigned)(RPI * L.nx) * 4u;
-#pragma unroll
-                for (int k = 0; k < KM; k++)
-                    v[k] = *(const float4_a4 *)(base + (size_t)(moff + (unsigned)k * rstep));
-            }
-            return t;
-        };
-        auto store = [&](const Staged &t) {
-            if (t.inside) {
-#pragma unroll
-                for (int k = 0; k < KM; k++) *(float4_a16 *)(tile + (k * RPI + mrow) * TS + mcol) = v[k];
-            } else {
-#pragma unroll
-                for (int k = 0; k < KM; k++)
-                    if (k * RPI + mrow < TW) {
-                        int gy = t.ty0 + k * RPI + mrow;
-                        gy -= gy >= t.ny ? t.ny : 0;
-#pragma unroll
-                        for (int q = 0; q < 4; q++)
-                            if (mcol + q < TW) {
-                                int gx = t.tx0 + mcol + q;
-                                gx -= gx >= t.nx ? t.nx : 0;
-                                tile[(k * RPI + mrow) * TS + mcol + q] = t.p[(long)gy * t.nx + gx];
-                            }
-                    }
-            }
-        };
-        // tile-relative coordinates of layer L into slot s; returns its
-        // tile origin through tx0, ty0
-        // jump: some row step of the grid is not 0 or 1 tile row (a step
-        // of one pixel rounding over a row): that layer interpolates each
-        // point from two tile rows instead of carrying the upper one
-        auto publish = [&](const DevLayer &L, int lidx, int s, int &tx0, int &ty0, bool &jump) {
-            int ii = 0;
-            float ff = 0.f;
-            if (line < 2 * NXSA) {
-                const double *m = ctab + 2 * (2 * lidx + (isx ? 0 : 1));
-                screen_wrap(L, isx, ci, m[0], m[1], ii, ff);
-            }
-            tx0 = __builtin_amdgcn_readlane(ii, 0);
-            ty0 = __builtin_amdgcn_readlane(ii, NXSA);
-            int rel = ii - (isx ? tx0 : ty0);
-            rel += rel < 0 ? (isx ? L.nx : L.ny) : 0;
-            const int prev = __shfl_up(rel, 1);
-            jump = tworow || __any(line > NXSA && line < 2 * NXSA && (rel - prev > 1 || rel < prev));
-            if (line < 2 * NXSA) {
-                cidx[s * 2 * NXSA + line] = isx ? rel : rel * TS;
-                cfrac[s * 2 * NXSA + line] = ff;
-            }
-        };
-        // grid-uniform axis maps of every layer, lane 2 l + (y axis), once
-        if (line < 2 * nps) {
-            const bool ax = (line & 1) == 0;
-            double dout, oout;
-            axis_map(layers[line >> 1], ax, ihs, ax ? thetax : thetay, ax ? misregx : misregy,
-                     ax ? shift0x : shift0y, isim, dt, ptsdx, ax ? origx : origy, dout, oout);
-            ctab[2 * line] = dout;
-            ctab[2 * line + 1] = oout;
-        }
-        __syncthreads();
-        int l = next_layer(-1), s = 0;
-        Staged cur{};
-        bool jcur = false;
-        if (l < nps) {
-            int tx0, ty0;
-            const DevLayer L0 = layers[l];
-            publish(L0, l, 0, tx0, ty0, jcur);
-            cur = fetch(L0, tx0, ty0);
-        }
-        // (also keeps the layer table loads in the loop scalar: the compiler
-        // proves them unclobbered across a barrier, not across the stores
-        // above)
-        __syncthreads();
-        while (l < nps) {
-            const int ln = next_layer(l);
-            const DevLayer L1 = layers[ln < nps ? ln : l];
-            int tx1 = 0, ty1 = 0;
-            bool jnext = false;
-            if (ln < nps) publish(L1, ln, s ^ 1, tx1, ty1, jnext); // overlaps the loads of layer l
-            __syncthreads(); // layer l-1's interpolation done with the tile
-            store(cur);
-            __syncthreads();
-            if (ln < nps) cur = fetch(L1, tx1, ty1); // in flight during the interpolation
-            // The lane's rows jb .. jb + PPT - 1 are consecutive and their
-            // tile rows advance by 0 or 1 (a step <= 1 pixel; else jump):
-            // the x-interpolated upper row of one point is the lower row of
-            // the next one that advances, so each point reads one tile row.
-            // Scheduling barriers every 4 points bound the registers that
-            // preloaded coordinates take.
-            const int *cx = cidx + s * 2 * NXSA;
-            const float *cf = cfrac + s * 2 * NXSA;
-            const float *tc = tile + cx[ix];
-            const float fx = cf[ix];
-            auto xlerp = [&](int roff) {
-                const float *t = tc + roff;
-                return fmaf(fx, t[1] - t[0], t[0]);
-            };
-            if (!jcur) {
-                int rp = cx[NXSA + jb];
-                float lo = xlerp(rp), up = xlerp(rp + TS);
-                acc[0] += fmaf(cf[NXSA + jb], up - lo, lo);
-#pragma unroll
-                for (int j = 1; j < PPT; j++) {
-                    if (j % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-                    const int r = cx[NXSA + jb + j];
-                    const float nu = xlerp(r + TS);
-                    if (r != rp) {
-                        lo = up;
-                        up = nu;
-                    }
-                    rp = r;
-                    acc[j] += fmaf(cf[NXSA + jb + j], up - lo, lo);
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < PPT; j++) {
-                    if (j % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-                    const int r = cx[NXSA + jb + j];
-                    const float lo = xlerp(r), up = xlerp(r + TS);
-                    acc[j] += fmaf(cf[NXSA + jb + j], up - lo, lo);
-                }
-            }
-            l = ln;
-            s ^= 1;
-            jcur = jnext;
-        }
+        l = ln;
+        s ^= 1;
+        jcur = jnext;
     }
 #pragma unroll
     for (int j = 0; j < PPT; j++) acc[j] *= (float)atmscale;
@@ -961,8 +928,8 @@ constexpr int MX_TILE_MINSCREEN = 40;
 #endif
 // TILED: a subaperture grid is tiles x tiles blocks (else one block, with
 // the register budget of the one-tile case untouched).
-template <int NXSA, bool DIRECT, bool TILED>
-__global__ __launch_bounds__(MX_OPD_THREADS) __attribute__((amdgpu_waves_per_eu(DIRECT || TILED ? MX_OPD_WAVES - 1 : MX_OPD_WAVES))) void k_wfs_opd(OpdArgs a) {
+template <int NXSA, bool TILED>
+__global__ __launch_bounds__(MX_OPD_THREADS) __attribute__((amdgpu_waves_per_eu(TILED ? MX_OPD_WAVES - 1 : MX_OPD_WAVES))) void k_wfs_opd(OpdArgs a) {
     __shared__ int cidx[4 * NXSA];
     __shared__ float cfrac[4 * NXSA];
     __shared__ double ctab[4 * MX_MAXLAYER];
@@ -975,7 +942,7 @@ __global__ __launch_bounds__(MX_OPD_THREADS) __attribute__((amdgpu_waves_per_eu(
         const int lt = a.llt_tiles, lt2 = lt * lt, iw = b / lt2, t = b % lt2, tx = t % lt, ty = t / lt;
         const int side = NXSA * lt;
         const DevWfs &W = a.wfs[iw];
-        ray_trace<MX_OPD_THREADS, NXSA, DIRECT>(a.layers + W.ireal * MX_MAXLAYER, a.nps, W.hs, W.thetax - a.llt_ox / W.hs,
+        ray_trace<MX_OPD_THREADS, NXSA>(a.layers + W.ireal * MX_MAXLAYER, a.nps, W.hs, W.thetax - a.llt_ox / W.hs,
                                         W.thetay - a.llt_oy / W.hs, 0., 0., a.llt_ox, a.llt_oy, a.isim, a.dt,
                                         a.atmscale[W.ireal], a.ptsdx, a.llt_origx + a.ptsdx * (double)(NXSA * tx),
                                         a.llt_origy + a.ptsdx * (double)(NXSA * ty), threadIdx.x,
@@ -987,7 +954,7 @@ __global__ __launch_bounds__(MX_OPD_THREADS) __attribute__((amdgpu_waves_per_eu(
         const int unit = xcd_unit(b - a.nllt, a.nsa * a.nwfs);
         const int iwfs = unit % a.nwfs, isa = unit / a.nwfs;
         const DevWfs &W = a.wfs[iwfs];
-        ray_trace<MX_OPD_THREADS, NXSA, DIRECT>(a.layers + W.ireal * MX_MAXLAYER, a.nps, W.hs, W.thetax, W.thetay,
+        ray_trace<MX_OPD_THREADS, NXSA>(a.layers + W.ireal * MX_MAXLAYER, a.nps, W.hs, W.thetax, W.thetay,
                                                 W.misregx, W.misregy, 0., 0., a.isim, a.dt, a.atmscale[W.ireal],
                                                 a.ptsdx, a.ptsx[isa], a.ptsy[isa], threadIdx.x,
                                                 a.opd + ((long)iwfs * a.nsa + isa) * NXSA * NXSA, cidx, cfrac, tile, ctab, a.tworow,
@@ -1003,7 +970,7 @@ __global__ __launch_bounds__(MX_OPD_THREADS) __attribute__((amdgpu_waves_per_eu(
     const int isa = rest / T2, it = rest % T2, tx = it % a.tiles, ty = it / a.tiles;
     const DevWfs &W = a.wfs[iwfs];
     const int side = NXSA * a.tiles;
-    ray_trace<MX_OPD_THREADS, NXSA, DIRECT>(a.layers + W.ireal * MX_MAXLAYER, a.nps, W.hs, W.thetax, W.thetay, W.misregx,
+    ray_trace<MX_OPD_THREADS, NXSA>(a.layers + W.ireal * MX_MAXLAYER, a.nps, W.hs, W.thetax, W.thetay, W.misregx,
                                     W.misregy, 0., 0., a.isim, a.dt, a.atmscale[W.ireal], a.ptsdx,
                                     a.ptsx[isa] + a.ptsdx * (double)(NXSA * tx), a.ptsy[isa] + a.ptsdx * (double)(NXSA * ty),
                                     threadIdx.x,
@@ -1013,6 +980,168 @@ __global__ __launch_bounds__(MX_OPD_THREADS) __attribute__((amdgpu_waves_per_eu(
                                            (long)isa * side * side + (long)ty * NXSA * side + tx * NXSA,
                                            a.ptsx[isa] + a.ptsdx * (double)(NXSA * tx),
                                            a.ptsy[isa] + a.ptsdx * (double)(NXSA * ty), a.ptsdx));
+}
+
+// ------------------------------------------------------------ DM surfaces
+// The deformable mirrors seen by each WFS (maos/wfsgrad.c:236-242 with the
+// propdata of maos/sim_utils.c:1035-1052): every DM surface map is traced
+// onto the subaperture grids like a screen at the DM's conjugate height
+// (cone scale 1 - ht/hs, displacement ht theta + scale misreg, no wind) with
+// alpha = -1 and without wrapping: a point is used when its row lies in
+// [irows, rowdiv0) and its column in [icols, coldiv), the ranges of
+// prop_grid_block's unequal-sampling form (lib/accphi_grid_do.c:147-302),
+// so points beyond the map's last column or row are left alone.
+constexpr int MX_MAXDM = 8;
+// One DM's map onto a grid: point (ix, iy) is at (ix dxout + oxout,
+// iy dyout + oyout) of the surface and takes it inside the ranges.
+struct DmMap {
+    double dxout, dyout, oxout, oyout;
+    long icols, coldiv, irows, rowdiv;
+};
+__device__ __forceinline__ DmMap dm_map(const DevLayer &L, const DevWfs &W, double ptsdx, double x0, double y0) {
+    const double ihs = W.hs != 0. ? 1. / W.hs : 0.;
+    const double scale = 1. - L.ht * ihs;
+    DmMap m;
+    m.dxout = ptsdx * L.dx1 * scale;
+    m.dyout = ptsdx * L.dy1 * scale;
+    m.oxout = x0 * L.dx1 * scale + (L.ht * W.thetax + scale * W.misregx - L.ox) * L.dx1;
+    m.oyout = y0 * L.dy1 * scale + (L.ht * W.thetay + scale * W.misregy - L.oy) * L.dy1;
+    const double dxout1 = 1. / m.dxout, dyout1 = 1. / m.dyout;
+    const int wrapx = L.nx - 1, wrapy = L.ny - 1;
+    m.icols = m.oyout < 0 ? (long)ceil(-m.oyout * dyout1) : 0;
+    m.coldiv = (long)floor((wrapy - m.oyout) * dyout1) + 1;
+    m.irows = m.oxout < 0 ? (long)ceil(-m.oxout * dxout1) : 0;
+    m.rowdiv = (long)ceil((wrapx - m.oxout) * dxout1);
+    return m;
+}
+// v minus the surface at point (ix, iy)
+__device__ __forceinline__ float dm_sub(const DevLayer &L, const DmMap &m, float v, int ix, int iy) {
+    if (iy < m.icols || iy >= m.coldiv || ix < m.irows || ix >= m.rowdiv) return v;
+    const int wrapx = L.nx - 1, wrapy = L.ny - 1;
+    const double x = fma((double)ix, m.dxout, m.oxout), y = fma((double)iy, m.dyout, m.oyout);
+    // the ranges keep x in [0, nx-1) and y in [0, ny-1]; the clamps
+    // only catch rounding at those edges
+    const int nx0 = min(max((int)floor(x), 0), wrapx - 1), ny0 = min(max((int)floor(y), 0), wrapy);
+    const float fx = (float)(x - nx0), fy = (float)(y - ny0);
+    const float *r0 = L.p + (long)ny0 * L.nx, *r1 = L.p + (long)(ny0 == wrapy ? 0 : ny0 + 1) * L.nx;
+    const float v0 = fmaf(fx, r0[nx0 + 1] - r0[nx0], r0[nx0]);
+    const float v1 = fmaf(fx, r1[nx0 + 1] - r1[nx0], r1[nx0]);
+    return v - fmaf(fy, v1 - v0, v0);
+}
+struct DmArgs {
+    int nsa, nxsa, nwfs, ndm;
+    double ptsdx;
+    const double *ptsx, *ptsy;
+    const DevLayer *dms; // [MX_MAXREAL][MX_MAXDM]
+    const DevWfs *wfs;
+    float *opd;
+    const float *opdadd; // as in OpdArgs, added after the surfaces
+    long opdadd_ws;
+    const double *ptt;
+};
+__global__ __launch_bounds__(64) void k_dm_opd(DmArgs a) {
+    const int unit = xcd_unit((int)blockIdx.x, a.nsa * a.nwfs);
+    const int iwfs = unit % a.nwfs, isa = unit / a.nwfs;
+    const DevWfs &W = a.wfs[iwfs];
+    const int n = a.nxsa;
+    float *op = a.opd + ((long)iwfs * a.nsa + isa) * n * n;
+    for (int d = 0; d < a.ndm; d++) {
+        const DevLayer L = a.dms[W.ireal * MX_MAXDM + d];
+        if (W.hs != 0. && L.ht > W.hs) continue;
+        const DmMap m = dm_map(L, W, a.ptsdx, a.ptsx[isa], a.ptsy[isa]);
+        for (int pt = threadIdx.x; pt < n * n; pt += 64) op[pt] = dm_sub(L, m, op[pt], pt % n, pt / n);
+    }
+    if (a.opdadd || a.ptt) { // (each lane adds to the points it traced)
+        const OpdIn in = opd_in(a.opdadd, a.opdadd_ws, a.ptt, iwfs, (long)isa * n * n, a.ptsx[isa], a.ptsy[isa], a.ptsdx);
+        for (int pt = threadIdx.x; pt < n * n; pt += 64) op[pt] = opd_add(in, op[pt], pt % n, pt / n, pt);
+    }
+}
+
+// ------------------------------------------------------------ coarse grids
+// OPD of grids coarser than a screen (the low-order NGS grids at 1/16 m over
+// 1/64 m screens, or a screen under 40 pixels), whose screen footprint the
+// staged tiles of k_wfs_opd do not hold: one point per thread gathers its
+// four neighbours from every layer, and the DM surfaces and the OPD inputs
+// are applied before the one store.  Bound by the latency of the gathers, so
+// the chip is filled with points (900 blocks for one 480^2 grid) and four
+// layers' gathers are in flight per lane; the grid-uniform FP64 maps are
+// formed once per block.  One wave per 32^2 or 16^2 tile with one layer after
+// another, as the staged form has it, left most of the chip idle: 77 us for
+// the 480^2 tip-tilt grid and seven layers, whose step fell from 191 to 120 us.
+constexpr int MX_OPD_PT_THREADS = 256;
+// blocks of one grid of side n
+constexpr int pt_blocks(int n) { return (n * n + MX_OPD_PT_THREADS - 1) / MX_OPD_PT_THREADS; }
+__global__ __launch_bounds__(MX_OPD_PT_THREADS) void k_wfs_opd_pt(OpdArgs a) {
+    constexpr int G = 4; // layers in flight
+    __shared__ double map[MX_MAXLAYER][4]; // x step, x origin, y step, y origin of each traced layer
+    __shared__ DmMap dmap[MX_MAXDM];
+    const int b = (int)blockIdx.x, tid = (int)threadIdx.x;
+    const bool llt = b < a.nllt; // the LLT uplink grids come first
+    const int n = llt ? a.llt_side : a.nxsa, nb = pt_blocks(n);
+    int iwfs, isa = 0, blk;
+    if (llt) {
+        iwfs = b / nb;
+        blk = b % nb;
+    } else {
+        const int unit = xcd_unit(b - a.nllt, a.nsa * a.nwfs * nb), rest = unit / a.nwfs;
+        iwfs = unit % a.nwfs;
+        isa = rest / nb;
+        blk = rest % nb;
+    }
+    const DevWfs &W = a.wfs[iwfs];
+    const DevLayer *layers = a.layers + W.ireal * MX_MAXLAYER;
+    const double ihs = W.hs != 0. ? 1. / W.hs : 0.;
+    const double x0 = llt ? a.llt_origx : a.ptsx[isa], y0 = llt ? a.llt_origy : a.ptsy[isa];
+    if (tid < 2 * a.nps) {
+        const DevLayer &L = layers[tid >> 1];
+        const bool ax = (tid & 1) == 0;
+        const double th = ax ? W.thetax : W.thetay, lo = ax ? a.llt_ox : a.llt_oy;
+        axis_map(L, ax, ihs, llt ? th - lo / W.hs : th, llt ? 0. : (ax ? W.misregx : W.misregy), llt ? lo : 0., a.isim,
+                 a.dt, a.ptsdx, ax ? x0 : y0, map[tid >> 1][ax ? 0 : 2], map[tid >> 1][ax ? 1 : 3]);
+    }
+    const int ndm = llt ? 0 : a.ndm;
+    if (tid >= 64 && tid < 64 + ndm) dmap[tid - 64] = dm_map(a.dms[W.ireal * MX_MAXDM + tid - 64], W, a.ptsdx, x0, y0);
+    __syncthreads();
+    const int pt = blk * MX_OPD_PT_THREADS + tid;
+    if (pt >= n * n) return;
+    const int ix = pt % n, iy = pt / n;
+    float acc = 0.f;
+    for (int l0 = 0; l0 < a.nps; l0 += G) {
+        float fx[G], fy[G], q[G][4];
+#pragma unroll
+        for (int u = 0; u < G; u++) {
+            const int l = min(l0 + u, a.nps - 1); // (past the last layer: its loads again, not used)
+            const DevLayer &L = layers[l];
+            int c0, r0;
+            screen_wrap(L, true, ix, map[l][0], map[l][1], c0, fx[u]);
+            screen_wrap(L, false, iy, map[l][2], map[l][3], r0, fy[u]);
+            const int c1 = c0 + 1 == L.nx ? 0 : c0 + 1, r1 = r0 + 1 == L.ny ? 0 : r0 + 1;
+            const float *p0 = L.p + (long)r0 * L.nx, *p1 = L.p + (long)r1 * L.nx;
+            q[u][0] = p0[c0];
+            q[u][1] = p0[c1];
+            q[u][2] = p1[c0];
+            q[u][3] = p1[c1];
+        }
+#pragma unroll
+        for (int u = 0; u < G; u++) {
+            if (l0 + u >= a.nps || (W.hs != 0. && layers[l0 + u].ht > W.hs)) continue; // uniform; layers above the source
+            const float r0 = fmaf(fx[u], q[u][1] - q[u][0], q[u][0]), r1 = fmaf(fx[u], q[u][3] - q[u][2], q[u][2]);
+            acc += fmaf(fy[u], r1 - r0, r0);
+        }
+    }
+    float v = (float)a.atmscale[W.ireal] * acc;
+    const long first = (long)isa * n * n;
+    if (llt) {
+        a.llt_opd[(long)iwfs * n * n + pt] = v;
+        return;
+    }
+    for (int d = 0; d < ndm; d++) {
+        const DevLayer &L = a.dms[W.ireal * MX_MAXDM + d];
+        if (W.hs != 0. && L.ht > W.hs) continue;
+        v = dm_sub(L, dmap[d], v, ix, iy);
+    }
+    v = opd_add(opd_in(a.opdadd, a.opdadd_ws, a.ptt, iwfs, first, x0, y0, a.ptsdx), v, ix, iy, pt);
+    a.opd[((long)iwfs * a.nsa) * n * n + first + pt] = v;
 }
 
 // ------------------------------------------------------------ dither fold
@@ -1265,67 +1394,6 @@ __global__ __launch_bounds__(MX_MTCH_THREADS) void k_mtch_fin(MtchArgs a) {
             a.nea[4 * u] = a.nea[4 * u + 3] = a.nea2thres;
             a.nea[4 * u + 1] = a.nea[4 * u + 2] = 0.;
         }
-    }
-}
-
-// ------------------------------------------------------------ DM surfaces
-// The deformable mirrors seen by each WFS (maos/wfsgrad.c:236-242 with the
-// propdata of maos/sim_utils.c:1035-1052): every DM surface map is traced
-// onto the subaperture grids like a screen at the DM's conjugate height
-// (cone scale 1 - ht/hs, displacement ht theta + scale misreg, no wind) with
-// alpha = -1 and without wrapping: a point is used when its row lies in
-// [irows, rowdiv0) and its column in [icols, coldiv), the ranges of
-// prop_grid_block's unequal-sampling form (lib/accphi_grid_do.c:147-302),
-// so points beyond the map's last column or row are left alone.
-constexpr int MX_MAXDM = 8;
-struct DmArgs {
-    int nsa, nxsa, nwfs, ndm;
-    double ptsdx;
-    const double *ptsx, *ptsy;
-    const DevLayer *dms; // [MX_MAXREAL][MX_MAXDM]
-    const DevWfs *wfs;
-    float *opd;
-    const float *opdadd; // as in OpdArgs, added after the surfaces
-    long opdadd_ws;
-    const double *ptt;
-};
-__global__ __launch_bounds__(64) void k_dm_opd(DmArgs a) {
-    const int unit = xcd_unit((int)blockIdx.x, a.nsa * a.nwfs);
-    const int iwfs = unit % a.nwfs, isa = unit / a.nwfs;
-    const DevWfs &W = a.wfs[iwfs];
-    const int n = a.nxsa;
-    float *op = a.opd + ((long)iwfs * a.nsa + isa) * n * n;
-    const double ihs = W.hs != 0. ? 1. / W.hs : 0.;
-    for (int d = 0; d < a.ndm; d++) {
-        const DevLayer L = a.dms[W.ireal * MX_MAXDM + d];
-        if (W.hs != 0. && L.ht > W.hs) continue;
-        const double scale = 1. - L.ht * ihs;
-        const double dxout = a.ptsdx * L.dx1 * scale, dyout = a.ptsdx * L.dy1 * scale;
-        const double oxout = a.ptsx[isa] * L.dx1 * scale + (L.ht * W.thetax + scale * W.misregx - L.ox) * L.dx1;
-        const double oyout = a.ptsy[isa] * L.dy1 * scale + (L.ht * W.thetay + scale * W.misregy - L.oy) * L.dy1;
-        const double dxout1 = 1. / dxout, dyout1 = 1. / dyout;
-        const int wrapx = L.nx - 1, wrapy = L.ny - 1;
-        const long icols = oyout < 0 ? (long)ceil(-oyout * dyout1) : 0;
-        const long coldiv = (long)floor((wrapy - oyout) * dyout1) + 1;
-        const long irows = oxout < 0 ? (long)ceil(-oxout * dxout1) : 0;
-        const long rowdiv0 = (long)ceil((wrapx - oxout) * dxout1);
-        for (int pt = threadIdx.x; pt < n * n; pt += 64) {
-            const int ix = pt % n, iy = pt / n;
-            if (iy < icols || iy >= coldiv || ix < irows || ix >= rowdiv0) continue;
-            const double x = fma((double)ix, dxout, oxout), y = fma((double)iy, dyout, oyout);
-            // the ranges keep x in [0, nx-1) and y in [0, ny-1]; the clamps
-            // only catch rounding at those edges
-            const int nx0 = min(max((int)floor(x), 0), wrapx - 1), ny0 = min(max((int)floor(y), 0), wrapy);
-            const float fx = (float)(x - nx0), fy = (float)(y - ny0);
-            const float *r0 = L.p + (long)ny0 * L.nx, *r1 = L.p + (long)(ny0 == wrapy ? 0 : ny0 + 1) * L.nx;
-            const float v0 = fmaf(fx, r0[nx0 + 1] - r0[nx0], r0[nx0]);
-            const float v1 = fmaf(fx, r1[nx0 + 1] - r1[nx0], r1[nx0]);
-            op[pt] -= fmaf(fy, v1 - v0, v0);
-        }
-    }
-    if (a.opdadd || a.ptt) { // (each lane adds to the points it traced)
-        const OpdIn in = opd_in(a.opdadd, a.opdadd_ws, a.ptt, iwfs, (long)isa * n * n, a.ptsx[isa], a.ptsy[isa], a.ptsdx);
-        for (int pt = threadIdx.x; pt < n * n; pt += 64) op[pt] = opd_add(in, op[pt], pt % n, pt / n, pt);
     }
 }
 
@@ -1845,12 +1913,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MX_MFMA_WAV
         const int qx = wave & 1, qy = wave >> 1;
         const double o16 = t.ptsdx * 16.;
         if constexpr (UPLINK)
-            ray_trace<64, 16, false>(t.layers + W.ireal * MX_MAXLAYER, t.nps, W.hs, W.thetax - t.llt_ox / W.hs,
+            ray_trace<64, 16>(t.layers + W.ireal * MX_MAXLAYER, t.nps, W.hs, W.thetax - t.llt_ox / W.hs,
                                      W.thetay - t.llt_oy / W.hs, 0., 0., t.llt_ox, t.llt_oy, t.isim, t.dt,
                                      t.atmscale[W.ireal], t.ptsdx, t.llt_origx + o16 * qx, t.llt_origy + o16 * qy,
                                      lane, opdl + 16 * NX * qy + 16 * qx, cidx, cfrac, tile, ctab, t.tworow, NX);
         else
-            ray_trace<64, 16, false>(t.layers + W.ireal * MX_MAXLAYER, t.nps, W.hs, W.thetax, W.thetay, W.misregx,
+            ray_trace<64, 16>(t.layers + W.ireal * MX_MAXLAYER, t.nps, W.hs, W.thetax, W.thetay, W.misregx,
                                      W.misregy, 0., 0., t.isim, t.dt, t.atmscale[W.ireal], t.ptsdx,
                                      t.ptsx[isa] + o16 * qx, t.ptsy[isa] + o16 * qy, lane,
                                      opdl + 16 * NX * qy + 16 * qx, cidx, cfrac, tile, ctab, t.tworow, NX);
@@ -4099,7 +4167,12 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
     const float *opdadd = h->opdadd_set ? h->d_opdadd : nullptr;
     const long opdadd_ws = h->opdadd_same ? 0 : h->nsa * h->nxsa * h->nxsa;
     const double *ptt = h->ptt_set ? h->d_ptt : nullptr;
-    if (ndm == 0) {
+    if (direct) {
+        o.nxsa = (int)h->nxsa;
+        o.ndm = ndm;
+        o.dms = g_ddms;
+    }
+    if (ndm == 0 || direct) {
         o.opdadd = opdadd;
         o.opdadd_ws = opdadd_ws;
         o.ptt = ptt;
@@ -4109,7 +4182,9 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
     const int opd_nx = h->opd_tile ? h->opd_tile : ((h->lf && h->nxsa % 32 == 0) || h->nxsa == 32 ? 32 : 16);
     o.tiles = (int)(h->nxsa / opd_nx);
     o.llt_tiles = (int)((h->cfg.llt_nx + opd_nx - 1) / opd_nx);
-    o.nllt = llt ? h->nwfs * o.llt_tiles * o.llt_tiles : 0;
+    o.llt_side = o.llt_tiles * opd_nx;
+    const int llt_blocks = direct ? pt_blocks(o.llt_side) : o.llt_tiles * o.llt_tiles; // per LLT grid
+    o.nllt = llt ? h->nwfs * llt_blocks : 0;
     KArgs &a = h->arg_step;
     a = KArgs{};
     a.nsa = (int)h->nsa;
@@ -4265,16 +4340,10 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
     StepLaunch *L = sp.L;
     int nl = 0;
     const bool mf = variant == MX_VARIANT_MFMA_BF16 || f16;
-    const void *kopd_t[2][2][2] = {
-        {{reinterpret_cast<const void *>(&k_wfs_opd<16, false, false>),
-          reinterpret_cast<const void *>(&k_wfs_opd<16, false, true>)},
-         {reinterpret_cast<const void *>(&k_wfs_opd<16, true, false>),
-          reinterpret_cast<const void *>(&k_wfs_opd<16, true, true>)}},
-        {{reinterpret_cast<const void *>(&k_wfs_opd<32, false, false>),
-          reinterpret_cast<const void *>(&k_wfs_opd<32, false, true>)},
-         {reinterpret_cast<const void *>(&k_wfs_opd<32, true, false>),
-          reinterpret_cast<const void *>(&k_wfs_opd<32, true, true>)}}};
-    const void *kopd = kopd_t[opd_nx == 32][direct][o.tiles > 1];
+    const void *kopd_t[2][2] = {
+        {reinterpret_cast<const void *>(&k_wfs_opd<16, false>), reinterpret_cast<const void *>(&k_wfs_opd<16, true>)},
+        {reinterpret_cast<const void *>(&k_wfs_opd<32, false>), reinterpret_cast<const void *>(&k_wfs_opd<32, true>)}};
+    const void *kopd = direct ? reinterpret_cast<const void *>(&k_wfs_opd_pt) : kopd_t[opd_nx == 32][o.tiles > 1];
     // MX_FUSED=1 in the environment: the MFMA imaging and uplink kernels trace
     // their own grids (no ray-trace launch, the OPD staged in LDS), for the
     // MFMA forms on the 32-point grid without DM surfaces or OPD inputs.
@@ -4292,10 +4361,11 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
         m.opd_out = h->d_opd;
         m.llt_opd_out = h->d_llt_opd;
     } else {
-        L[nl++] = {kopd,
-                   dim3((unsigned)(h->nsa * h->nwfs * o.tiles * o.tiles + o.nllt)), dim3(MX_OPD_THREADS), &o};
+        const long nblk = direct ? pt_blocks((int)h->nxsa) : o.tiles * o.tiles; // per subaperture grid
+        L[nl++] = {kopd, dim3((unsigned)(h->nsa * h->nwfs * nblk + o.nllt)),
+                   dim3(direct ? MX_OPD_PT_THREADS : MX_OPD_THREADS), &o};
     }
-    if (ndm > 0) {
+    if (ndm > 0 && !direct) {
         DmArgs &dm = h->arg_dm;
         dm = DmArgs{};
         dm.nsa = (int)h->nsa;
@@ -4629,8 +4699,8 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
         q = o;
         q.isim = isim + 1;
         q.llt_opd = h->d_llt_opd2;
-        q.nllt = h->nwfs * o.llt_tiles * o.llt_tiles;
-        L[nl] = {kopd, dim3((unsigned)q.nllt), dim3(MX_OPD_THREADS), &q};
+        q.nllt = h->nwfs * llt_blocks;
+        L[nl] = {kopd, dim3((unsigned)q.nllt), dim3(direct ? MX_OPD_PT_THREADS : MX_OPD_THREADS), &q};
         L[nl++].dep = -1;
         if (uplink_direct) {
             LltAcorrArgs &u = h->arg_lltac_pre;
