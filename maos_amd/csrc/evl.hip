@@ -305,6 +305,31 @@ __global__ __launch_bounds__(evl_cthreads<N>()) void k_psf_cols(PsfColArgs a) {
     }
 }
 
+// Rows y0 .. y0 + ny - 1 of the mean PSF for the host: the accumulator (x
+// outer, y contiguous) transposed through LDS tiles and scaled in FP64.  The
+// host did this with a stride of one PSF row per value, 7 ms for 1024^2 of
+// them; here it is a few us and the copy to the host is what is left.
+struct PsfOutArgs {
+    const float *acc; // [P (x)][P (y)]
+    double *out;      // [ny][P]
+    int P, y0, ny;
+    double sc;
+};
+constexpr long MX_PSF_OUT = 1L << 21; // most values of one strip (16 MB, kept by the handle)
+__global__ __launch_bounds__(256) void k_psf_out(PsfOutArgs a) {
+    __shared__ float t[32][33];
+    const int x0 = (int)blockIdx.x * 32, r0 = (int)blockIdx.y * 32, tx = threadIdx.x % 32, ty = threadIdx.x / 32;
+    for (int j = ty; j < 32; j += 8) {
+        const int x = x0 + j, r = r0 + tx;
+        if (x < a.P && r < a.ny) t[j][tx] = a.acc[(long)x * a.P + a.y0 + r];
+    }
+    __syncthreads();
+    for (int j = ty; j < 32; j += 8) {
+        const int x = x0 + tx, r = r0 + j;
+        if (x < a.P && r < a.ny) a.out[(long)r * a.P + x] = (double)t[tx][j] * a.sc;
+    }
+}
+
 #define MX_STREHL_PARTS 64
 struct StrehlArgs {
     const float *opd;
@@ -514,6 +539,8 @@ struct mx_evl_s {
     double *d_amp64 = nullptr, *d_ptt = nullptr; // FP64 amplitude and p/t/t partial sums (with coordinates)
     double imcc[9] = {}, ipcc = 0;               // inverse of sum amp [1 x y]^T [1 x y], 1 / sum amp
     float2 *d_B = nullptr;
+    double *d_out = nullptr; // PSF rows on their way to the host, [out_len]
+    long out_len = 0;
     EvlWvl w[MX_MAXWVL];
     long nacc = 0;
     int ireal = 0; // realisation whose screens and DM surfaces mx_evl_trace reads
@@ -566,7 +593,8 @@ void evl_release(mx_evl_t *h) {
     if (!h) return;
     hipSetDevice(h->device);
     if (h->stream) hipStreamSynchronize(h->stream);
-    void *ptrs[] = {h->d_amp, h->d_opd, h->d_locx, h->d_locy, h->d_part, h->d_B, h->d_amp64, h->d_ptt};
+    void *ptrs[] = {h->d_amp, h->d_opd, h->d_locx, h->d_locy, h->d_part, h->d_B, h->d_amp64, h->d_ptt,
+                    h->d_out};
     for (void *p : ptrs)
         if (p) hipFree(p);
     for (int iw = 0; iw < MX_MAXWVL; iw++) {
@@ -772,6 +800,7 @@ int mx_evl_init(mx_evl_t **out, long nloc, const double *locx, const double *loc
         EVCHK(hipMemcpy(w.d_tw, tw.data(), sizeof(float2) * N, hipMemcpyHostToDevice));
         EVCHK(hipMemset(w.d_acc, 0, sizeof(float) * ndir * w.P * w.P));
         bmax = std::max(bmax, (size_t)ndir * w.nband * w.P);
+        h->out_len = std::max(h->out_len, std::min((long)w.P * w.P, std::max((long)w.P, MX_PSF_OUT)));
     }
     if (bmax && (rc = dev_alloc(&h->d_B, bmax))) return fail(rc);
     EVCHK(hipDeviceSynchronize());
@@ -913,11 +942,17 @@ int mx_evl_psf_get(mx_evl_t *h, int idir, int iwvl, double *psf, long *nacc) {
         psf[0] = v * sc;
         return MX_OK;
     }
-    const long P = w.P;
-    std::vector<float> t((size_t)P * P);
-    HIPCHK(hipMemcpy(t.data(), w.d_acc + (size_t)idir * P * P, sizeof(float) * P * P, hipMemcpyDeviceToHost));
-    for (long ix = 0; ix < P; ix++)
-        for (long iy = 0; iy < P; iy++) psf[ix + iy * P] = t[ix * P + iy] * sc;
+    // strips of rows through the handle's output buffer
+    const long P = w.P, rows = std::min(P, std::max(1L, MX_PSF_OUT / P));
+    if (const int rc = dev_alloc(&h->d_out, (size_t)h->out_len)) return rc;
+    for (long y0 = 0; y0 < P; y0 += rows) {
+        const long ny = std::min(rows, P - y0);
+        PsfOutArgs a{w.d_acc + (size_t)idir * P * P, h->d_out, (int)P, (int)y0, (int)ny, sc};
+        k_psf_out<<<dim3((unsigned)((P + 31) / 32), (unsigned)((ny + 31) / 32)), dim3(256), 0, h->stream>>>(a);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(psf + y0 * P, h->d_out, sizeof(double) * ny * P, hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(hipStreamSynchronize(h->stream));
+    }
     return MX_OK;
 }
 
