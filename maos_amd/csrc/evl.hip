@@ -390,20 +390,31 @@ __global__ __launch_bounds__(64) void k_strehl_fin(StrehlArgs a) {
 
 // Piston/tip/tilt sums of one slice of the points, FP64 (calc_ptt,
 // cuda/sim/perfevl.cu:60-103, in the FP64 form of loc_calc_ptt_stride,
-// math/loc.c:653-704): sum amp opd, amp opd x, amp opd y, amp opd^2.
+// math/loc.c:653-704): sum amp opd, amp opd x, amp opd y, amp opd^2.  Bound by
+// the 28 bytes of a point, so the slices number enough blocks to keep the
+// chip loading: 64 of them, one for four CUs, took 81 us for 2.85 M points
+// (one direction); with up to 1024 a step of that evaluation, its sums read
+// back, is 75 us shorter.
 struct PttArgs {
     const float *opd;
     const double *amp, *locx, *locy;
-    double *part; // [ndir][MX_STREHL_PARTS][4]
+    double *part; // [ndir][nparts][4]
     long nloc;
+    int nparts;
 };
+constexpr int MX_PTT_PARTS = 4096; // most slices of all directions together
+// slices of one direction: at least 1024 points each, at most 1024
+inline int ptt_parts(long nloc, int ndir) {
+    return (int)std::max(1L, std::min({(nloc + 1023) / 1024, (long)MX_PTT_PARTS / ndir, 1024L}));
+}
 __global__ __launch_bounds__(256) void k_evl_ptt(PttArgs a) {
     __shared__ double sh[4];
     const int idir = blockIdx.y, part = blockIdx.x;
-    const long per = (a.nloc + MX_STREHL_PARTS - 1) / MX_STREHL_PARTS;
+    const long per = (a.nloc + a.nparts - 1) / a.nparts;
     const long i0 = part * per, i1 = min(a.nloc, i0 + per);
     const float *op = a.opd + (long)idir * a.nloc;
     double c0 = 0, cx = 0, cy = 0, tot = 0;
+#pragma unroll 4
     for (long i = i0 + threadIdx.x; i < i1; i += 256) {
         const double o = op[i], w = a.amp[i] * o;
         c0 += w;
@@ -411,7 +422,7 @@ __global__ __launch_bounds__(256) void k_evl_ptt(PttArgs a) {
         cy += w * a.locy[i];
         tot += w * o;
     }
-    double *dst = a.part + ((long)idir * MX_STREHL_PARTS + part) * 4;
+    double *dst = a.part + ((long)idir * a.nparts + part) * 4;
     c0 = block_sum_d(c0, sh);
     cx = block_sum_d(cx, sh);
     cy = block_sum_d(cy, sh);
@@ -424,16 +435,23 @@ __global__ __launch_bounds__(256) void k_evl_ptt(PttArgs a) {
     }
 }
 
-// The four p/t/t sums of each direction from its MX_STREHL_PARTS partial
-// sums, added in part order (the order mx_evl_wfe adds them on the host, so
-// the totals are the same numbers): one thread per (direction, sum).
-__global__ __launch_bounds__(256) void k_evl_ptt_fin(const double *part, double *tot, int ndir) {
-    const int i = (int)(blockIdx.x * 256 + threadIdx.x);
-    if (i >= ndir * 4) return;
-    const int d = i / 4, k = i % 4;
+// The four p/t/t sums of each direction from its partial sums, one block per
+// direction: lane 4 q + k adds sum k of the slices q, q + 64, ... in order,
+// then the 64 lanes of a sum are added pairwise (the same order at every
+// call, so mx_evl_wfe and mx_evl_wfe_noalloc give the same numbers).  tot may
+// be host memory that the GPU maps.
+__global__ __launch_bounds__(256) void k_evl_ptt_fin(const double *part, double *tot, int nparts) {
+    __shared__ double sh[256];
+    const int tid = (int)threadIdx.x, d = (int)blockIdx.x;
     double s = 0;
-    for (int p = 0; p < MX_STREHL_PARTS; p++) s += part[((long)d * MX_STREHL_PARTS + p) * 4 + k];
-    tot[i] = s;
+    for (int p = tid / 4; p < nparts; p += 64) s += part[((long)d * nparts + p) * 4 + tid % 4];
+    sh[tid] = s;
+    __syncthreads();
+    for (int o = 128; o >= 4; o >>= 1) {
+        if (tid < o) sh[tid] += sh[tid + o];
+        __syncthreads();
+    }
+    if (tid < 4) tot[d * 4 + tid] = sh[tid];
 }
 
 // OPD of the evaluation directions on the aperture points: the screens,
@@ -537,6 +555,7 @@ struct mx_evl_s {
     float *d_amp = nullptr, *d_opd = nullptr;
     double *d_locx = nullptr, *d_locy = nullptr, *d_part = nullptr;
     double *d_amp64 = nullptr, *d_ptt = nullptr; // FP64 amplitude and p/t/t partial sums (with coordinates)
+    double *h_tot = nullptr;                     // pinned: the p/t/t sums [ndir][4], written by the GPU
     double imcc[9] = {}, ipcc = 0;               // inverse of sum amp [1 x y]^T [1 x y], 1 / sum amp
     float2 *d_B = nullptr;
     double *d_out = nullptr; // PSF rows on their way to the host, [out_len]
@@ -603,6 +622,7 @@ void evl_release(mx_evl_t *h) {
         for (void *p : q)
             if (p) hipFree(p);
     }
+    if (h->h_tot) hipHostFree(h->h_tot);
     for (hipEvent_t e : h->ev)
         if (e) hipEventDestroy(e);
     if (h->stream) hipStreamDestroy(h->stream);
@@ -724,8 +744,9 @@ int mx_evl_init(mx_evl_t **out, long nloc, const double *locx, const double *loc
         if (!(m[0] > 0)) return fail(set_err(MX_EINVAL, "mx_evl_init: the amplitudes sum to %g", m[0]));
         if (inv3x3(m, h->imcc)) return fail(set_err(MX_EINVAL, "mx_evl_init: the points span no plane"));
         h->ipcc = 1. / m[0];
-        if ((rc = dev_alloc(&h->d_amp64, nloc)) || (rc = dev_alloc(&h->d_ptt, (size_t)ndir * MX_STREHL_PARTS * 4)))
+        if ((rc = dev_alloc(&h->d_amp64, nloc)) || (rc = dev_alloc(&h->d_ptt, (size_t)ndir * ptt_parts(nloc, ndir) * 4)))
             return fail(rc);
+        EVCHK(hipHostMalloc((void **)&h->h_tot, sizeof(double) * 4 * ndir));
         EVCHK(hipMemcpy(h->d_amp64, amp, sizeof(double) * nloc, hipMemcpyHostToDevice));
     }
     size_t bmax = 0;
@@ -889,36 +910,33 @@ int mx_evl_wfe(mx_evl_t *h, double *rms, double *coeff) {
     if (!h || (!rms && !coeff)) return set_err(MX_EINVAL, "mx_evl_wfe: null argument");
     if (!h->d_ptt) return set_err(MX_ESTATE, "mx_evl_wfe: the handle was made without point coordinates");
     HIPCHK(hipSetDevice(h->device));
-    PttArgs a{h->d_opd, h->d_amp64, h->d_locx, h->d_locy, h->d_ptt, h->nloc};
-    k_evl_ptt<<<dim3(MX_STREHL_PARTS, (unsigned)h->ndir), dim3(256), 0, h->stream>>>(a);
+    const int np = ptt_parts(h->nloc, h->ndir);
+    PttArgs a{h->d_opd, h->d_amp64, h->d_locx, h->d_locy, h->d_ptt, h->nloc, np};
+    k_evl_ptt<<<dim3((unsigned)np, (unsigned)h->ndir), dim3(256), 0, h->stream>>>(a);
+    k_evl_ptt_fin<<<dim3((unsigned)h->ndir), dim3(256), 0, h->stream>>>(h->d_ptt, h->h_tot, np);
     HIPCHK(hipGetLastError());
-    std::vector<double> part((size_t)h->ndir * MX_STREHL_PARTS * 4);
-    HIPCHK(hipMemcpyAsync(part.data(), h->d_ptt, sizeof(double) * part.size(), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
-    std::vector<double> sums((size_t)h->ndir * 4, 0.);
-    for (int d = 0; d < h->ndir; d++)
-        for (int p = 0; p < MX_STREHL_PARTS; p++)
-            for (int k = 0; k < 4; k++) sums[d * 4 + k] += part[((size_t)d * MX_STREHL_PARTS + p) * 4 + k];
-    wfe_post(h, sums.data(), rms, coeff);
+    wfe_post(h, h->h_tot, rms, coeff);
     return MX_OK;
 }
 
 int mx_evl_wfe_noalloc(mx_evl_t *h, const float *d_opd, double *rms, double *coeff) {
     if (!h || !d_opd || (!rms && !coeff)) return set_err(MX_EINVAL, "mx_evl_wfe_noalloc: null argument");
     if (!h->d_amp64) return set_err(MX_ESTATE, "mx_evl_wfe_noalloc: the handle was made without point coordinates");
-    if ((long)h->ndir * (MX_STREHL_PARTS + 1) * 4 > MX_SCRATCH_DOUBLES)
+    const int np = ptt_parts(h->nloc, h->ndir);
+    if ((long)h->ndir * (np + 1) * 4 > MX_SCRATCH_DOUBLES)
         return set_err(MX_EINVAL, "mx_evl_wfe_noalloc: %d directions need more than the %d-double scratch array",
                        h->ndir, MX_SCRATCH_DOUBLES);
     HIPCHK(hipSetDevice(h->device));
     double *sc = nullptr;
     if (const int rc = scratch_on(h->device, &sc)) return rc;
-    // scratch: partial sums [ndir][MX_STREHL_PARTS][4], then totals [ndir][4];
-    // every entry read is written first by this call
-    double *part = sc, *tot = sc + (size_t)h->ndir * MX_STREHL_PARTS * 4;
-    PttArgs a{d_opd, h->d_amp64, h->d_locx, h->d_locy, part, h->nloc};
-    k_evl_ptt<<<dim3(MX_STREHL_PARTS, (unsigned)h->ndir), dim3(256), 0, h->stream>>>(a);
+    // scratch: partial sums [ndir][np][4], then totals [ndir][4]; every entry
+    // read is written first by this call
+    double *part = sc, *tot = sc + (size_t)h->ndir * np * 4;
+    PttArgs a{d_opd, h->d_amp64, h->d_locx, h->d_locy, part, h->nloc, np};
+    k_evl_ptt<<<dim3((unsigned)np, (unsigned)h->ndir), dim3(256), 0, h->stream>>>(a);
     HIPCHK(hipGetLastError());
-    k_evl_ptt_fin<<<dim3((unsigned)((h->ndir * 4 + 255) / 256)), dim3(256), 0, h->stream>>>(part, tot, h->ndir);
+    k_evl_ptt_fin<<<dim3((unsigned)h->ndir), dim3(256), 0, h->stream>>>(part, tot, np);
     HIPCHK(hipGetLastError());
     double sums[MX_EVL_MAXDIR * 4];
     HIPCHK(hipMemcpyAsync(sums, tot, sizeof(double) * 4 * h->ndir, hipMemcpyDeviceToHost, h->stream));

@@ -3132,7 +3132,7 @@ int g_device = 0;
 // held until the process ends.  On the host, `scratch` names a host-side
 // stand-in, not device memory: kernels and copies take the device address
 // that hipGetSymbolAddress returns for the current GPU (g_scratch_dev).
-constexpr int MX_SCRATCH_DOUBLES = 16640; // 130 KiB: 64 directions x (64 partial + 1 total) x 4 sums
+constexpr int MX_SCRATCH_DOUBLES = 16640; // 130 KiB: (4096 partial + 64 total) x 4 sums: 64 directions, at most 4096 slices together
 constexpr int MX_SCRATCH_MAXDEV = 64;
 static __device__ __align__(256) double scratch[MX_SCRATCH_DOUBLES];
 double *g_scratch_dev[MX_SCRATCH_MAXDEV] = {};
