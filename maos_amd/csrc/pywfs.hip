@@ -17,6 +17,120 @@
 // tiled transpose, and a second line pass; the orientation alternates so
 // that each pass reads and writes whole rows.  Layouts are [row][column]
 // with the column contiguous; "transposed" arrays hold [x][y].
+constexpr int MX_LF_MAXRAD = 12;
+constexpr int MX_LF_LDS = 4352;    // complex elements of one LDS line buffer
+// LDS position of element e of a line: one pad element after every 32, so
+// that the power-of-two write strides of the early Stockham stages spread
+// over the LDS banks
+__host__ __device__ constexpr int lf_pos(int e) { return e + (e >> 5); }
+// LDS stride of lines of length n: the padded length, made odd
+__host__ __device__ constexpr int lf_stride(int n) { return lf_pos(n) | 1; }
+// lines of length n per block: a power of two <= 32 that one buffer holds;
+// for lines of 768 and more at most 2048 / n of them, so that a one-chain
+// plane (the 960^2 and 1024^2 tip-tilt sizes: 2 lines, 480-512 blocks)
+// spreads over more blocks than CUs (53 -> 46 us per step for the 1024^2
+// tip-tilt imaging; the 512^2 planes, with many chains, keep 8 lines)
+__host__ __device__ constexpr int pyl_lines(int n) {
+    int L = 32;
+    while (L > 1 && (L * lf_stride(n) > MX_LF_LDS || (n >= 768 && L * n > 2048))) L /= 2;
+    return L;
+}
+// radix of stage s in the plan of n (radix 8 first, then 4, 2, 3, 5, 7); 0
+// past the last stage or if n has another prime factor
+__host__ __device__ constexpr int lf_radix(int n, int s) {
+    const int rad[6] = {8, 4, 2, 3, 5, 7};
+    int r = n, c = 0;
+    for (int k = 0; k < 6; k++)
+        while (r > 1 && r % rad[k] == 0) {
+            if (c == s) return rad[k];
+            c++;
+            r /= rad[k];
+        }
+    return 0;
+}
+
+struct LfPlan {
+    int n, nrad;
+    int rad[MX_LF_MAXRAD]; // lf_radix(n, s)
+    int off[MX_LF_MAXRAD]; // twiddle offset of each stage
+    const float2 *tw;      // stage s: exp(-2 pi i r k / (Ns R)) at off[s] + k (R-1) + r-1
+};
+// a / b: by the compiler when b is a constant (CT), else by qdiv
+template <bool CT>
+__device__ __forceinline__ int ldiv(int a, int b, float rb) {
+    if constexpr (CT) return a / b;
+    else return qdiv(a, b, rb);
+}
+
+// One Stockham stage of radix R and span Ns over L lines (line l at l S,
+// element e at lf_pos(e)) by a block of T threads: item (l, j), j < n/R,
+// takes x[j + r n/R] times w^(r k) (w = exp(-+ 2 pi i / (Ns R)), k = j % Ns),
+// transforms and writes x'[(j/Ns) Ns R + k + r Ns].  CT: n, Ns and L are
+// compile-time constants.  Forward is FFTW_FORWARD (exp(-i ...)).
+template <int R, bool INV, bool CT, int T>
+__device__ __forceinline__ void lds_stage(const float2 *src, float2 *dst, int n, int Ns, int L, int S,
+                                          const float2 *tw) {
+    const int nb = n / R, total = L * nb;
+    const float rnb = 1.f / (float)nb, rns = 1.f / (float)Ns;
+    for (int it = (int)threadIdx.x; it < total; it += T) {
+        const int l = ldiv<CT>(it, nb, rnb), j = it - l * nb;
+        const int g = ldiv<CT>(j, Ns, rns), k = j - g * Ns;
+        const float2 *x = src + l * S;
+        const float2 *w = tw + k * (R - 1);
+        float2 v[R];
+        v[0] = x[lf_pos(j)];
+#pragma unroll
+        for (int r = 1; r < R; r++) {
+            float2 wr = w[r - 1];
+            if (INV) wr.y = -wr.y;
+            v[r] = cmul(x[lf_pos(j + r * nb)], wr);
+        }
+        small_dft<R>(v, INV ? 1.f : -1.f);
+        float2 *y = dst + l * S;
+        const int d = g * Ns * R + k;
+#pragma unroll
+        for (int r = 0; r < R; r++) y[lf_pos(d + r * Ns)] = v[r];
+    }
+}
+
+// Stockham autosort FFT of L lines of length P.n in src; returns the buffer
+// that holds the result (src or dst).  Stages from the plan at run time.
+template <bool INV, int T>
+__device__ float2 *lds_fft_rt(float2 *src, float2 *dst, const LfPlan &P, int L, int S) {
+    int Ns = 1;
+    for (int s = 0; s < P.nrad; s++) {
+        const int R = P.rad[s];
+        const float2 *tw = P.tw + P.off[s];
+        if (R == 8) lds_stage<8, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
+        else if (R == 4) lds_stage<4, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
+        else if (R == 2) lds_stage<2, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
+        else if (R == 3) lds_stage<3, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
+        else if (R == 5) lds_stage<5, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
+        else lds_stage<7, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
+        __syncthreads();
+        float2 *t = src;
+        src = dst;
+        dst = t;
+        Ns *= R;
+    }
+    return src;
+}
+// twiddles exp(-2 pi i r k / (Ns R)) of a plan's stages (k < Ns, 1 <= r <
+// R) appended to tw; sets P.off relative to the plan's first entry
+inline void lf_twiddles(LfPlan &P, std::vector<float2> &tw) {
+    const size_t base = tw.size();
+    int Ns = 1;
+    for (int s = 0; s < P.nrad; s++) {
+        const int R = P.rad[s];
+        P.off[s] = (int)(tw.size() - base);
+        for (int k = 0; k < Ns; k++)
+            for (int r = 1; r < R; r++) {
+                const double ang = -2. * M_PI * (double)(r * k) / (double)(Ns * R);
+                tw.push_back(make_float2((float)std::cos(ang), (float)std::sin(ang)));
+            }
+        Ns *= R;
+    }
+}
 constexpr int MX_PY_MAXN = 4096;
 constexpr int MX_PY_T = 1024;
 constexpr int MX_PY_MAXSIDE = 4;
@@ -305,7 +419,7 @@ int py_rows(mx_pywfs_t *h, int mode, PyRowArgs a, int nrows) {
     a.plan.tw = h->d_tw;
     a.n = (int)h->n;
     a.S = lf_stride(a.n);
-    a.L = lf_lines(a.n);
+    a.L = pyl_lines(a.n);
     a.nrows = nrows;
     const dim3 grid((unsigned)((nrows + a.L - 1) / a.L)), block(MX_PY_T);
     const size_t lds = sizeof(float2) * 2 * (size_t)a.L * a.S; // two line buffers, <= 2 MX_LF_LDS complex

@@ -2170,6 +2170,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MX_MFMA_WAV
 }
 
 #include "shwfs_fft.hip"
+#include "linefft.hip"
 
 // psfout of wfsints (maos/wfsints.c:243-253; GPU form cuda/sim/wfsints.cu:
 // 443-450): the complex PSF scaled by norm_psf / nwvf^2 and transformed
@@ -2258,72 +2259,49 @@ __global__ __launch_bounds__(256) void k_llt_acorr(LltAcorrArgs a) {
 }
 
 // ------------------------------------------------------------ large fields
-// Fields larger than the one-workgroup subaperture forms hold: nwvf and notf
-// up to 1024 with prime factors 2, 3, 5 and 7 (the 2x2 and 1x1 NGS of 15 and
-// 30 m, a 128^2 padding of an LGS subaperture).  Each (WFS, subaperture,
-// wavelength) chain c = (iwfs nsa + isa) nwvl + iwvl runs five batched
-// line-transform passes; a block transforms L lines held in LDS (rows, or L
-// adjacent columns read and written as L-wide row segments):
+// FP32 imaging of subapertures of any other size (low-order NGS: 2x2 or 1x1
+// subapertures with 240^2 to 480^2 point fields, and the 128^2 padding of the
+// LGS field): chain c = (WFS, subaperture, wavelength) runs four passes of
+// line FFTs in LDS (linefft.hip), each block transforming L lines, rows
+// directly and columns as L-wide row segments:
 //   A  embed amp exp(+i 2 pi opd/wvl) (cembed_wvf, math/matcomp.c:56-82) on
 //      the nxsa rows of the field band, FFT along x  -> B1 [nxsa][nwvf]
-//   B  FFT the columns of B1 (rows outside the band are zero), |E|^2
-//                                                     -> PSF [nwvf][nwvf]
-//   C  FFT the PSF rows padded to notf by the corner copy (ccpcorner,
-//      math/matcomp.c:176-216: x < nwvf/2 stays, the rest moves up by
-//      notf - nwvf, the middle is zero), two real rows per complex FFT,
-//      columns <= notf/2 kept                       -> B2 [nwvf][notf/2+1]
-//   D  FFT those columns of B2 (rows padded the same way), x nominal DTF,
-//      inverse FFT, keep the rows the detector samples
-//                                                     -> B3 [ny][notf/2+1]
-//   E  inverse FFT of those rows (the other columns are the conjugate
-//      mirror), keep the sampled columns (real part) -> image [ny][nx]
+//   B  FFT the columns of B1 (rows outside the band are zero), |E|^2, and in
+//      the same block the PSF columns padded to notf by the corner copy
+//      (ccpcorner, math/matcomp.c:176-216: y < nwvf/2 stays, the rest moves
+//      up by notf - nwvf, the middle is zero) and transformed, two real
+//      columns per complex FFT, rows <= notf/2 kept -> B2 [notf/2+1][nwvf]
+//   D  FFT those rows of B2 (columns padded the same way), x nominal or
+//      conj(lotf) ETF, inverse FFT, keep the columns the detector samples
+//                                                     -> B3 [nx][notf/2+1]
+//   E  the sampled rows of those columns, summed directly over uy (the other
+//      half plane is the conjugate)                  -> image [ny][nx]
 // then k_lf_sample applies si (maos/wfsints.c:286) and the pixel processing.
+// The |E|^2 never leaves the chip, and every factor after it is the transform
+// of a real function, so half the plane is enough.
+//
+// Measured against five passes that wrote the PSF out and transformed it back
+// in (ping-pong Stockham stages of radix 8 at most, the plan read at run
+// time): 24 chains of 480^2 in 512^2 165 -> 85 us (1.1 TB/s of B1 and B2),
+// one chain of 960^2 in 1024^2 61 -> 55 us (latency of the passes, one or two
+// blocks a CU), 1,968 chains of 128^2 with their uplink 808 -> 220 us.
 constexpr int MX_LF_MAXN = 1024;
-constexpr int MX_LF_MAXRAD = 12;
-constexpr int MX_LF_THREADS = 512; // most threads of a block (128, 256 or 512 run)
-constexpr int MX_LF_LDS = 4352;    // complex elements of one LDS line buffer
+constexpr int MX_LF_THREADS = 512; // most threads per block the choice of L aims at (128, 256 or 512)
 constexpr int MX_LF_MAXS = 128;    // most sampled rows / columns kept (else the full image)
-
-// LDS position of element e of a line: one pad element after every 32, so
-// that the power-of-two write strides of the early Stockham stages spread
-// over the LDS banks
-__host__ __device__ constexpr int lf_pos(int e) { return e + (e >> 5); }
-// LDS stride of lines of length n: the padded length, made odd
-__host__ __device__ constexpr int lf_stride(int n) { return lf_pos(n) | 1; }
-// lines of length n per block: a power of two <= 32 that one buffer holds;
-// for lines of 768 and more at most 2048 / n of them, so that a one-chain
-// plane (the 960^2 and 1024^2 tip-tilt sizes: 2 lines, 480-512 blocks)
-// spreads over more blocks than CUs (53 -> 46 us per step for the 1024^2
-// tip-tilt imaging; the 512^2 planes, with many chains, keep 8 lines)
-__host__ __device__ constexpr int lf_lines(int n) {
-    int L = 32;
-    while (L > 1 && (L * lf_stride(n) > MX_LF_LDS || (n >= 768 && L * n > 2048))) L /= 2;
-    return L;
-}
-// radix of stage s in the plan of n (radix 8 first, then 4, 2, 3, 5, 7); 0
-// past the last stage or if n has another prime factor
-__host__ __device__ constexpr int lf_radix(int n, int s) {
-    const int rad[6] = {8, 4, 2, 3, 5, 7};
-    int r = n, c = 0;
-    for (int k = 0; k < 6; k++)
-        while (r > 1 && r % rad[k] == 0) {
-            if (c == s) return rad[k];
-            c++;
-            r /= rad[k];
-        }
-    return 0;
+constexpr int MX_LF_ESUB = 8;      // lanes that share one output of pass E
+constexpr int MX_LF_ESHORT = 129;  // longest column (m/2 + 1) of its staged form
+// complex elements of pass E's column buffer
+constexpr int MX_LF_ECOL = 2080;
+// columns per block of pass E: as many as the buffer holds, at most 16
+__host__ __device__ constexpr int lf_ecols(int mh) {
+    const int x = MX_LF_ECOL / mh;
+    return x > 16 ? 16 : (x < 1 ? 1 : x);
 }
 
-struct LfPlan {
-    int n, nrad;
-    int rad[MX_LF_MAXRAD]; // lf_radix(n, s)
-    int off[MX_LF_MAXRAD]; // twiddle offset of each stage
-    const float2 *tw;      // stage s: exp(-2 pi i r k / (Ns R)) at off[s] + k (R-1) + r-1
-};
 struct LfWvl {
-    float inv_wvl;
-    const float *nominal; // [ux][uy] (transposed), or null
-    const float2 *etf, *etf2; // [nsa][ux][uy] ETF with the nominal fused (LLT), second profile or null
+    double inv_wvl64;
+    const float *nominal; // [uy][ux], or null
+    const float2 *etf, *etf2; // [nsa][uy][ux] ETF with the nominal fused (LLT), second profile or null
     int ny, nx;           // sampled image rows / columns
     const int *rows, *cols;
     const int4 *si_c;     // si in compact indices iy * nx + ix
@@ -2331,188 +2309,18 @@ struct LfWvl {
     int si_sa, nom_sa;    // per-subaperture strides of si_c / si_w and nominal (0: shared)
 };
 struct LfArgs {
-    LfPlan pn, pm;        // lengths nwvf and notf
+    LinePlan pn, pm;      // lengths nwvf and notf
     int nwvf, notf, nxsa, nsa, nwfs, nwvl, nchain;
-    int L, lgL;           // lines per block in this pass (lf_lines of its length)
-    int maxny, maxnx;     // B3 rows and image capacity per chain
+    int L, lgL;           // lines per block in this pass
+    int maxny, maxnx;     // B3 columns and image capacity per chain
     const float *opd, *amp;
     const LfWvl *wv;
     float2 *b1, *b2, *b3;
-    float *psf, *img;
-    float psf_scale;      // pass C multiplies the PSF by this (1/nlwvf^2 for the uplink)
-    float2 *lotf;         // [nwfs][nwvl][ux][uy] conj(lotfc): written by the uplink, read by imaging; or null
+    float *img;
+    float psf_scale;      // pass B multiplies the PSF by this (1/nlwvf^2 for the uplink)
+    float2 *lotf;         // [nwfs][nwvl][uy][ux] conj(lotfc), uy <= notf/2: written by the uplink, read by imaging; or null
     float etf1wt, etf2wt; // ETF profile weights (maos/wfsints.c:215-223)
 };
-
-// a / b for 0 <= a < 2^22 from a rounded reciprocal rb of b, corrected
-__device__ __forceinline__ int qdiv(int a, int b, float rb) {
-    int q = (int)((float)a * rb);
-    const int r = a - q * b;
-    q += r >= b ? 1 : (r < 0 ? -1 : 0);
-    return q;
-}
-// a / b: by the compiler when b is a constant (CT), else by qdiv
-template <bool CT>
-__device__ __forceinline__ int ldiv(int a, int b, float rb) {
-    if constexpr (CT) return a / b;
-    else return qdiv(a, b, rb);
-}
-
-__device__ __forceinline__ float2 mul_ti(float2 z, float t) { return make_float2(-t * z.y, t * z.x); }
-// v[q] <- sum_r v[r] exp(t 2 pi i r q / R), t = +-1
-template <int R>
-__device__ __forceinline__ void small_dft(float2 (&v)[R], float t) {
-    if constexpr (R == 2) {
-        const float2 a = v[0], b = v[1];
-        v[0] = cadd(a, b);
-        v[1] = csub(a, b);
-    } else if constexpr (R == 4) {
-        const float2 s02 = cadd(v[0], v[2]), d02 = csub(v[0], v[2]);
-        const float2 s13 = cadd(v[1], v[3]), d13 = mul_ti(csub(v[1], v[3]), t);
-        v[0] = cadd(s02, s13);
-        v[2] = csub(s02, s13);
-        v[1] = cadd(d02, d13);
-        v[3] = csub(d02, d13);
-    } else if constexpr (R == 8) {
-        // even and odd halves by 4-point transforms, then w8^q = exp(t 2 pi i q / 8)
-        // on the odd half: w8 = (1 + t i) / sqrt 2, w8^2 = t i, w8^3 = (-1 + t i) / sqrt 2
-        const float h = 0.70710678118654752f;
-        float2 e[4] = {v[0], v[2], v[4], v[6]}, o[4] = {v[1], v[3], v[5], v[7]};
-        small_dft<4>(e, t);
-        small_dft<4>(o, t);
-        const float2 o1 = mul_ti(o[1], t), o3 = mul_ti(o[3], t);
-        o[1] = make_float2(h * (o[1].x + o1.x), h * (o[1].y + o1.y));
-        o[2] = mul_ti(o[2], t);
-        o[3] = make_float2(h * (o3.x - o[3].x), h * (o3.y - o[3].y));
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            v[q] = cadd(e[q], o[q]);
-            v[q + 4] = csub(e[q], o[q]);
-        }
-    } else if constexpr (R == 3) {
-        const float h = 0.86602540378443865f; // sqrt(3)/2
-        const float2 s = cadd(v[1], v[2]), d = csub(v[1], v[2]);
-        const float2 m = make_float2(v[0].x - 0.5f * s.x, v[0].y - 0.5f * s.y);
-        const float2 r = mul_ti(make_float2(h * d.x, h * d.y), t);
-        v[0] = cadd(v[0], s);
-        v[1] = cadd(m, r);
-        v[2] = csub(m, r);
-    } else if constexpr (R == 7) {
-        // pairs r, 7 - r: v[k] = v0 + sum_r cos(2 pi r k / 7) (v[r] + v[7-r])
-        //                      + t i sum_r sin(2 pi r k / 7) (v[r] - v[7-r])
-        constexpr float c[4] = {1.f, 0.62348980185873353f, -0.22252093395631440f, -0.90096886790241913f};
-        constexpr float sn[4] = {0.f, 0.78183148246802981f, 0.97492791218182361f, 0.43388373911755812f};
-        float2 a[4], b[4];
-#pragma unroll
-        for (int r = 1; r <= 3; r++) {
-            a[r] = cadd(v[r], v[7 - r]);
-            b[r] = csub(v[r], v[7 - r]);
-        }
-        const float2 v0 = v[0];
-#pragma unroll
-        for (int k = 1; k <= 3; k++) {
-            float2 p = v0, q = make_float2(0.f, 0.f);
-#pragma unroll
-            for (int r = 1; r <= 3; r++) {
-                const int m = (r * k) % 7; // cos(2 pi m / 7), sin of it with the sign of m <= 3
-                const float cm = c[m <= 3 ? m : 7 - m], sm = m <= 3 ? sn[m] : -sn[7 - m];
-                p = make_float2(p.x + cm * a[r].x, p.y + cm * a[r].y);
-                q = make_float2(q.x + sm * b[r].x, q.y + sm * b[r].y);
-            }
-            q = mul_ti(q, t);
-            v[k] = cadd(p, q);
-            v[7 - k] = csub(p, q);
-        }
-        v[0] = cadd(v0, cadd(a[1], cadd(a[2], a[3])));
-    } else { // 5: cos and sin of 2 pi/5 and 4 pi/5
-        const float c1 = 0.30901699437494742f, c2 = -0.80901699437494742f;
-        const float s1 = 0.95105651629515357f, s2 = 0.58778525229247313f;
-        const float2 a1 = cadd(v[1], v[4]), a2 = cadd(v[2], v[3]);
-        const float2 b1 = csub(v[1], v[4]), b2 = csub(v[2], v[3]);
-        const float2 p1 = make_float2(v[0].x + c1 * a1.x + c2 * a2.x, v[0].y + c1 * a1.y + c2 * a2.y);
-        const float2 p2 = make_float2(v[0].x + c2 * a1.x + c1 * a2.x, v[0].y + c2 * a1.y + c1 * a2.y);
-        const float2 q1 = mul_ti(make_float2(s1 * b1.x + s2 * b2.x, s1 * b1.y + s2 * b2.y), t);
-        const float2 q2 = mul_ti(make_float2(s2 * b1.x - s1 * b2.x, s2 * b1.y - s1 * b2.y), t);
-        v[0] = cadd(v[0], cadd(a1, a2));
-        v[1] = cadd(p1, q1);
-        v[4] = csub(p1, q1);
-        v[2] = cadd(p2, q2);
-        v[3] = csub(p2, q2);
-    }
-}
-
-// One Stockham stage of radix R and span Ns over L lines (line l at l S,
-// element e at lf_pos(e)) by a block of T threads: item (l, j), j < n/R,
-// takes x[j + r n/R] times w^(r k) (w = exp(-+ 2 pi i / (Ns R)), k = j % Ns),
-// transforms and writes x'[(j/Ns) Ns R + k + r Ns].  CT: n, Ns and L are
-// compile-time constants.  Forward is FFTW_FORWARD (exp(-i ...)).
-template <int R, bool INV, bool CT, int T>
-__device__ __forceinline__ void lds_stage(const float2 *src, float2 *dst, int n, int Ns, int L, int S,
-                                          const float2 *tw) {
-    const int nb = n / R, total = L * nb;
-    const float rnb = 1.f / (float)nb, rns = 1.f / (float)Ns;
-    for (int it = (int)threadIdx.x; it < total; it += T) {
-        const int l = ldiv<CT>(it, nb, rnb), j = it - l * nb;
-        const int g = ldiv<CT>(j, Ns, rns), k = j - g * Ns;
-        const float2 *x = src + l * S;
-        const float2 *w = tw + k * (R - 1);
-        float2 v[R];
-        v[0] = x[lf_pos(j)];
-#pragma unroll
-        for (int r = 1; r < R; r++) {
-            float2 wr = w[r - 1];
-            if (INV) wr.y = -wr.y;
-            v[r] = cmul(x[lf_pos(j + r * nb)], wr);
-        }
-        small_dft<R>(v, INV ? 1.f : -1.f);
-        float2 *y = dst + l * S;
-        const int d = g * Ns * R + k;
-#pragma unroll
-        for (int r = 0; r < R; r++) y[lf_pos(d + r * Ns)] = v[r];
-    }
-}
-
-// Stockham autosort FFT of L lines of length P.n in src; returns the buffer
-// that holds the result (src or dst).  Stages from the plan at run time.
-template <bool INV, int T>
-__device__ float2 *lds_fft_rt(float2 *src, float2 *dst, const LfPlan &P, int L, int S) {
-    int Ns = 1;
-    for (int s = 0; s < P.nrad; s++) {
-        const int R = P.rad[s];
-        const float2 *tw = P.tw + P.off[s];
-        if (R == 8) lds_stage<8, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        else if (R == 4) lds_stage<4, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        else if (R == 2) lds_stage<2, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        else if (R == 3) lds_stage<3, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        else if (R == 5) lds_stage<5, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        else lds_stage<7, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        __syncthreads();
-        float2 *t = src;
-        src = dst;
-        dst = t;
-        Ns *= R;
-    }
-    return src;
-}
-// the same for a compile-time length N, from stage SI of span NS on
-template <bool INV, int T, int N, int SI, int NS>
-__device__ __forceinline__ float2 *lds_fft_ct(float2 *src, float2 *dst, const float2 *tw) {
-    constexpr int R = lf_radix(N, SI);
-    if constexpr (R == 0) {
-        return src;
-    } else {
-        constexpr int L = lf_lines(N), S = lf_stride(N);
-        lds_stage<R, INV, true, T>(src, dst, N, NS, L, S, tw);
-        __syncthreads();
-        return lds_fft_ct<INV, T, N, SI + 1, NS * R>(dst, src, tw + NS * (R - 1));
-    }
-}
-// FFT of the block's lines: compile-time plan for N > 0, else P's
-template <bool INV, int T, int N>
-__device__ __forceinline__ float2 *lf_fft(float2 *src, float2 *dst, const LfPlan &P, int L, int S) {
-    if constexpr (N > 0) return lds_fft_ct<INV, T, N, 0, 1>(src, dst, P.tw);
-    else return lds_fft_rt<INV, T>(src, dst, P, L, S);
-}
 
 // block -> (line group g of ngroup, chain c); consecutive groups of a chain
 // share an XCD and its L2
@@ -2522,227 +2330,231 @@ __device__ __forceinline__ void lf_unit(const LfArgs &a, int ngroup, int &g, int
     c = u / ngroup;
 }
 __device__ __forceinline__ void lf_chain(const LfArgs &a, int c, int &iwfs, int &isa, int &iwvl) {
+    // (the WFS of one subaperture, which share its ETF, are neighbours: the ETF
+    // of a 128^2 padded LGS field is as large as its spectrum)
     iwvl = c % a.nwvl;
-    isa = (c / a.nwvl) % a.nsa;
-    iwfs = c / (a.nwvl * a.nsa);
+    iwfs = (c / a.nwvl) % a.nwfs;
+    isa = c / (a.nwvl * a.nwfs);
 }
-// padded position -> source index of the corner copy (-1 in the zero middle)
-__device__ __forceinline__ int corner_src(int x2, int m, int n) {
-    const int h = n / 2;
-    return x2 < h ? x2 : (x2 >= m - h ? x2 - (m - n) : -1);
-}
-
-// Each pass is a template on the block size T and the length N of its lines
-// (0: taken from the arguments at run time).
-#define MX_LF_GEOM(LEN, ARGL)                                                   \
-    constexpr int LC = N > 0 ? lf_lines(N) : 1, SC = N > 0 ? lf_stride(N) : 1; \
-    const int n_ = N > 0 ? N : (LEN), L = N > 0 ? LC : (ARGL), S = N > 0 ? SC : lf_stride(n_);
+// the passes run in dynamic LDS of lf_lds() bytes
+extern __shared__ float2 lfs[];
 
 // pass A: embed the field-band rows and FFT them along x
-template <int T, int N>
-__global__ __launch_bounds__(T) void k_lf_a(LfArgs a) {
-    __shared__ float2 X[MX_LF_LDS], Y[MX_LF_LDS];
-    MX_LF_GEOM(a.nwvf, a.L)
-    const int n = n_, nxsa = a.nxsa, skip = (n - nxsa) / 2;
+__global__ __launch_bounds__(1024) void k_lf_a(LfArgs a) {
+    const int n = a.nwvf, nxsa = a.nxsa, skip = (n - nxsa) / 2, L = a.L, S = a.pn.S;
+    const LxLines ln{L, a.lgL};
     int g, c, iwfs, isa, iwvl;
     lf_unit(a, (nxsa + L - 1) / L, g, c);
     lf_chain(a, c, iwfs, isa, iwvl);
     const long np = (long)nxsa * nxsa;
-    const float *op = a.opd + ((long)iwfs * a.nsa + isa) * np;
-    const float *am = a.amp + (long)isa * np;
-    const float inv_wvl = a.wv[iwvl].inv_wvl;
-    const float rn = 1.f / (float)n;
-    for (int e = threadIdx.x; e < L * n; e += T) {
-        const int l = ldiv<(N > 0)>(e, n, rn), x = e - l * n, iy = g * L + l, ix = x - skip;
-        float2 v = make_float2(0.f, 0.f);
-        if (iy < nxsa && ix >= 0 && ix < nxsa) {
-            float sn, cs;
-            sincospif(2.f * op[(long)iy * nxsa + ix] * inv_wvl, &sn, &cs);
-            const float A = am[(long)iy * nxsa + ix];
-            v = make_float2(A * cs, A * sn);
-        }
-        X[l * S + lf_pos(x)] = v;
+    const float *op = a.opd + ((long)iwfs * a.nsa + isa) * np + (long)g * L * nxsa;
+    const float *am = a.amp + (long)isa * np + (long)g * L * nxsa;
+    const double iw = a.wv[iwvl].inv_wvl64;
+    const float rn = 1.f / (float)nxsa;
+    const int nrow = min(L, nxsa - g * L);
+    for (int e = threadIdx.x; e < nrow * nxsa; e += blockDim.x) {
+        const int l = qdiv(e, nxsa, rn), ix = e - l * nxsa;
+        // the phase in revolutions, reduced in FP64: an OPD of many
+        // wavelengths loses nothing to the FP32 product
+        double rev = (double)lx_at(op, e) * iw;
+        rev -= rint(rev);
+        float sn, cs;
+        sincospif(2.f * (float)rev, &sn, &cs);
+        const float A = lx_at(am, e);
+        lfs[l * S + skip + ix] = make_float2(A * cs, A * sn);
     }
     __syncthreads();
-    const float2 *r = lf_fft<false, T, N>(X, Y, a.pn, L, S);
-    float2 *out = a.b1 + (long)c * nxsa * n;
-    for (int e = threadIdx.x; e < L * n; e += T) {
-        const int l = ldiv<(N > 0)>(e, n, rn), x = e - l * n, iy = g * L + l;
-        if (iy < nxsa) out[(long)iy * n + x] = r[l * S + lf_pos(x)];
-    }
+    float2 *out = a.b1 + ((long)c * nxsa + g * L) * n;
+    lx_fft<false, LX_ROW, LX_ROW, true>(
+        lfs, LX_PLAN(LfArgs, pn), ln,
+        [&](int l, int j, int off) LX_INLINE {
+            const int e = j + off;
+            return lx_sel(l < nrow && e >= skip && e < skip + nxsa, lfs[__mul24(l, S) + j + off]);
+        },
+        [&](int l, int d, int off, float2 v, int) LX_INLINE {
+            if (l < nrow) lx_at(out + off, __mul24(l, n) + d) = v;
+        });
 }
 
-// pass B: FFT the columns of B1 and take |E|^2
-template <int T, int N>
-__global__ __launch_bounds__(T) void k_lf_b(LfArgs a) {
-    __shared__ float2 X[MX_LF_LDS], Y[MX_LF_LDS];
-    MX_LF_GEOM(a.nwvf, a.L)
-    const int n = n_, nxsa = a.nxsa, skip = (n - nxsa) / 2, lgL = N > 0 ? ilog2c(LC) : a.lgL;
+// pass B: FFT the columns of B1, |E|^2, and the PSF columns' FFT along y: the
+// PSF is real, so columns 2q and 2q+1 go through one complex FFT as z = a + i
+// b, and A[k] = (Z[k] + conj Z[m-k]) / 2, B[k] = (Z[k] - conj Z[m-k]) / 2i are
+// kept for k <= m/2 only.
+__global__ __launch_bounds__(1024) void k_lf_b(LfArgs a) {
+    const int n = a.nwvf, m = a.notf, nxsa = a.nxsa, skip = (n - nxsa) / 2, L = a.L, mh = m / 2 + 1, h = n / 2;
+    const LxLines ln{L, a.lgL}, l2{L / 2, a.lgL - 1};
+    const int S2 = a.pm.S;
     int g, c;
     lf_unit(a, (n + L - 1) / L, g, c);
     const int x0 = g * L;
-    const float2 *in = a.b1 + (long)c * nxsa * n;
-    for (int e = threadIdx.x; e < L * n; e += T) {
-        const int l = e & (L - 1), y = e >> lgL, x = x0 + l, iy = y - skip;
-        float2 v = make_float2(0.f, 0.f);
-        if (x < n && iy >= 0 && iy < nxsa) v = in[(long)iy * n + x];
-        X[l * S + lf_pos(y)] = v;
-    }
+    const float2 *in = a.b1 + (long)c * nxsa * n + x0;
+    const float sc = a.psf_scale;
+    float *psf = reinterpret_cast<float *>(lfs);
+    lx_fft<false, LX_COL, LX_COL, false>(
+        lfs, LX_PLAN(LfArgs, pn), ln,
+        [&](int l, int j, int off) LX_INLINE {
+            const int e = j + off;
+            const bool ok = x0 + l < n && e >= skip && e < skip + nxsa;
+            return lx_sel(ok, lx_at(in, ok ? __mul24(j, n) + l + (off - skip) * n : 0));
+        },
+        [&](int l, int d, int off, float2 v, int) LX_INLINE {
+            const int y = d + off + (d + off < h ? 0 : m - n);
+            psf[__mul24(l >> 1, 2 * S2) + (l & 1) + 2 * y] = (v.x * v.x + v.y * v.y) * sc;
+        });
     __syncthreads();
-    const float2 *r = lf_fft<false, T, N>(X, Y, a.pn, L, S);
-    float *out = a.psf + (long)c * n * n;
-    for (int e = threadIdx.x; e < L * n; e += T) {
-        const int l = e & (L - 1), y = e >> lgL, x = x0 + l;
-        if (x < n) {
-            const float2 v = r[l * S + lf_pos(y)];
-            out[(long)y * n + x] = v.x * v.x + v.y * v.y;
-        }
+    lx_fft<false, LX_COL, LX_COL, true>(
+        lfs, LX_PLAN(LfArgs, pm), l2,
+        [&](int l, int j, int off) LX_INLINE {
+            const int e = j + off;
+            return lx_sel(e < h || e >= m - h, lfs[__mul24(l, S2) + j + off]);
+        },
+        [&](int l, int d, int off, float2 v, int) LX_INLINE { lfs[__mul24(l, S2) + d + off] = v; });
+    __syncthreads();
+    float2 *out = a.b2 + (long)c * mh * n + x0;
+    for (int i = threadIdx.x; i < l2.L * mh; i += blockDim.x) {
+        const int q = i & (l2.L - 1), k = i >> l2.lgL;
+        if (x0 + 2 * q >= n) continue;
+        const float2 z = lfs[q * S2 + k], w = lfs[q * S2 + (k == 0 ? 0 : m - k)];
+        float2 *o = out + (long)k * n + 2 * q;
+        o[0] = make_float2(0.5f * (z.x + w.x), 0.5f * (z.y - w.y));
+        o[1] = make_float2(0.5f * (z.y + w.y), 0.5f * (w.x - z.x));
     }
 }
 
-// pass C: FFT the PSF rows, padded to notf by the corner copy.  The PSF is
-// real, so rows 2p and 2p+1 go through one complex FFT as z = a + i b, and
-// A[k] = (Z[k] + conj Z[m-k]) / 2, B[k] = (Z[k] - conj Z[m-k]) / 2i are kept
-// for k <= m/2 only (the rest is their conjugate mirror): B2 is [nwvf][m/2+1].
-template <int T, int N>
-__global__ __launch_bounds__(T) void k_lf_c(LfArgs a) {
-    __shared__ float2 X[MX_LF_LDS], Y[MX_LF_LDS];
-    MX_LF_GEOM(a.notf, a.L)
-    const int n = a.nwvf, m = n_, mh = m / 2 + 1, np = n / 2;
-    int g, c;
-    lf_unit(a, (np + L - 1) / L, g, c);
-    const float *in = a.psf + (long)c * n * n;
-    const float rm = 1.f / (float)m, rmh = 1.f / (float)mh, s = a.psf_scale;
-    for (int e = threadIdx.x; e < L * m; e += T) {
-        const int l = ldiv<(N > 0)>(e, m, rm), x2 = e - l * m, p = g * L + l, x = corner_src(x2, m, n);
-        X[l * S + lf_pos(x2)] = p < np && x >= 0
-                                    ? make_float2(in[(long)(2 * p) * n + x] * s, in[(long)(2 * p + 1) * n + x] * s)
-                                    : make_float2(0.f, 0.f);
-    }
-    __syncthreads();
-    const float2 *r = lf_fft<false, T, N>(X, Y, a.pm, L, S);
-    float2 *out = a.b2 + (long)c * n * mh;
-    for (int e = threadIdx.x; e < L * mh; e += T) {
-        const int l = ldiv<(N > 0)>(e, mh, rmh), k = e - l * mh, p = g * L + l;
-        if (p < np) {
-            const float2 z = r[l * S + lf_pos(k)], w = r[l * S + lf_pos(k == 0 ? 0 : m - k)];
-            out[(long)(2 * p) * mh + k] = make_float2(0.5f * (z.x + w.x), 0.5f * (z.y - w.y));
-            out[(long)(2 * p + 1) * mh + k] = make_float2(0.5f * (z.y + w.y), 0.5f * (w.x - z.x));
-        }
-    }
-}
-
-// pass D: FFT the columns ux <= m/2 of B2 (rows padded by the corner copy),
-// x conj(lotf) x ETF (LLT) or x nominal, inverse FFT, keep the sampled rows:
-// B3 is [ny][m/2+1].  Every factor is the transform of a real function, so
-// the product at -u is the conjugate of that at u and the other columns are
-// not needed.  UPLINK: the chains are (WFS, wavelength) LLT fields and the
-// column FFT is conj-stored as the uplink OTF lotfc over ux <= m/2
-// (maos/wfsints.c:149-199).
-template <int T, int N, bool UPLINK>
-__global__ __launch_bounds__(T) void k_lf_d(LfArgs a) {
-    __shared__ float2 X[MX_LF_LDS], Y[MX_LF_LDS];
-    MX_LF_GEOM(a.notf, a.L)
-    const int n = a.nwvf, m = n_, mh = m / 2 + 1, lgL = N > 0 ? ilog2c(LC) : a.lgL;
+// pass D: FFT the rows uy <= m/2 of B2 (columns padded by the corner copy),
+// x conj(lotf) x ETF (LLT) or x nominal, inverse FFT, keep the sampled
+// columns: B3 is [nx][m/2+1].  UPLINK: the chains are (WFS, wavelength) LLT
+// fields and the row FFT is conj-stored as the uplink OTF lotfc over
+// uy <= m/2 (maos/wfsints.c:149-199).
+template <bool UPLINK>
+__global__ __launch_bounds__(1024) void k_lf_d(LfArgs a) {
+    const int n = a.nwvf, m = a.notf, mh = m / 2 + 1, L = a.L, S = a.pm.S, h = n / 2;
+    const LxLines ln{L, a.lgL};
     int g, c, iwfs, isa, iwvl;
     lf_unit(a, (mh + L - 1) / L, g, c);
     lf_chain(a, c, iwfs, isa, iwvl);
-    const int x0 = g * L;
-    const float2 *in = a.b2 + (long)c * n * mh;
-    for (int e = threadIdx.x; e < L * m; e += T) {
-        const int l = e & (L - 1), y2 = e >> lgL, x2 = x0 + l, y = corner_src(y2, m, n);
-        X[l * S + lf_pos(y2)] = x2 < mh && y >= 0 ? in[(long)y * mh + x2] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();
-    float2 *r = lf_fft<false, T, N>(X, Y, a.pm, L, S);
+    const int y0 = g * L, nrow = min(L, mh - y0);
+    const float2 *in = a.b2 + ((long)c * mh + y0) * n;
+    auto load = [&](int l, int j, int off) LX_INLINE { // (corner copy: the row's ends, zeros between)
+        const int e = j + off, x = e < h ? e : e - (m - n);
+        const bool ok = l < nrow && (e < h || e >= m - h);
+        return lx_sel(ok, lx_at(in, ok ? __mul24(l, n) + x : 0));
+    };
     if constexpr (UPLINK) {
-        float2 *lo = a.lotf + (long)c * m * m;
-        for (int e = threadIdx.x; e < L * m; e += T) {
-            const int l = e & (L - 1), y2 = e >> lgL, x2 = x0 + l;
-            if (x2 < mh) {
-                const float2 z = r[l * S + lf_pos(y2)];
-                lo[(long)x2 * m + y2] = make_float2(z.x, -z.y);
-            }
-        }
+        float2 *lo = a.lotf + (long)c * m * m + (long)y0 * m;
+        lx_fft<false, LX_ROW, LX_ROW, false>(lfs, LX_PLAN(LfArgs, pm), ln, load, [&](int l, int d, int off, float2 v, int) LX_INLINE {
+            if (l < nrow) lx_at(lo + off, __mul24(l, m) + d) = make_float2(v.x, -v.y);
+        });
         return;
     }
     const LfWvl &W = a.wv[iwvl];
-    if (a.lotf) { // x conj(lotfc) x ETF (apply_dtf_etf, maos/wfsints.c:38-64)
-        const float2 *lo = a.lotf + ((long)iwfs * a.nwvl + iwvl) * m * m;
-        const float2 *e1 = W.etf + (long)isa * m * m, *e2 = W.etf2 ? W.etf2 + (long)isa * m * m : nullptr;
-        const float rm = 1.f / (float)m;
-        for (int e = threadIdx.x; e < L * m; e += T) {
-            const int l = ldiv<(N > 0)>(e, m, rm), y2 = e - l * m, x2 = x0 + l;
-            if (x2 < mh) {
-                const long i = (long)x2 * m + y2;
-                float2 et = e1[i];
-                if (e2) {
-                    const float2 t2 = e2[i];
-                    et = make_float2(et.x * a.etf1wt + t2.x * a.etf2wt, et.y * a.etf1wt + t2.y * a.etf2wt);
-                }
-                float2 &z = r[l * S + lf_pos(y2)];
-                z = cmul(cmul(z, lo[i]), et);
-            }
-        }
-        __syncthreads();
+    // x conj(lotfc) x ETF (apply_dtf_etf, maos/wfsints.c:38-64), or x nominal
+    const float2 *lo = nullptr, *e1 = nullptr, *e2 = nullptr;
+    const float *nm = nullptr;
+    const float w1 = a.etf1wt, w2 = a.etf2wt;
+    if (a.lotf) {
+        lo = a.lotf + (((long)iwfs * a.nwvl + iwvl) * m + y0) * m;
+        e1 = W.etf + ((long)isa * m + y0) * m;
+        e2 = W.etf2 ? W.etf2 + ((long)isa * m + y0) * m : nullptr;
     } else if (W.nominal) {
-        const float rm = 1.f / (float)m;
-        for (int e = threadIdx.x; e < L * m; e += T) {
-            const int l = ldiv<(N > 0)>(e, m, rm), y2 = e - l * m, x2 = x0 + l;
-            if (x2 < mh) {
-                const float f = W.nominal[(long)isa * W.nom_sa + (long)x2 * m + y2];
-                float2 &z = r[l * S + lf_pos(y2)];
-                z = make_float2(z.x * f, z.y * f);
+        nm = W.nominal + (long)isa * W.nom_sa + (long)y0 * m;
+    }
+    lx_fft<false, LX_ROW, LX_ROW, false>(lfs, LX_PLAN(LfArgs, pm), ln, load, [&](int l, int d, int off, float2 v, int) LX_INLINE {
+        const int i = __mul24(l, m) + d;
+        if (l < nrow) {
+            if (lo) {
+                float2 et = lx_at(e1 + off, i);
+                if (e2) {
+                    const float2 t2 = lx_at(e2 + off, i);
+                    et = make_float2(et.x * w1 + t2.x * w2, et.y * w1 + t2.y * w2);
+                }
+                v = cmul(cmul(v, lx_at(lo + off, i)), et);
+            } else if (nm) {
+                const float f = lx_at(nm + off, i);
+                v = make_float2(v.x * f, v.y * f);
             }
         }
-        __syncthreads();
-    }
-    const float2 *q = lf_fft<true, T, N>(r, r == X ? Y : X, a.pm, L, S);
-    float2 *out = a.b3 + (long)c * a.maxny * mh;
-    for (int e = threadIdx.x; e < L * W.ny; e += T) {
-        const int l = e & (L - 1), iyy = e >> lgL, x2 = x0 + l;
-        if (x2 < mh) out[(long)iyy * mh + x2] = q[l * S + lf_pos(W.rows[iyy])];
+        lfs[__mul24(l, S) + d + off] = v;
+    });
+    __syncthreads();
+    lx_fft<true, LX_ROW, LX_ROW, true>(
+        lfs, LX_PLAN(LfArgs, pm), ln, [&](int l, int j, int off) LX_INLINE { return lfs[__mul24(l, S) + j + off]; },
+        [&](int l, int d, int off, float2 v, int) LX_INLINE { lfs[__mul24(l, S) + d + off] = v; });
+    __syncthreads();
+    float2 *out = a.b3 + (long)c * a.maxnx * mh + y0;
+    for (int e = threadIdx.x; e < L * W.nx; e += blockDim.x) {
+        const int l = e & (L - 1), ixx = e >> a.lgL;
+        if (l < nrow) out[(long)ixx * mh + l] = lfs[l * S + W.cols[ixx]];
     }
 }
 
-// pass E: inverse FFT of the sampled rows, real part at the sampled columns;
-// a row's columns past m/2 are the conjugates of columns m - ux
-template <int T, int N>
-__global__ __launch_bounds__(T) void k_lf_e(LfArgs a) {
-    __shared__ float2 X[MX_LF_LDS], Y[MX_LF_LDS];
-    MX_LF_GEOM(a.notf, a.L)
-    const int m = n_;
+// pass E: the inverse transform along y of the sampled columns at the sampled
+// rows, real part: I[ys][xs] = Re sum_{uy <= m/2} w(uy) B3[xs][uy]
+// exp(+2 pi i uy ys / m), w = 1 at 0 and m/2, else 2.  A few tens of outputs
+// per column, so they are summed directly, in FP64, rather than transformed.
+// Short columns (mh <= MX_LF_ESHORT): XG columns staged in LDS, MX_LF_ESUB
+// lanes an output (k_lf_e).  Long ones, of which there are few: a wave per
+// output straight from L2 (k_lf_e_wave), since the staged form leaves too few
+// blocks, each with a long chain of sums (21 us for one 1024^2 chain).
+__device__ __forceinline__ double lf_eterm(float2 v, float2 w, int k, int mh) { // w = exp(-2 pi i k ys / m)
+    const double p = (double)v.x * w.x + (double)v.y * w.y;
+    return k == 0 || k == mh - 1 ? p : 2. * p;
+}
+__global__ __launch_bounds__(256) void k_lf_e_wave(LfArgs a) {
+    const int m = a.notf, mh = m / 2 + 1, ng = (a.maxny * a.maxnx + 3) / 4, lane = threadIdx.x % 64;
     int g, c, iwfs, isa, iwvl;
-    lf_unit(a, (a.maxny + L - 1) / L, g, c);
+    lf_unit(a, ng, g, c);
     lf_chain(a, c, iwfs, isa, iwvl);
     const LfWvl &W = a.wv[iwvl];
-    if (g * L >= W.ny) return; // uniform: no sampled row in this group
-    const int mh = m / 2 + 1;
-    const float2 *in = a.b3 + (long)c * a.maxny * mh;
-    const float rm = 1.f / (float)m;
-    for (int e = threadIdx.x; e < L * m; e += T) {
-        const int l = ldiv<(N > 0)>(e, m, rm), x = e - l * m, iyy = g * L + l;
-        float2 v = make_float2(0.f, 0.f);
-        if (iyy < W.ny) {
-            if (x < mh) {
-                v = in[(long)iyy * mh + x];
-            } else {
-                v = in[(long)iyy * mh + m - x];
-                v.y = -v.y;
-            }
-        }
-        X[l * S + lf_pos(x)] = v;
+    const int o = g * 4 + threadIdx.x / 64;
+    if (o >= W.ny * W.nx) return; // uniform in the wave
+    const int xs = o / W.ny, iyy = o - xs * W.ny, ys = W.rows[iyy], step = 64 * ys % m;
+    const float2 *col = a.b3 + ((long)c * a.maxnx + xs) * mh;
+    int t = lane * ys % m;
+    double acc = 0;
+#pragma unroll 4
+    for (int k = lane; k < mh; k += 64) {
+        acc += lf_eterm(col[k], a.pm.tw[t], k, mh);
+        t += step;
+        t -= t >= m ? m : 0;
     }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) acc += __shfl_xor(acc, d);
+    if (lane == 0) a.img[(long)c * a.maxny * a.maxnx + (long)iyy * W.nx + xs] = (float)acc;
+}
+__global__ __launch_bounds__(256) void k_lf_e(LfArgs a) {
+    __shared__ float2 tw[2 * MX_LF_ESHORT], col[MX_LF_ECOL];
+    const int m = a.notf, mh = m / 2 + 1, XG = lf_ecols(mh), ng = (a.maxnx + XG - 1) / XG;
+    int g, c, iwfs, isa, iwvl;
+    lf_unit(a, ng, g, c);
+    lf_chain(a, c, iwfs, isa, iwvl);
+    const LfWvl &W = a.wv[iwvl];
+    const int xs0 = g * XG, nxg = min(XG, W.nx - xs0);
+    if (nxg <= 0) return; // uniform: no sampled column in this group
+    const float2 *in = a.b3 + ((long)c * a.maxnx + xs0) * mh;
+    for (int t = threadIdx.x; t < m; t += 256) tw[t] = a.pm.tw[t];
+    for (int e = threadIdx.x; e < nxg * mh; e += 256) col[e] = in[e];
     __syncthreads();
-    const float2 *r = lf_fft<true, T, N>(X, Y, a.pm, L, S);
     float *out = a.img + (long)c * a.maxny * a.maxnx;
-    const float rnx = 1.f / (float)W.nx;
-    for (int e = threadIdx.x; e < L * W.nx; e += T) {
-        const int l = qdiv(e, W.nx, rnx), ixx = e - l * W.nx, iyy = g * L + l;
-        if (iyy < W.ny) out[(long)iyy * W.nx + ixx] = r[l * S + lf_pos(W.cols[ixx])].x;
+    const int sub = threadIdx.x % MX_LF_ESUB, nout = W.ny * nxg;
+    const float rx = 1.f / (float)nxg;
+    for (int o0 = 0; o0 < nout; o0 += 256 / MX_LF_ESUB) {
+        const int o = o0 + threadIdx.x / MX_LF_ESUB;
+        const bool on = o < nout;
+        const int iyy = on ? qdiv(o, nxg, rx) : 0, xl = on ? o - iyy * nxg : 0;
+        const int ys = W.rows[iyy], step = MX_LF_ESUB * ys % m;
+        int t = sub * ys % m;
+        double acc = 0;
+        for (int k = sub; k < mh; k += MX_LF_ESUB) {
+            acc += lf_eterm(col[xl * mh + k], tw[t], k, mh);
+            t += step;
+            t -= t >= m ? m : 0;
+        }
+#pragma unroll
+        for (int d = 1; d < MX_LF_ESUB; d <<= 1) acc += __shfl_xor(acc, d);
+        if (on && sub == 0) out[(long)iyy * W.nx + xs0 + xl] = (float)acc;
     }
 }
-#undef MX_LF_GEOM
 
 // si sampling over the wavelengths and the pixel processing of one (WFS,
 // subaperture) (dspmulcreal, maos/wfsints.c:286; shwfs_grad,
@@ -2763,15 +2575,18 @@ struct LfSampleArgs {
     DtArgs dt;
 };
 __global__ __launch_bounds__(MX_LF_THREADS) void k_lf_sample(LfSampleArgs a) {
-    __shared__ float red[3][MX_LF_THREADS / 64];
+    __shared__ double red[3][MX_LF_THREADS / 64];
     const int isa = blockIdx.x % a.nsa, iwfs = blockIdx.x / a.nsa;
     const DevWfs &W = a.wfs[iwfs];
     const long ibase = ((long)iwfs * a.nsa + isa) * a.npix;
-    float s0 = 0.f, s1 = 0.f, s2 = 0.f;
+    // the moments are summed in FP64: the centre of gravity is the small
+    // difference of s0 / s2 and the middle pixel, and in FP32 its rounding was
+    // most of the gradient error of a 16 x 16 pixel detector
+    double s0 = 0., s1 = 0., s2 = 0.;
     for (int p = threadIdx.x; p < a.npix; p += blockDim.x) {
         float pv = 0.f;
         for (int iwvl = 0; iwvl < a.nwvl; iwvl++) {
-            const float *im = a.img + (((long)iwfs * a.nsa + isa) * a.nwvl + iwvl) * a.imgstride;
+            const float *im = a.img + (((long)isa * a.nwfs + iwfs) * a.nwvl + iwvl) * a.imgstride; // (lf_chain)
             const LfWvl &SW = a.wv[iwvl];
             const int4 id = SW.si_c[isa * SW.si_sa + p];
             const float4 w = SW.si_w[isa * SW.si_sa + p];
@@ -2784,22 +2599,25 @@ __global__ __launch_bounds__(MX_LF_THREADS) void k_lf_sample(LfSampleArgs a) {
         dither_add(a.dith, iwfs, ibase + p, pv);
         if (a.phytype == MX_PTYPE_MF) {
             const float *mt = a.mtche + ibase * 2 + 2 * p;
-            s0 += mt[0] * pv;
-            s1 += mt[1] * pv;
+            s0 += (double)mt[0] * pv;
+            s1 += (double)mt[1] * pv;
             s2 += pv;
         } else {
             const float iI = pv - a.cogoff;
             if (iI > a.cogthres) {
-                s0 += iI * (float)(p % a.pixpsax);
-                s1 += iI * (float)(p / a.pixpsax);
+                s0 += (double)iI * (p % a.pixpsax);
+                s1 += (double)iI * (p / a.pixpsax);
                 s2 += iI;
             }
         }
     }
     if (!(a.dt.phase & MX_DT_OUT)) return; // uniform
-    seg_sum<64>(s0);
-    seg_sum<64>(s1);
-    seg_sum<64>(s2);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        s0 += __shfl_xor(s0, o);
+        s1 += __shfl_xor(s1, o);
+        s2 += __shfl_xor(s2, o);
+    }
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     if (lane == 0) {
         red[0][wave] = s0;
@@ -2808,7 +2626,7 @@ __global__ __launch_bounds__(MX_LF_THREADS) void k_lf_sample(LfSampleArgs a) {
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        s0 = s1 = s2 = 0.f;
+        s0 = s1 = s2 = 0.;
         for (int w = 0; w < (int)blockDim.x / 64; w++) {
             s0 += red[0][w];
             s1 += red[1][w];
@@ -2817,22 +2635,22 @@ __global__ __launch_bounds__(MX_LF_THREADS) void k_lf_sample(LfSampleArgs a) {
         if (!(a.saa[isa] < a.saat)) {
             float gx = 0.f, gy = 0.f;
             if (a.sigmatch == 2) { // raw moments; k_sigmatch2 forms the gradients
-                gx = s0;
-                gy = s1;
+                gx = (float)s0;
+                gy = (float)s1;
             } else if (a.phytype == MX_PTYPE_MF) {
-                float scale = 1.f;
+                double scale = 1.;
                 if (a.sigmatch == 1) {
                     scale = a.i0sum[(long)iwfs * a.nsa + isa] / s2;
-                    if (scale <= 0.f || scale > 10.f || !isfinite(scale)) scale = 1.f;
+                    if (scale <= 0. || scale > 10. || !isfinite(scale)) scale = 1.;
                 }
-                gx = s0 * scale;
-                gy = s1 * scale;
+                gx = (float)(s0 * scale);
+                gy = (float)(s1 * scale);
             } else {
-                float sum = s2;
+                double sum = s2;
                 if (a.sigmatch == 0) sum = a.i0sum ? a.i0sum[(long)iwfs * a.nsa + isa] : a.sigtot * a.saa[isa];
                 if (sum > a.cogthres) {
-                    gx = (s0 / sum - (float)(a.pixpsax - 1) * 0.5f) * a.pixthetax;
-                    gy = (s1 / sum - (float)(a.pixpsay - 1) * 0.5f) * a.pixthetay;
+                    gx = (float)(s0 / sum - (a.pixpsax - 1) * 0.5) * a.pixthetax;
+                    gy = (float)(s1 / sum - (a.pixpsay - 1) * 0.5) * a.pixthetay;
                 }
             }
             a.grad[(long)iwfs * 2 * a.nsa + isa] = gx;
@@ -2930,6 +2748,7 @@ struct StepLaunch {
     dim3 grid, block;
     void *arg;
     int dep = -2; // the launch it waits for: -2 the previous one, -1 none (a branch's first)
+    unsigned lds = 0; // dynamic LDS bytes
 };
 struct StepPlan {
     StepLaunch L[MX_MAXLAUNCH];
@@ -3031,17 +2850,17 @@ struct mx_wfsgrad_s {
     bool lf = false;
     int lf_threads = 256;              // threads per large-field block
     int opd_tile = 0;                  // ray-trace tile side (16 or 32), 0: the default
-    LfPlan lf_pn{}, lf_pm{};           // twiddles in d_lf_tw
+    LinePlan lf_pn{}, lf_pm{};         // twiddles in d_lf_tw
     float2 *d_lf_tw = nullptr;
     float2 *d_b1 = nullptr, *d_b2 = nullptr, *d_b3 = nullptr;
-    float *d_psf = nullptr, *d_img = nullptr;
+    float *d_img = nullptr;
     int lf_ny[MX_MAXWVL] = {}, lf_nx[MX_MAXWVL] = {}; // sampled rows / columns per wavelength
     int *d_lf_rows[MX_MAXWVL] = {}, *d_lf_cols[MX_MAXWVL] = {};
     int4 *d_lf_sic[MX_MAXWVL] = {};
     int lf_maxny = 0, lf_maxnx = 0;    // capacity of B3 and the image per chain
     LfWvl *d_lfw = nullptr;
     LfWvl h_lfw[MX_MAXWVL] = {};
-    LfArgs arg_lf_base{}, arg_lf[5] = {}, arg_lf_up[4] = {};
+    LfArgs arg_lf_base{}, arg_lf[4] = {}, arg_lf_up[3] = {};
     LfSampleArgs arg_lfs{};
     float *d_mtche = nullptr, *d_i0sum = nullptr;
     bool have_mtche = false, have_i0sum = false;
@@ -3178,80 +2997,31 @@ bool supported(long notf, long nxsa, long embfac) {
     return (notf == 64 && nxsa == 32 && embfac == 2) || (notf == 32 && nxsa == 16 && embfac == 2);
 }
 
-// Stockham plan of a line length n <= MX_LF_MAXN whose prime factors are 2,
-// 3, 5 and 7: radix 8 first, then 4, 2, 3, 5, 7.  False if n does not factor so.
-bool lf_plan(long n, LfPlan &P) {
-    P = LfPlan{};
-    if (n < 2 || n > MX_LF_MAXN) return false;
-    P.n = (int)n;
-    long prod = 1;
-    while (P.nrad < MX_LF_MAXRAD && lf_radix((int)n, P.nrad)) {
-        P.rad[P.nrad] = lf_radix((int)n, P.nrad);
-        prod *= P.rad[P.nrad++];
-    }
-    return prod == n;
+// pass q of the large-field form (0..3: A, B, D, E; 4: the uplink's D; 5: E of long columns)
+const void *lf_kernel(int q) {
+    const void *k[6] = {reinterpret_cast<const void *>(&k_lf_a), reinterpret_cast<const void *>(&k_lf_b),
+                        reinterpret_cast<const void *>(&k_lf_d<false>), reinterpret_cast<const void *>(&k_lf_e),
+                        reinterpret_cast<const void *>(&k_lf_d<true>), reinterpret_cast<const void *>(&k_lf_e_wave)};
+    return k[q];
 }
-
-// twiddles exp(-2 pi i r k / (Ns R)) of a plan's stages (k < Ns, 1 <= r <
-// R) appended to tw; sets P.off relative to the plan's first entry
-void lf_twiddles(LfPlan &P, std::vector<float2> &tw) {
-    const size_t base = tw.size();
-    int Ns = 1;
-    for (int s = 0; s < P.nrad; s++) {
-        const int R = P.rad[s];
-        P.off[s] = (int)(tw.size() - base);
-        for (int k = 0; k < Ns; k++)
-            for (int r = 1; r < R; r++) {
-                const double ang = -2. * M_PI * (double)(r * k) / (double)(Ns * R);
-                tw.push_back(make_float2((float)std::cos(ang), (float)std::sin(ang)));
-            }
-        Ns *= R;
-    }
-}
-
-// pass q (0..4 = A..E) of the large-field form for blocks of T threads and
-// lines of length n: a kernel compiled for that length where there is one
-// (the field and OTF sizes of the configured NGS and padded-LGS powfs)
-template <int T, int N>
-const void *lf_kernel_ab(int q) {
-    return q == 0 ? reinterpret_cast<const void *>(&k_lf_a<T, N>) : reinterpret_cast<const void *>(&k_lf_b<T, N>);
-}
-template <int T, int N>
-const void *lf_kernel_cde(int q) {
-    return q == 2 ? reinterpret_cast<const void *>(&k_lf_c<T, N>)
-                  : q == 3 ? reinterpret_cast<const void *>(&k_lf_d<T, N, false>)
-                  : q == 5 ? reinterpret_cast<const void *>(&k_lf_d<T, N, true>)
-                           : reinterpret_cast<const void *>(&k_lf_e<T, N>);
-}
-template <int T>
-const void *lf_kernel_t(int q, int n) {
-    if constexpr (T == 512) {
-        if (q < 2) {
-            if (n == 96) return lf_kernel_ab<T, 96>(q);
-            if (n == 128) return lf_kernel_ab<T, 128>(q);
-            if (n == 480) return lf_kernel_ab<T, 480>(q);
-            if (n == 960) return lf_kernel_ab<T, 960>(q);
-        } else {
-            if (n == 120) return lf_kernel_cde<T, 120>(q);
-            if (n == 128) return lf_kernel_cde<T, 128>(q);
-            if (n == 512) return lf_kernel_cde<T, 512>(q);
-            if (n == 1024) return lf_kernel_cde<T, 1024>(q);
-        }
-    }
-    return q < 2 ? lf_kernel_ab<T, 0>(q) : lf_kernel_cde<T, 0>(q);
-}
-// q: 0..4 passes A..E, 5 the uplink's column pass
-const void *lf_kernel(int q, int T, int n) {
-    return T == 128 ? lf_kernel_t<128>(q, n) : T == 256 ? lf_kernel_t<256>(q, n) : lf_kernel_t<512>(q, n);
+// lines per block of a pass over nlines lines of n points in each of nchain
+// chains: a power of two up to 16 of at most 16 points for each of `threads`
+// threads (4096 points at 256, about 35 KB of LDS), fewer while that leaves
+// less than two blocks for a CU, but at least lmin.
+int lf_lines(int n, int nlines, int nchain, int threads, int lmin) {
+    int L = 16;
+    while (L > lmin && L * n > 16 * threads) L /= 2;
+    while (L > lmin && (long)((nlines + L - 1) / L) * nchain < 512) L /= 2;
+    return L;
 }
 
 // the large-field form applies: OPD grid a multiple of 16 points, even
 // field and OTF sizes that plan, notf >= nwvf (ccpcorner pads)
 bool lf_supported(long notf, long nxsa, long embfac) {
-    LfPlan a, b;
+    LinePlan a, b;
     const long nwvf = nxsa * embfac;
     return nxsa >= 16 && nxsa % 16 == 0 && embfac >= 1 && nwvf % 2 == 0 && notf % 2 == 0 && notf >= nwvf &&
-           lf_plan(nwvf, a) && lf_plan(notf, b);
+           notf <= MX_LF_MAXN && lx_plan(nwvf, a) && lx_plan(notf, b);
 }
 
 // FP32 -> BF16 with round-to-nearest-even (finite inputs)
@@ -3482,18 +3252,17 @@ int mx_wfsgrad_init_batch(mx_wfsgrad_t **out, const mx_powfs_t *p, const mx_wfs_
     h->lf = lf;
     std::vector<float2> lf_tw;
     if (lf) {
-        lf_plan(h->nwvf, h->lf_pn);
-        lf_plan(N, h->lf_pm);
-        lf_twiddles(h->lf_pn, lf_tw);
+        lx_plan(h->nwvf, h->lf_pn);
+        lx_plan(N, h->lf_pm);
+        lx_twiddles(h->nwvf, lf_tw);
         const size_t nt_n = lf_tw.size();
-        lf_twiddles(h->lf_pm, lf_tw);
+        lx_twiddles(N, lf_tw);
         const long nchain = (long)nwfs * nsa * h->nwvl;
         ALLOC(h->d_lf_tw, lf_tw.size());
         h->lf_pn.tw = h->d_lf_tw;
         h->lf_pm.tw = h->d_lf_tw + nt_n;
         ALLOC(h->d_b1, nchain * h->nxsa * h->nwvf);
-        ALLOC(h->d_psf, nchain * h->nwvf * h->nwvf);
-        ALLOC(h->d_b2, nchain * h->nwvf * N);
+        ALLOC(h->d_b2, nchain * h->nwvf * (N / 2 + 1));
         ALLOC(h->d_lfw, MX_MAXWVL);
     }
     if (p->llt_nx > 0) {
@@ -3638,7 +3407,7 @@ int mx_wfsgrad_free(mx_wfsgrad_t *h) {
     if (h->stream2) hipStreamSynchronize(h->stream2);
     drop_graph(h);
     void *ptrs[] = {h->d_ptsx, h->d_ptsy, h->d_amp, h->d_saa, h->d_wfs, h->d_wv, h->d_llt_amp, h->d_llt_opd, h->d_lotf,
-                    h->d_lotf_t, h->d_F, h->d_F16, h->d_mwv, h->d_imcc, h->d_opdadd, h->d_ptt, h->d_lf_tw, h->d_b1, h->d_b2, h->d_b3, h->d_psf, h->d_img,
+                    h->d_lotf_t, h->d_F, h->d_F16, h->d_mwv, h->d_imcc, h->d_opdadd, h->d_ptt, h->d_lf_tw, h->d_b1, h->d_b2, h->d_b3, h->d_img,
                     h->d_lfw,
                     h->d_mtche, h->d_i0sum, h->d_ints, h->d_grad, h->d_opd, h->d_i0acc,
                     h->d_imb, h->d_imx, h->d_imy, h->d_fi0, h->d_fgx, h->d_fgy, h->d_mi0, h->d_mgx, h->d_mgy,
@@ -3731,7 +3500,8 @@ int set_dtf_tables(mx_wfsgrad_t *h, int iwvl, long ntab, const double *nominal, 
     HIPCHK(hipMemcpy(h->d_si_w[iwvl], wt.data(), sizeof(float4) * ntab * npix, hipMemcpyHostToDevice));
     if (nominal && h->cfg.llt_nx == 0) {
         if ((rc = dev_alloc(&h->d_nominal[iwvl], ntab * N * N))) return rc;
-        // The large-field form transforms only the columns ux <= N/2 and takes
+        // (Stored [uy][ux] for the large-field form, whose rows it multiplies.)
+        // The large-field form transforms only the rows uy <= N/2 and takes
         // the rest as conjugates, which gives MAOS's real part of the inverse
         // transform exactly when the nominal is even: (n(u) + n(-u)) / 2 is
         // stored for it (the same real part for any nominal; rotated pixels
@@ -3742,8 +3512,10 @@ int set_dtf_tables(mx_wfsgrad_t *h, int iwvl, long ntab, const double *nominal, 
                 for (long ux = 0; ux < N; ux++) {
                     const double *nm = nominal + t * N * N;
                     const double v = nm[ux + uy * N];
-                    nt[t * N * N + ux * N + uy] =
-                        h->lf ? (float)(0.5 * (v + nm[(N - ux) % N + (N - uy) % N * N])) : (float)v;
+                    if (h->lf)
+                        nt[t * N * N + uy * N + ux] = (float)(0.5 * (v + nm[(N - ux) % N + (N - uy) % N * N]));
+                    else
+                        nt[t * N * N + ux * N + uy] = (float)v;
                 }
         HIPCHK(hipMemcpy(h->d_nominal[iwvl], nt.data(), sizeof(float) * ntab * N * N, hipMemcpyHostToDevice));
     }
@@ -3856,7 +3628,7 @@ int set_dtf_tables(mx_wfsgrad_t *h, int iwvl, long ntab, const double *nominal, 
             h->d_b3 = nullptr;
             h->d_img = nullptr;
             h->lf_maxny = h->lf_maxnx = 0;
-            if ((rc = dev_alloc(&h->d_b3, (size_t)nchain * maxny * N)) ||
+            if ((rc = dev_alloc(&h->d_b3, (size_t)nchain * maxnx * (N / 2 + 1))) ||
                 (rc = dev_alloc(&h->d_img, (size_t)nchain * maxny * maxnx)))
                 return rc;
             h->lf_maxny = maxny;
@@ -3902,7 +3674,10 @@ int mx_wfsgrad_update_etf(mx_wfsgrad_t *h, int iwvl, const double *etf, const do
             }
             continue;
         }
-        for (long isa = 0; isa < nsa; isa++) transpose_c(t.data() + isa * N * N, src + 2 * isa * N * N, N, false);
+        if (h->lf) // the large-field form keeps the ETF as given, [uy][ux]
+            for (long i = 0; i < nsa * N * N; i++) t[i] = make_float2((float)src[2 * i], (float)src[2 * i + 1]);
+        else
+            for (long isa = 0; isa < nsa; isa++) transpose_c(t.data() + isa * N * N, src + 2 * isa * N * N, N, false);
         float2 **dst = which ? &h->d_etf2[iwvl] : &h->d_etf[iwvl];
         if ((rc = dev_alloc(dst, nsa * N * N))) return rc;
         HIPCHK(hipMemcpy(*dst, t.data(), sizeof(float2) * nsa * N * N, hipMemcpyHostToDevice));
@@ -4069,6 +3844,33 @@ int mx_dm2gpu_real(int ireal, const mx_atm_layer_t *dms, int ndm) {
 int mx_dm2gpu(const mx_atm_layer_t *dms, int ndm) { return mx_dm2gpu_real(0, dms, ndm); }
 
 } // extern "C"
+
+// launch of pass q (0..3: A, B, D, E; up: the uplink's D) over u's chains,
+// its lines per block set in u
+StepLaunch lf_launch(const mx_wfsgrad_t *h, LfArgs &u, int q, bool up) {
+    const int n = u.nwvf, m = u.notf, mh = m / 2 + 1, T = h->lf_threads;
+    if (q == 3 && mh > MX_LF_ESHORT) {
+        StepLaunch e{lf_kernel(5), dim3((unsigned)((u.maxny * u.maxnx + 3) / 4 * u.nchain)), dim3(256), &u};
+        return e;
+    }
+    if (q == 3) {
+        const int XG = lf_ecols(mh);
+        StepLaunch e{lf_kernel(3), dim3((unsigned)((u.maxnx + XG - 1) / XG * u.nchain)), dim3(256), &u};
+        return e;
+    }
+    const int nlines = q == 0 ? u.nxsa : q == 1 ? n : mh;
+    // (pass B pairs columns; pass D writes runs of L along uy)
+    u.L = lf_lines(q == 2 ? m : n, nlines, u.nchain, T, q == 0 ? 1 : 2);
+    u.lgL = ilog2c(u.L);
+    int threads = lx_threads(q == 2 ? u.pm : u.pn, u.L), elems = u.L * (q == 2 ? u.pm.S : u.pn.S);
+    if (q == 1) {
+        threads = std::max(threads, lx_threads(u.pm, u.L / 2));
+        elems = std::max(elems, u.L / 2 * u.pm.S);
+    }
+    StepLaunch e{lf_kernel(up ? 4 : q), dim3((unsigned)((nlines + u.L - 1) / u.L * u.nchain)), dim3((unsigned)threads), &u};
+    e.lds = (unsigned)(sizeof(float2) * elems);
+    return e;
+}
 
 namespace {
 // Check the engine's state and fill its argument blocks and kernel list for
@@ -4432,7 +4234,7 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
     if (h->lf) {
         LfWvl hw[MX_MAXWVL] = {};
         for (int w = 0; w < h->nwvl; w++) {
-            hw[w].inv_wvl = (float)(1. / h->wvl[w]);
+            hw[w].inv_wvl64 = 1. / h->wvl[w];
             hw[w].nominal = h->d_nominal[w];
             hw[w].ny = h->lf_ny[w];
             hw[w].nx = h->lf_nx[w];
@@ -4470,7 +4272,6 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
         f.b1 = h->d_b1;
         f.b2 = h->d_b2;
         f.b3 = h->d_b3;
-        f.psf = h->d_psf;
         f.img = h->d_img;
         f.psf_scale = 1.f;
         f.lotf = llt ? h->d_lotf : nullptr;
@@ -4479,19 +4280,10 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
     }
     const int slot_llt = llt && !pre_hit ? nl : -1;
     if (llt && h->lf) {
-        // uplink OTF of each (WFS, wavelength) by passes A-C and the uplink
-        // column pass on the LLT grids (nlwvf == nwvf == notf); pass C takes
-        // the PSF rows two at a time, the column passes the columns <= N/2
-        const int Ln = lf_lines((int)h->nwvf), Lm = lf_lines((int)N), nch = (int)(h->nwfs * h->nwvl);
-        const int nph = (int)(h->nwvf / 2), mh = (int)(N / 2 + 1);
-        const int nlx = (int)h->cfg.llt_nx;
-        const struct {
-            int q, len, L, ngroup;
-        } up[4] = {{0, (int)h->nwvf, Ln, (nlx + Ln - 1) / Ln},
-                   {1, (int)h->nwvf, Ln, (int)((h->nwvf + Ln - 1) / Ln)},
-                   {2, (int)N, Lm, (nph + Lm - 1) / Lm},
-                   {5, (int)N, Lm, (mh + Lm - 1) / Lm}};
-        for (int q = 0; q < 4; q++) {
+        // uplink OTF of each (WFS, wavelength) by passes A, B and the uplink's
+        // D on the LLT grids (nlwvf == nwvf == notf)
+        const int nch = (int)(h->nwfs * h->nwvl), nlx = (int)h->cfg.llt_nx;
+        for (int q = 0; q < 3; q++) {
             LfArgs &u = h->arg_lf_up[q];
             u = h->arg_lf_base;
             u.nsa = 1;
@@ -4500,10 +4292,7 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
             u.opd = h->d_llt_opd;
             u.amp = h->d_llt_amp;
             u.psf_scale = (float)(1. / ((double)h->nwvf * (double)h->nwvf));
-            u.L = up[q].L;
-            u.lgL = ilog2c(up[q].L);
-            L[nl++] = {lf_kernel(up[q].q, h->lf_threads, up[q].len), dim3((unsigned)(up[q].ngroup * nch)),
-                       dim3((unsigned)h->lf_threads), &u};
+            L[nl++] = lf_launch(h, u, q, q == 2);
         }
     } else if (llt && !pre_hit && uplink_direct) {
         LltAcorrArgs &u = h->arg_lltac;
@@ -4540,24 +4329,9 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
     const int slot_img = nl;
     if (h->lf) {
         const LfArgs &f = h->arg_lf_base;
-        const int Ln = lf_lines((int)h->nwvf), Lm = lf_lines((int)N);
-        const int nph = (int)(h->nwvf / 2), mh = (int)(N / 2 + 1);
-        // pass: kernel, lines per block, line groups per chain (pass C: pairs
-        // of PSF rows; pass D: the columns <= N/2)
-        const struct {
-            const void *k;
-            int L, ngroup;
-        } pass[5] = {{lf_kernel(0, h->lf_threads, (int)h->nwvf), Ln, (int)((h->nxsa + Ln - 1) / Ln)},
-                     {lf_kernel(1, h->lf_threads, (int)h->nwvf), Ln, (int)((h->nwvf + Ln - 1) / Ln)},
-                     {lf_kernel(2, h->lf_threads, (int)N), Lm, (nph + Lm - 1) / Lm},
-                     {lf_kernel(3, h->lf_threads, (int)N), Lm, (mh + Lm - 1) / Lm},
-                     {lf_kernel(4, h->lf_threads, (int)N), Lm, (h->lf_maxny + Lm - 1) / Lm}};
-        const dim3 blk((unsigned)h->lf_threads);
-        for (int q = 0; q < 5; q++) {
+        for (int q = 0; q < 4; q++) {
             h->arg_lf[q] = f;
-            h->arg_lf[q].L = pass[q].L;
-            h->arg_lf[q].lgL = ilog2c(pass[q].L);
-            L[nl++] = {pass[q].k, dim3((unsigned)(pass[q].ngroup * f.nchain)), blk, &h->arg_lf[q]};
+            L[nl++] = lf_launch(h, h->arg_lf[q], q, false);
         }
         LfSampleArgs &g = h->arg_lfs;
         g = LfSampleArgs{};
@@ -4768,7 +4542,7 @@ void node_params(const StepPlan &sp, hipKernelNodeParams *kp, void *(*argv)[1]) 
         kp[i].func = const_cast<void *>(sp.L[i].f);
         kp[i].gridDim = sp.L[i].grid;
         kp[i].blockDim = sp.L[i].block;
-        kp[i].sharedMemBytes = 0;
+        kp[i].sharedMemBytes = sp.L[i].lds;
         kp[i].kernelParams = argv[i];
         kp[i].extra = nullptr;
     }
@@ -4801,7 +4575,7 @@ int launch_step(mx_wfsgrad_t *h, const StepPlan &in) {
     HIPCHK(hipStreamWaitEvent(h->stream2, h->ev_main, 0));
     for (int i = in.nmain; i < in.nl; i++) {
         void *argv[1] = {in.L[i].arg};
-        HIPCHK(hipLaunchKernel(in.L[i].f, in.L[i].grid, in.L[i].block, argv, 0, h->stream2));
+        HIPCHK(hipLaunchKernel(in.L[i].f, in.L[i].grid, in.L[i].block, argv, in.L[i].lds, h->stream2));
     }
     HIPCHK(hipEventRecord(h->ev_branch, h->stream2));
     h->branch_pending = true;
@@ -4862,7 +4636,7 @@ int launch_chain(mx_wfsgrad_t *h, const StepPlan &sp) {
                                                                    : nullptr;
             if (h->timing && eb) HIPCHK(hipEventRecord(eb, h->stream));
             void *argv[1] = {L[i].arg};
-            HIPCHK(hipLaunchKernel(L[i].f, L[i].grid, L[i].block, argv, 0, h->stream));
+            HIPCHK(hipLaunchKernel(L[i].f, L[i].grid, L[i].block, argv, L[i].lds, h->stream));
             if (h->timing && ee) HIPCHK(hipEventRecord(ee, h->stream));
         }
         if (h->timing) {
@@ -5348,9 +5122,9 @@ int mx_wfsgrad_debug_lotf(mx_wfsgrad_t *h, int iwfs, int iwvl, double *lotf) {
                      hipMemcpyDeviceToHost));
     for (long ux = 0; ux < N; ux++)
         for (long uy = 0; uy < N; uy++) {
-            // the large-field form stores ux <= N/2; lotf(-u) = conj lotf(u)
-            const bool mirror = h->lf && ux > N / 2;
-            const float2 v = mirror ? t[(N - ux) * N + (N - uy) % N] : t[ux * N + uy];
+            // the large-field form stores [uy][ux] for uy <= N/2; lotf(-u) = conj lotf(u)
+            const bool mirror = h->lf && uy > N / 2;
+            const float2 v = mirror ? t[(N - uy) * N + (N - ux) % N] : h->lf ? t[uy * N + ux] : t[ux * N + uy];
             lotf[2 * (ux + uy * N)] = v.x;
             lotf[2 * (ux + uy * N) + 1] = mirror ? v.y : -v.y; // stored conjugated
         }
