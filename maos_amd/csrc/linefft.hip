@@ -65,6 +65,14 @@ __device__ __forceinline__ int qdiv(int a, int b, float rb) {
     return q;
 }
 
+// x k for a constant k, as if k were not rounded to FP32: the rounding of a
+// root of unity shifts the gain of every transform alike (the radix-3 sine by
+// 2e-8 a stage, 5e-7 of an intensity after the 24 stages of a pyramid's 2916^2
+// grid), where everything else is random
+__device__ __forceinline__ float mulk(float x, double k) {
+    return fmaf(x, (float)k, x * (float)(k - (double)(float)k));
+}
+__device__ __forceinline__ float2 mulk2(float2 z, double k) { return make_float2(mulk(z.x, k), mulk(z.y, k)); }
 __device__ __forceinline__ float2 mul_ti(float2 z, float t) { return make_float2(-t * z.y, t * z.x); }
 // v[q] <- sum_r v[r] exp(t 2 pi i r q / R), t = +-1
 template <int R>
@@ -83,32 +91,32 @@ __device__ __forceinline__ void small_dft(float2 (&v)[R], float t) {
     } else if constexpr (R == 8) {
         // even and odd halves by 4-point transforms, then w8^q = exp(t 2 pi i q / 8)
         // on the odd half: w8 = (1 + t i) / sqrt 2, w8^2 = t i, w8^3 = (-1 + t i) / sqrt 2
-        const float h = 0.70710678118654752f;
+        const double h = 0.70710678118654752440;
         float2 e[4] = {v[0], v[2], v[4], v[6]}, o[4] = {v[1], v[3], v[5], v[7]};
         small_dft<4>(e, t);
         small_dft<4>(o, t);
         const float2 o1 = mul_ti(o[1], t), o3 = mul_ti(o[3], t);
-        o[1] = make_float2(h * (o[1].x + o1.x), h * (o[1].y + o1.y));
+        o[1] = mulk2(cadd(o[1], o1), h);
         o[2] = mul_ti(o[2], t);
-        o[3] = make_float2(h * (o3.x - o[3].x), h * (o3.y - o[3].y));
+        o[3] = mulk2(csub(o3, o[3]), h);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             v[q] = cadd(e[q], o[q]);
             v[q + 4] = csub(e[q], o[q]);
         }
     } else if constexpr (R == 3) {
-        const float h = 0.86602540378443865f; // sqrt(3)/2
+        const double h = 0.86602540378443864676; // sqrt(3)/2
         const float2 s = cadd(v[1], v[2]), d = csub(v[1], v[2]);
         const float2 m = make_float2(v[0].x - 0.5f * s.x, v[0].y - 0.5f * s.y);
-        const float2 r = mul_ti(make_float2(h * d.x, h * d.y), t);
+        const float2 r = mul_ti(mulk2(d, h), t);
         v[0] = cadd(v[0], s);
         v[1] = cadd(m, r);
         v[2] = csub(m, r);
     } else if constexpr (R == 7) {
         // pairs r, 7 - r: v[k] = v0 + sum_r cos(2 pi r k / 7) (v[r] + v[7-r])
         //                      + t i sum_r sin(2 pi r k / 7) (v[r] - v[7-r])
-        constexpr float c[4] = {1.f, 0.62348980185873353f, -0.22252093395631440f, -0.90096886790241913f};
-        constexpr float sn[4] = {0.f, 0.78183148246802981f, 0.97492791218182361f, 0.43388373911755812f};
+        constexpr double c[4] = {1., 0.62348980185873353053, -0.22252093395631440429, -0.90096886790241912624};
+        constexpr double sn[4] = {0., 0.78183148246802980871, 0.97492791218182360702, 0.43388373911755812048};
         float2 a[4], b[4];
 #pragma unroll
         for (int r = 1; r <= 3; r++) {
@@ -122,9 +130,9 @@ __device__ __forceinline__ void small_dft(float2 (&v)[R], float t) {
 #pragma unroll
             for (int r = 1; r <= 3; r++) {
                 const int m = (r * k) % 7; // cos(2 pi m / 7), sin of it with the sign of m <= 3
-                const float cm = c[m <= 3 ? m : 7 - m], sm = m <= 3 ? sn[m] : -sn[7 - m];
-                p = make_float2(p.x + cm * a[r].x, p.y + cm * a[r].y);
-                q = make_float2(q.x + sm * b[r].x, q.y + sm * b[r].y);
+                const double cm = c[m <= 3 ? m : 7 - m], sm = m <= 3 ? sn[m] : -sn[7 - m];
+                p = cadd(p, mulk2(a[r], cm));
+                q = cadd(q, mulk2(b[r], sm));
             }
             q = mul_ti(q, t);
             v[k] = cadd(p, q);
@@ -132,14 +140,14 @@ __device__ __forceinline__ void small_dft(float2 (&v)[R], float t) {
         }
         v[0] = cadd(v0, cadd(a[1], cadd(a[2], a[3])));
     } else { // 5: cos and sin of 2 pi/5 and 4 pi/5
-        const float c1 = 0.30901699437494742f, c2 = -0.80901699437494742f;
-        const float s1 = 0.95105651629515357f, s2 = 0.58778525229247313f;
+        const double c1 = 0.30901699437494742410, c2 = -0.80901699437494742410;
+        const double s1 = 0.95105651629515357212, s2 = 0.58778525229247312917;
         const float2 a1 = cadd(v[1], v[4]), a2 = cadd(v[2], v[3]);
         const float2 b1 = csub(v[1], v[4]), b2 = csub(v[2], v[3]);
-        const float2 p1 = make_float2(v[0].x + c1 * a1.x + c2 * a2.x, v[0].y + c1 * a1.y + c2 * a2.y);
-        const float2 p2 = make_float2(v[0].x + c2 * a1.x + c1 * a2.x, v[0].y + c2 * a1.y + c1 * a2.y);
-        const float2 q1 = mul_ti(make_float2(s1 * b1.x + s2 * b2.x, s1 * b1.y + s2 * b2.y), t);
-        const float2 q2 = mul_ti(make_float2(s2 * b1.x - s1 * b2.x, s2 * b1.y - s1 * b2.y), t);
+        const float2 p1 = cadd(v[0], cadd(mulk2(a1, c1), mulk2(a2, c2)));
+        const float2 p2 = cadd(v[0], cadd(mulk2(a1, c2), mulk2(a2, c1)));
+        const float2 q1 = mul_ti(cadd(mulk2(b1, s1), mulk2(b2, s2)), t);
+        const float2 q2 = mul_ti(csub(mulk2(b1, s2), mulk2(b2, s1)), t);
         v[0] = cadd(v[0], cadd(a1, a2));
         v[1] = cadd(p1, q1);
         v[4] = csub(p1, q1);
@@ -152,7 +160,7 @@ __device__ __forceinline__ void small_dft(float2 (&v)[R], float t) {
 // of the angle reduced to [-pi, pi])
 template <int R>
 struct LxRoots {
-    float c[R], s[R];
+    double c[R], s[R];
     constexpr LxRoots() : c(), s() {
         for (int m = 0; m < R; m++) {
             const double x = 6.283185307179586476925 * (2 * m > R ? m - R : m) / R;
@@ -163,8 +171,8 @@ struct LxRoots {
                 sc += tc;
                 ss += ts;
             }
-            c[m] = (float)sc;
-            s[m] = (float)ss;
+            c[m] = sc;
+            s[m] = ss;
         }
     }
 };
@@ -183,8 +191,12 @@ __device__ __forceinline__ void comp_dft(float2 (&v)[R1 * R2]) {
         small_dft<R1>(u, t);
 #pragma unroll
         for (int k1 = 0; k1 < R1; k1++)
-            a[n2][k1] = n2 * k1 ? cmul(u[k1], make_float2(W.c[(n2 * k1) % (R1 * R2)], t * W.s[(n2 * k1) % (R1 * R2)]))
-                                : u[k1];
+            if (n2 * k1) {
+                const double c = W.c[(n2 * k1) % (R1 * R2)], s = t * W.s[(n2 * k1) % (R1 * R2)];
+                a[n2][k1] = make_float2(mulk(u[k1].x, c) - mulk(u[k1].y, s), mulk(u[k1].x, s) + mulk(u[k1].y, c));
+            } else {
+                a[n2][k1] = u[k1];
+            }
     }
 #pragma unroll
     for (int k1 = 0; k1 < R1; k1++) {
@@ -232,7 +244,7 @@ __device__ __forceinline__ void lx_stage(float2 *s, LxPlan P, const LxLines &g, 
     constexpr int PER = lx_per(R);
     const int nb = P->nb[i], total = g.L * nb, T = (int)blockDim.x;
     const float rnb = 1.f / (float)nb, rns = 1.f / (float)Ns;
-    float2 v[PER][R], w[PER][R]; // (the twiddles' loads are in flight across the barrier)
+    float2 v[PER][R];
 #pragma unroll
     for (int p = 0; p < PER; p++) {
         const int it = (int)threadIdx.x + p * T;
@@ -243,10 +255,7 @@ __device__ __forceinline__ void lx_stage(float2 *s, LxPlan P, const LxLines &g, 
 #pragma unroll
                 for (int r = 0; r < R; r++) v[p][r] = ld(l, j, r * nb);
             } else {
-                const int q = qdiv(j, Ns, rns), t = __mul24(j - __mul24(q, Ns), P->ts[i]);
-                int tm = t;
-#pragma unroll
-                for (int m = 1; m < R; m++, tm += t) w[p][m] = lx_at(P->tw, tm);
+                const int q = qdiv(j, Ns, rns);
                 const float2 *x = s + __mul24(l, P->S) + j + __mul24(q, P->pad[i - 1]);
 #pragma unroll
                 for (int r = 0; r < R; r++) v[p][r] = x[r * P->rstep[i]];
@@ -262,8 +271,13 @@ __device__ __forceinline__ void lx_stage(float2 *s, LxPlan P, const LxLines &g, 
             lx_item<MAP>(it, nb, rnb, g, l, j);
             const int q = FIRST ? j : qdiv(j, Ns, rns), k = FIRST ? 0 : j - __mul24(q, Ns);
             if constexpr (!FIRST) {
+                const int t = __mul24(k, P->ts[i]);
+                int tm = t;
 #pragma unroll
-                for (int m = 1; m < R; m++) v[p][m] = cmul(v[p][m], make_float2(w[p][m].x, INV ? -w[p][m].y : w[p][m].y));
+                for (int m = 1; m < R; m++, tm += t) {
+                    const float2 w = lx_at(P->tw, tm);
+                    v[p][m] = cmul(v[p][m], make_float2(w.x, INV ? -w.y : w.y));
+                }
             }
             lx_dft<R, INV>(v[p]);
             if constexpr (LAST) {
@@ -301,6 +315,27 @@ __device__ __forceinline__ void lx_fft(float2 *s, LxPlan P, const LxLines &g, LD
         Ns *= P->rad[i];
     }
 #define LX_CASE(R) case R: lx_stage<R, INV, false, true, MO, false>(s, P, g, i, Ns, ld, st); break;
+    switch (P->rad[i]) { LX_CASE(1) LX_RADIX(LX_CASE) default: break; }
+#undef LX_CASE
+}
+
+// f(l, d, off, slot) for every point that lx_fft's last stage hands this
+// thread by map MO (the last span is the line, so d is the butterfly)
+template <int MO, class F>
+__device__ __forceinline__ void lx_outputs(LxPlan P, const LxLines &g, F &&f) {
+    const int i = P->nst - 1, nb = P->nb[i], total = g.L * nb;
+    const float rnb = 1.f / (float)nb;
+#define LX_CASE(R)                                                                                                   \
+    case R:                                                                                                          \
+        _Pragma("unroll") for (int p = 0; p < lx_per(R); p++) {                                                      \
+            const int it = (int)threadIdx.x + p * (int)blockDim.x;                                                   \
+            if (it < total) {                                                                                        \
+                int l, j;                                                                                            \
+                lx_item<MO>(it, nb, rnb, g, l, j);                                                                   \
+                _Pragma("unroll") for (int r = 0; r < R; r++) f(l, j, r * nb, p * R + r);                            \
+            }                                                                                                        \
+        }                                                                                                            \
+        break;
     switch (P->rad[i]) { LX_CASE(1) LX_RADIX(LX_CASE) default: break; }
 #undef LX_CASE
 }

@@ -12,269 +12,208 @@
 //           inverse FFT;
 //   sample  bilinear at every subaperture centre of each pupil image;
 //   grads   the quad-cell (or three-facet) combination, flux-normalised.
-// Every 2-D transform is a pass of line FFTs along the contiguous axis
-// (Stockham stages in LDS, radices 8, 4, 2, 3, 5, 7: lds_fft_rt), a 32 x 32
-// tiled transpose, and a second line pass; the orientation alternates so
-// that each pass reads and writes whole rows.  Layouts are [row][column]
-// with the column contiguous; "transposed" arrays hold [x][y].
-constexpr int MX_LF_MAXRAD = 12;
-constexpr int MX_LF_LDS = 4352;    // complex elements of one LDS line buffer
-// LDS position of element e of a line: one pad element after every 32, so
-// that the power-of-two write strides of the early Stockham stages spread
-// over the LDS banks
-__host__ __device__ constexpr int lf_pos(int e) { return e + (e >> 5); }
-// LDS stride of lines of length n: the padded length, made odd
-__host__ __device__ constexpr int lf_stride(int n) { return lf_pos(n) | 1; }
-// lines of length n per block: a power of two <= 32 that one buffer holds;
-// for lines of 768 and more at most 2048 / n of them, so that a one-chain
-// plane (the 960^2 and 1024^2 tip-tilt sizes: 2 lines, 480-512 blocks)
-// spreads over more blocks than CUs (53 -> 46 us per step for the 1024^2
-// tip-tilt imaging; the 512^2 planes, with many chains, keep 8 lines)
-__host__ __device__ constexpr int pyl_lines(int n) {
-    int L = 32;
-    while (L > 1 && (L * lf_stride(n) > MX_LF_LDS || (n >= 768 && L * n > 2048))) L /= 2;
-    return L;
-}
-// radix of stage s in the plan of n (radix 8 first, then 4, 2, 3, 5, 7); 0
-// past the last stage or if n has another prime factor
-__host__ __device__ constexpr int lf_radix(int n, int s) {
-    const int rad[6] = {8, 4, 2, 3, 5, 7};
-    int r = n, c = 0;
-    for (int k = 0; k < 6; k++)
-        while (r > 1 && r % rad[k] == 0) {
-            if (c == s) return rad[k];
-            c++;
-            r /= rad[k];
-        }
-    return 0;
-}
-
-struct LfPlan {
-    int n, nrad;
-    int rad[MX_LF_MAXRAD]; // lf_radix(n, s)
-    int off[MX_LF_MAXRAD]; // twiddle offset of each stage
-    const float2 *tw;      // stage s: exp(-2 pi i r k / (Ns R)) at off[s] + k (R-1) + r-1
-};
-// a / b: by the compiler when b is a constant (CT), else by qdiv
-template <bool CT>
-__device__ __forceinline__ int ldiv(int a, int b, float rb) {
-    if constexpr (CT) return a / b;
-    else return qdiv(a, b, rb);
-}
-
-// One Stockham stage of radix R and span Ns over L lines (line l at l S,
-// element e at lf_pos(e)) by a block of T threads: item (l, j), j < n/R,
-// takes x[j + r n/R] times w^(r k) (w = exp(-+ 2 pi i / (Ns R)), k = j % Ns),
-// transforms and writes x'[(j/Ns) Ns R + k + r Ns].  CT: n, Ns and L are
-// compile-time constants.  Forward is FFTW_FORWARD (exp(-i ...)).
-template <int R, bool INV, bool CT, int T>
-__device__ __forceinline__ void lds_stage(const float2 *src, float2 *dst, int n, int Ns, int L, int S,
-                                          const float2 *tw) {
-    const int nb = n / R, total = L * nb;
-    const float rnb = 1.f / (float)nb, rns = 1.f / (float)Ns;
-    for (int it = (int)threadIdx.x; it < total; it += T) {
-        const int l = ldiv<CT>(it, nb, rnb), j = it - l * nb;
-        const int g = ldiv<CT>(j, Ns, rns), k = j - g * Ns;
-        const float2 *x = src + l * S;
-        const float2 *w = tw + k * (R - 1);
-        float2 v[R];
-        v[0] = x[lf_pos(j)];
-#pragma unroll
-        for (int r = 1; r < R; r++) {
-            float2 wr = w[r - 1];
-            if (INV) wr.y = -wr.y;
-            v[r] = cmul(x[lf_pos(j + r * nb)], wr);
-        }
-        small_dft<R>(v, INV ? 1.f : -1.f);
-        float2 *y = dst + l * S;
-        const int d = g * Ns * R + k;
-#pragma unroll
-        for (int r = 0; r < R; r++) y[lf_pos(d + r * Ns)] = v[r];
-    }
-}
-
-// Stockham autosort FFT of L lines of length P.n in src; returns the buffer
-// that holds the result (src or dst).  Stages from the plan at run time.
-template <bool INV, int T>
-__device__ float2 *lds_fft_rt(float2 *src, float2 *dst, const LfPlan &P, int L, int S) {
-    int Ns = 1;
-    for (int s = 0; s < P.nrad; s++) {
-        const int R = P.rad[s];
-        const float2 *tw = P.tw + P.off[s];
-        if (R == 8) lds_stage<8, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        else if (R == 4) lds_stage<4, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        else if (R == 2) lds_stage<2, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        else if (R == 3) lds_stage<3, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        else if (R == 5) lds_stage<5, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        else lds_stage<7, INV, false, T>(src, dst, P.n, Ns, L, S, tw);
-        __syncthreads();
-        float2 *t = src;
-        src = dst;
-        dst = t;
-        Ns *= R;
-    }
-    return src;
-}
-// twiddles exp(-2 pi i r k / (Ns R)) of a plan's stages (k < Ns, 1 <= r <
-// R) appended to tw; sets P.off relative to the plan's first entry
-inline void lf_twiddles(LfPlan &P, std::vector<float2> &tw) {
-    const size_t base = tw.size();
-    int Ns = 1;
-    for (int s = 0; s < P.nrad; s++) {
-        const int R = P.rad[s];
-        P.off[s] = (int)(tw.size() - base);
-        for (int k = 0; k < Ns; k++)
-            for (int r = 1; r < R; r++) {
-                const double ang = -2. * M_PI * (double)(r * k) / (double)(Ns * R);
-                tw.push_back(make_float2((float)std::cos(ang), (float)std::sin(ang)));
-            }
-        Ns *= R;
-    }
-}
+// Every 2-D transform is a row pass and a column pass of line FFTs in LDS
+// (linefft.hip): rows are read and written whole, columns L adjacent ones at
+// a time.  Layouts are [row][column] with the column contiguous;
+// "transposed" arrays hold [x][y].
+//
+// The modulation positions go through in batches: one launch transforms the
+// rows of a batch's masked PSFs into a scratch plane each, one launch takes
+// the columns of those planes and sums |.|^2 over its positions in registers,
+// so the pupil intensity is read and written once for a batch and a small
+// grid still fills the chip (its positions shared out to splits, each with a
+// sum of its own that the detector's first pass adds up).  One position at a
+// time, with a transpose between the passes, the three launches of a 784^2
+// grid took 26 us a position, mostly latency (196 blocks), and those of a
+// 2916^2 grid 191 us, a seventh of them in the transpose.  @@MEAS@@
 constexpr int MX_PY_MAXN = 4096;
-constexpr int MX_PY_T = 1024;
 constexpr int MX_PY_MAXSIDE = 4;
+constexpr int MX_PY_MAXB = 32;              // most positions of a batch
+// bytes of scratch planes that a batch aims at (at least one plane): the
+// rows' mask and PSF reads and the sum's update are shared by a batch (784^2:
+// 32 MB 384 us a step, 64 MB 336, 160 MB 297; 2916^2: 64 MB 4293, 140 MB 4061,
+// 280 MB 3981)
+constexpr long MX_PY_SCRATCH = 256L << 20;
+constexpr int MX_PY_MAXSPLIT = 8;           // most partial pupil intensities
 
 enum PyMode { PY_EMBED = 0, PY_PSF, PY_MOD, PY_ACC, PY_REAL, PY_DTF, PY_IMG };
 
-struct PyRowArgs {
-    LfPlan plan;              // line length n
-    int n, L, S, nrows;       // lines per block, LDS line stride, rows of the pass
+struct PyArgs {
+    LinePlan plan;            // line length n
+    int n, L, lgL, nlines;    // lines per block, lines of the pass
     // PY_EMBED: CSR of the band rows: (x, point) entries, duplicates resolved
     const int *rowp;
     const int2 *ent;
     const float *opd, *amp;
-    float inv_wvl;
-    const float2 *in;         // input rows (all modes but PY_EMBED, PY_REAL)
-    const float *inr;         // PY_REAL: pupil intensity rows
-    float2 *out;              // output rows
-    float *outr;              // PY_ACC: pupil intensity (+=); PY_IMG: image
+    double inv_wvl;
+    const float2 *in;         // input (all modes but PY_EMBED, PY_REAL)
+    const float *inr;         // PY_REAL: the nsplit pupil intensities
+    float2 *out;
+    float *outr;              // PY_ACC: pupil intensities [nsplit][n][n]; PY_IMG: image
     const float2 *mask;       // PY_MOD: pyramid mask, transposed [ux][uy]
-    int ox, oy;               // PY_MOD: modulation offset (samples) of the window in the PSF
-    float scale;              // PY_PSF: PSF normalisation; PY_ACC: weight of |.|^2
+    int y0, y1;               // PY_PSF: rows of the input that hold the field
+    int npos, nsplit, first;  // PY_MOD, PY_ACC: positions of the batch, splits; first: ACC stores, else adds
+    int ox[MX_PY_MAXB], oy[MX_PY_MAXB]; // PY_MOD: modulation offset (samples) of the window in the PSF
+    float wt[MX_PY_MAXB];     // PY_ACC: weight of |.|^2
+    float scale;              // PY_PSF: PSF normalisation
     const float *nomt;        // PY_DTF: detector transfer function, transposed [kx][ky]
 };
+extern __shared__ float2 pyl[];
 
-// L rows of the pass through the LDS line FFT, one block per L rows; the
-// two line buffers (L S complex each) are the block's dynamic LDS.  1024
-// threads take at most one butterfly each per stage at the 2916-point lines
-// of a 30 m pyramid, so the stage's twiddle and line loads overlap across
-// 16 waves rather than queue within a thread.
+// (four waves a SIMD: the 18 points a thread holds and their twiddles)
 template <int MODE>
-__global__ __launch_bounds__(MX_PY_T) __attribute__((amdgpu_waves_per_eu(8))) void k_py_rows(PyRowArgs a) {
-    extern __shared__ float2 pyl[];
-    const int n = a.n, L = a.L, S = a.S, tid = threadIdx.x;
-    float2 *const X = pyl, *const Y = pyl + L * S;
-    const int r0 = (int)blockIdx.x * L;
-    for (int l = 0; l < L; l++) {
-        const int r = r0 + l;
-        float2 *x = X + l * S;
-        if (MODE == PY_EMBED) {
-            for (int e = tid; e < n; e += MX_PY_T) x[lf_pos(e)] = make_float2(0.f, 0.f);
-        } else if (r >= a.nrows) {
-            for (int e = tid; e < n; e += MX_PY_T) x[lf_pos(e)] = make_float2(0.f, 0.f);
-        } else if (MODE == PY_REAL) {
-            const float *src = a.inr + (long)r * n;
-            for (int e = tid; e < n; e += MX_PY_T) x[lf_pos(e)] = make_float2(src[e], 0.f);
-        } else if (MODE == PY_MOD) {
-            // row ux of the window: PSF row ux + ox (x), columns uy + oy (y)
-            const int sx = r + a.ox;
-            const bool rin = sx >= 0 && sx < n;
-            const float2 *src = a.in + (long)(rin ? sx : 0) * n;
-            const float2 *m = a.mask + (long)r * n;
-            for (int e = tid; e < n; e += MX_PY_T) {
-                const int sy = e + a.oy;
-                x[lf_pos(e)] = rin && sy >= 0 && sy < n ? cmul(src[sy], m[e]) : make_float2(0.f, 0.f);
-            }
-        } else {
-            const float2 *src = a.in + (long)r * n;
-            for (int e = tid; e < n; e += MX_PY_T) x[lf_pos(e)] = src[e];
-        }
-    }
-    if (MODE == PY_EMBED) {
+__global__ __launch_bounds__(1024) void k_py_rows(PyArgs a) {
+    const int n = a.n, L = a.L, S = a.plan.S, tid = threadIdx.x;
+    const LxLines ln{L, a.lgL};
+    const LxPlan plan = LX_PLAN(PyArgs, plan);
+    const int u = xcd_unit((int)blockIdx.x, (int)gridDim.x);
+    if constexpr (MODE == PY_EMBED) {
+        const int r0 = u * L;
+        for (int i = tid; i < L * S; i += blockDim.x) pyl[i] = make_float2(0.f, 0.f);
         __syncthreads(); // the zeroed lines before the scatter
-        for (int l = 0; l < L; l++) {
-            const int r = r0 + l;
-            if (r >= a.nrows) continue;
-            float2 *x = X + l * S;
-            for (int k = a.rowp[r] + tid; k < a.rowp[r + 1]; k += MX_PY_T) {
+        for (int l = 0; l < L && r0 + l < a.nlines; l++)
+            for (int k = a.rowp[r0 + l] + tid; k < a.rowp[r0 + l + 1]; k += blockDim.x) {
                 const int2 en = a.ent[k];
-                float re, im;
-                cis_rev(a.opd[en.y] * a.inv_wvl, a.amp[en.y], re, im);
-                x[lf_pos(en.x)] = make_float2(re, im);
+                // the phase in revolutions, reduced in FP64
+                double rev = (double)a.opd[en.y] * a.inv_wvl;
+                rev -= rint(rev);
+                float sn, cs;
+                sincospif(2.f * (float)rev, &sn, &cs);
+                const float A = a.amp[en.y];
+                pyl[l * S + en.x] = make_float2(A * cs, A * sn);
             }
-        }
-    }
-    __syncthreads();
-    constexpr bool INV = MODE == PY_MOD || MODE == PY_ACC || MODE == PY_IMG;
-    float2 *res = lds_fft_rt<INV, MX_PY_T>(X, Y, a.plan, L, S);
-    if (MODE == PY_DTF) {
-        // along ky: times the transfer function, then back to y
-        for (int l = 0; l < L; l++) {
-            const int r = r0 + l;
-            if (r >= a.nrows) continue;
-            float2 *x = res + l * S;
-            const float *t = a.nomt + (long)r * n;
-            for (int e = tid; e < n; e += MX_PY_T) {
-                const float2 v = x[lf_pos(e)];
-                x[lf_pos(e)] = make_float2(v.x * t[e], v.y * t[e]);
-            }
-        }
         __syncthreads();
-        res = lds_fft_rt<true, MX_PY_T>(res, res == X ? Y : X, a.plan, L, S);
+        float2 *out = a.out + (long)r0 * n;
+        const int nl = a.nlines - r0;
+        lx_fft<false, LX_ROW, LX_ROW, true>(
+            pyl, plan, ln, [&](int l, int j, int off) LX_INLINE { return pyl[__mul24(l, S) + j + off]; },
+            [&](int l, int d, int off, float2 v, int) LX_INLINE {
+                if (l < nl) lx_at(out + off, __mul24(l, n) + d) = v;
+            });
+    } else if constexpr (MODE == PY_MOD) {
+        // row ux of the window: PSF row ux + ox (x), columns uy + oy (y); the
+        // positions of one row group are neighbours, since they share the mask
+        const int pos = u % a.npos, r0 = u / a.npos * L, ox = a.ox[pos], oy = a.oy[pos];
+        const float2 *in = a.in, *mask = a.mask + (long)r0 * n;
+        float2 *out = a.out + (long)pos * n * n + (long)r0 * n;
+        const int nl = a.nlines - r0;
+        lx_fft<true, LX_ROW, LX_ROW, false>(
+            pyl, plan, ln,
+            [&](int l, int j, int off) LX_INLINE {
+                const int sx = r0 + l + ox, sy = j + off + oy;
+                const bool ok = l < nl && sx >= 0 && sx < n && sy >= 0 && sy < n;
+                const float2 p = lx_at(in, ok ? __mul24(sx, n) + sy : 0), m = lx_at(mask, ok ? __mul24(l, n) + j + off : 0);
+                return lx_sel(ok, cmul(p, m));
+            },
+            [&](int l, int d, int off, float2 v, int) LX_INLINE {
+                if (l < nl) lx_at(out + off, __mul24(l, n) + d) = v;
+            });
+    } else { // PY_REAL, PY_IMG
+        const int r0 = u * L, nl = a.nlines - r0;
+        const float2 *in = MODE == PY_IMG ? a.in + (long)r0 * n : nullptr;
+        const float *inr = MODE == PY_REAL ? a.inr + (long)r0 * n : nullptr;
+        const int nsplit = a.nsplit;
+        const long nn = (long)n * n;
+        lx_fft<MODE == PY_IMG, LX_ROW, LX_ROW, false>(
+            pyl, plan, ln,
+            [&](int l, int j, int off) LX_INLINE {
+                const bool ok = l < nl;
+                const int i = ok ? __mul24(l, n) + j + off : 0;
+                if constexpr (MODE == PY_IMG) return lx_sel(ok, lx_at(in, i));
+                float v = 0.f;
+#pragma unroll
+                for (int q = 0; q < MX_PY_MAXSPLIT; q++) { // (loads of all at once, past the last split the first again)
+                    const float t = lx_at(inr + (q < nsplit ? q * nn : 0), i);
+                    v += q < nsplit ? t : 0.f;
+                }
+                return make_float2(ok ? v : 0.f, 0.f);
+            },
+            [&](int l, int d, int off, float2 v, int) LX_INLINE {
+                if (l >= nl) return;
+                const int i = __mul24(l, n) + d;
+                if constexpr (MODE == PY_IMG) lx_at(a.outr + (long)r0 * n + off, i) = v.x;
+                else lx_at(a.out + (long)r0 * n + off, i) = v;
+            });
     }
+}
+
+// columns c0 .. c0 + L - 1
+template <int MODE>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(5))) void k_py_cols(PyArgs a) {
+    const int n = a.n, L = a.L, S = a.plan.S;
+    const LxLines ln{L, a.lgL};
+    const LxPlan plan = LX_PLAN(PyArgs, plan);
+    const int u = xcd_unit((int)blockIdx.x, (int)gridDim.x);
     const int n2 = n / 2;
-    for (int l = 0; l < L; l++) {
-        const int r = r0 + l;
-        if (r >= a.nrows) continue;
-        const float2 *x = res + l * S;
-        if (MODE == PY_PSF) {
-            // centred (cfftshift) and scaled: row x -> (x + n/2) % n, ky -> (ky + n/2) % n
-            float2 *dst = a.out + (long)((r + n2) % n) * n;
-            for (int e = tid; e < n; e += MX_PY_T) {
-                const float2 v = x[lf_pos(e)];
-                dst[(e + n2) % n] = make_float2(v.x * a.scale, v.y * a.scale);
-            }
-        } else if (MODE == PY_ACC) {
-            float *dst = a.outr + (long)r * n;
-            for (int e = tid; e < n; e += MX_PY_T) {
-                const float2 v = x[lf_pos(e)];
-                dst[e] += a.scale * (v.x * v.x + v.y * v.y);
-            }
-        } else if (MODE == PY_IMG) {
-            float *dst = a.outr + (long)r * n;
-            for (int e = tid; e < n; e += MX_PY_T) dst[e] = x[lf_pos(e)].x;
-        } else {
-            float2 *dst = a.out + (long)r * n;
-            for (int e = tid; e < n; e += MX_PY_T) dst[e] = x[lf_pos(e)];
+    if constexpr (MODE == PY_PSF) {
+        // centred (cfftshift) and scaled: column kx -> row (kx + n/2) % n of
+        // the transposed PSF, ky -> (ky + n/2) % n
+        const int c0 = u * L, nl = n - c0, y0 = a.y0, y1 = a.y1;
+        const float2 *in = a.in + c0;
+        float2 *out = a.out;
+        const float sc = a.scale;
+        lx_fft<false, LX_COL, LX_ROW, false>(
+            pyl, plan, ln,
+            [&](int l, int j, int off) LX_INLINE {
+                const int e = j + off;
+                const bool ok = l < nl && e >= y0 && e < y1;
+                return lx_sel(ok, lx_at(in, ok ? __mul24(e, n) + l : 0));
+            },
+            [&](int l, int d, int off, float2 v, int) LX_INLINE {
+                if (l >= nl) return;
+                const int x = c0 + l, ky = d + off;
+                lx_at(out, __mul24(x < n2 ? x + n2 : x - n2, n) + (ky < n2 ? ky + n2 : ky - n2)) =
+                    make_float2(v.x * sc, v.y * sc);
+            });
+    } else if constexpr (MODE == PY_ACC) {
+        // |.|^2 of this split's positions, in registers (slot: the thread's
+        // point of the last stage, the same one for every position)
+        const int split = u % a.nsplit, c0 = u / a.nsplit * L, nl = n - c0;
+        const long nn = (long)n * n;
+        float acc[LX_E];
+#pragma unroll
+        for (int k = 0; k < LX_E; k++) acc[k] = 0.f;
+        for (int pos = split; pos < a.npos; pos += a.nsplit) {
+            const float2 *in = a.in + pos * nn + c0;
+            const float wt = a.wt[pos];
+            __syncthreads(); // the previous position's last reads of the lines
+            lx_fft<true, LX_COL, LX_ROW, false>(
+                pyl, plan, ln,
+                [&](int l, int j, int off) LX_INLINE {
+                    const bool ok = l < nl;
+                    return lx_sel(ok, lx_at(in, ok ? __mul24(j + off, n) + l : 0));
+                },
+                [&](int, int, int, float2 v, int slot) LX_INLINE { acc[slot] += wt * (v.x * v.x + v.y * v.y); });
         }
+        float *out = a.outr + split * nn + (long)c0 * n;
+        const bool first = a.first != 0;
+        lx_outputs<LX_ROW>(plan, ln, [&](int l, int d, int off, int slot) LX_INLINE {
+            if (l >= nl) return;
+            float &o = lx_at(out + off, __mul24(l, n) + d);
+            o = first ? acc[slot] : o + acc[slot];
+        });
+    } else { // PY_DTF: along ky, times the transfer function, then back to y
+        const int c0 = u * L, nl = n - c0;
+        const float2 *in = a.in + c0;
+        const float *nm = a.nomt + (long)c0 * n;
+        float2 *out = a.out + c0;
+        lx_fft<false, LX_COL, LX_ROW, false>(
+            pyl, plan, ln,
+            [&](int l, int j, int off) LX_INLINE {
+                const bool ok = l < nl;
+                return lx_sel(ok, lx_at(in, ok ? __mul24(j + off, n) + l : 0));
+            },
+            [&](int l, int d, int off, float2 v, int) LX_INLINE {
+                const float f = lx_at(nm + off, l < nl ? __mul24(l, n) + d : 0);
+                pyl[__mul24(l, S) + d + off] = make_float2(v.x * f, v.y * f);
+            });
+        __syncthreads();
+        lx_fft<true, LX_ROW, LX_COL, true>(
+            pyl, plan, ln, [&](int l, int j, int off) LX_INLINE { return pyl[__mul24(l, S) + j + off]; },
+            [&](int l, int d, int off, float2 v, int) LX_INLINE {
+                if (l < nl) lx_at(out + (long)off * n, __mul24(d, n) + l) = v;
+            });
     }
-}
-
-// out[c][r] = in[r][c] for an n x n array in 32 x 32 tiles; rows of in
-// outside [y0, y1) are read as zero (the field rows without points).
-struct PyTrArgs {
-    const float2 *in;
-    float2 *out;
-    int n, y0, y1;
-};
-__global__ __launch_bounds__(256) void k_py_transpose(PyTrArgs a) {
-    __shared__ float2 t[32][33];
-    const int bx = (int)blockIdx.x * 32, by = (int)blockIdx.y * 32;
-    const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
-    for (int j = ty; j < 32; j += 8) {
-        const int r = by + j, c = bx + tx;
-        t[j][tx] = r < a.n && c < a.n && r >= a.y0 && r < a.y1 ? a.in[(long)r * a.n + c] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();
-    for (int j = ty; j < 32; j += 8) {
-        const int r = bx + j, c = by + tx;
-        if (r < a.n && c < a.n) a.out[(long)r * a.n + c] = t[tx][j];
-    }
-}
-
-__global__ __launch_bounds__(256) void k_py_zero(float *p, long n) {
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) p[i] = 0.f;
 }
 
 // ints[side][isa] = alpha * (bilinear sample of the image at the
@@ -286,7 +225,7 @@ struct PySampleArgs {
     const double *sax, *say;        // subaperture centres (m)
     double inv_dx;                  // 1 / pupil-image sampling
     double offx[MX_PY_MAXSIDE], offy[MX_PY_MAXSIDE]; // image centre of each side (samples), minus 1/2
-    float alpha;
+    double alpha;
     float *ints;
 };
 __global__ __launch_bounds__(256) void k_py_sample(PySampleArgs a) {
@@ -295,22 +234,21 @@ __global__ __launch_bounds__(256) void k_py_sample(PySampleArgs a) {
     const int side = i / a.nsa, isa = i - side * a.nsa;
     const double fx = a.sax[isa] * a.inv_dx + a.offx[side], fy = a.say[isa] * a.inv_dx + a.offy[side];
     const double ix = floor(fx), iy = floor(fy);
-    const float wx1 = (float)(fx - ix), wy1 = (float)(fy - iy);
-    const float wx[2] = {1.f - wx1, wx1}, wy[2] = {1.f - wy1, wy1};
-    float s = 0.f;
+    const double wx[2] = {1. - (fx - ix), fx - ix}, wy[2] = {1. - (fy - iy), fy - iy};
+    double s = 0;
     for (int q = 0; q < 4; q++) {
         const long x = (long)ix + (q & 1), y = (long)iy + (q >> 1);
-        const float w = wx[q & 1] * wy[q >> 1];
-        if (w > 1e-15f && x >= 0 && x < a.n && y >= 0 && y < a.n) s += w * a.img[y * a.n + x];
+        const double w = wx[q & 1] * wy[q >> 1];
+        if (w > 1e-15 && x >= 0 && x < a.n && y >= 0 && y < a.n) s += w * a.img[y * a.n + x];
     }
-    a.ints[i] = a.alpha * s;
+    a.ints[i] = (float)(a.alpha * s);
 }
 
 // gradients (pywfs_grad, lib/pywfs.c:457-522), one block
 struct PyGradArgs {
     const float *ints;
     int nsa, nside, sigmatch, raw;
-    float gain, siglev;
+    double gain, siglev;
     const float *saa, *gradoff; // gradoff may be null
     float *grad;
 };
@@ -326,30 +264,30 @@ __global__ __launch_bounds__(256) void k_py_grad(PyGradArgs a) {
         if (tid < k) red[tid] += red[tid + k];
         __syncthreads();
     }
-    const float imean = (float)(red[0] / nsa);
+    const double imean = red[0] / nsa;
     const bool raw = a.raw || a.nside < 3;
     const int ng = raw ? a.nside : 2;
     for (int isa = tid; isa < nsa; isa += 256) {
         const float *I = a.ints + isa;
-        float g[MX_PY_MAXSIDE] = {};
+        double g[MX_PY_MAXSIDE] = {};
         if (raw) {
-            for (int sd = 0; sd < a.nside; sd++) g[sd] = I[sd * nsa] * (a.gain / a.siglev);
+            for (int sd = 0; sd < a.nside; sd++) g[sd] = (double)I[sd * nsa] * (a.gain / a.siglev);
         } else {
-            float isum = 0.f;
+            double isum = 0;
             if (a.sigmatch == 0) isum = a.siglev * a.saa[isa];
             else if (a.sigmatch == 1)
                 for (int sd = 0; sd < a.nside; sd++) isum += I[sd * nsa];
             else isum = imean * a.saa[isa];
-            const float al = a.gain / isum;
+            const double al = a.gain / isum;
             if (a.nside == 3) {
-                g[0] = (I[nsa] - I[2 * nsa]) * al * 0.86602540378443865f;
-                g[1] = (I[0] - 0.5f * (I[nsa] + I[2 * nsa])) * al;
+                g[0] = ((double)I[nsa] - I[2 * nsa]) * al * 0.86602540378443865;
+                g[1] = ((double)I[0] - 0.5 * ((double)I[nsa] + I[2 * nsa])) * al;
             } else {
-                g[0] = (I[0] - I[nsa] + I[2 * nsa] - I[3 * nsa]) * al;
-                g[1] = (I[0] + I[nsa] - I[2 * nsa] - I[3 * nsa]) * al;
+                g[0] = ((double)I[0] - I[nsa] + I[2 * nsa] - I[3 * nsa]) * al;
+                g[1] = ((double)I[0] + I[nsa] - I[2 * nsa] - I[3 * nsa]) * al;
             }
         }
-        for (int k = 0; k < ng; k++) a.grad[isa + k * nsa] = g[k] - (a.gradoff ? a.gradoff[isa + k * nsa] : 0.f);
+        for (int k = 0; k < ng; k++) a.grad[isa + k * nsa] = (float)(g[k] - (a.gradoff ? a.gradoff[isa + k * nsa] : 0.f));
     }
 }
 
@@ -366,7 +304,8 @@ struct mx_pywfs_s {
     double sioff[2 * MX_PY_MAXSIDE] = {};
     int ylo = 0, nband = 0;  // grid rows holding points
     int ireal = 0;
-    LfPlan plan{};
+    LinePlan plan{};
+    int nbatch = 1, nsplit = 1; // scratch planes, partial pupil intensities
     float2 *d_tw = nullptr;
     int *d_rowp = nullptr;
     int2 *d_ent = nullptr;
@@ -374,8 +313,8 @@ struct mx_pywfs_s {
     float *d_amp = nullptr, *d_opd = nullptr, *d_saa = nullptr, *d_gradoff = nullptr;
     float2 *d_mask = nullptr;   // [nwvl][n][n] transposed
     float *d_nomt = nullptr;    // [n][n] transposed
-    float2 *d_A = nullptr, *d_B = nullptr, *d_P = nullptr; // work, work, centred PSF [nwvl] (transposed)
-    float *d_pup = nullptr, *d_img = nullptr;
+    float2 *d_A = nullptr, *d_B = nullptr, *d_P = nullptr; // work, scratch [nbatch], centred PSF [nwvl] (transposed)
+    float *d_pup = nullptr, *d_img = nullptr; // pupil intensity [nsplit], image
     float *d_ints = nullptr, *d_grad = nullptr;
     bool have_gradoff = false;
     bool timing = false;
@@ -401,43 +340,43 @@ void pywfs_release(mx_pywfs_t *h) {
     delete h;
 }
 
-// Stockham plan of a pyramid grid side n <= MX_PY_MAXN with factors 2, 3, 5, 7
-bool py_plan(long n, LfPlan &P) {
-    P = LfPlan{};
-    if (n < 2 || n > MX_PY_MAXN) return false;
-    P.n = (int)n;
-    long prod = 1;
-    while (P.nrad < MX_LF_MAXRAD && lf_radix((int)n, P.nrad)) {
-        P.rad[P.nrad] = lf_radix((int)n, P.nrad);
-        prod *= P.rad[P.nrad++];
-    }
-    return prod == n;
+// Lines per block: as many as 4096 points hold (a power of two, at most 16), so
+// that a block has about 256 threads and a CU several blocks; columns at least
+// two, since a run of L columns is what the pass reads of a row.  (784^2: 4
+// columns 305 us a step, 8 336, 16 377; 2916^2: 2 columns 4293, 1 4344, 4
+// 4299.)
+int py_row_lines(long n) {
+    int L = 16;
+    while (L > 1 && L * n > 4096) L /= 2;
+    return L;
+}
+int py_col_lines(long n) {
+    int L = 16;
+    while (L > 2 && L * n > 4096) L /= 2;
+    return L;
 }
 
-int py_rows(mx_pywfs_t *h, int mode, PyRowArgs a, int nrows) {
+int py_pass(mx_pywfs_t *h, int mode, PyArgs a, int nlines) {
+    const bool cols = mode == PY_PSF || mode == PY_ACC || mode == PY_DTF;
     a.plan = h->plan;
     a.plan.tw = h->d_tw;
     a.n = (int)h->n;
-    a.S = lf_stride(a.n);
-    a.L = pyl_lines(a.n);
-    a.nrows = nrows;
-    const dim3 grid((unsigned)((nrows + a.L - 1) / a.L)), block(MX_PY_T);
-    const size_t lds = sizeof(float2) * 2 * (size_t)a.L * a.S; // two line buffers, <= 2 MX_LF_LDS complex
+    a.L = cols ? py_col_lines(h->n) : py_row_lines(h->n);
+    a.lgL = ilog2c(a.L);
+    a.nlines = nlines;
+    const int many = mode == PY_MOD ? a.npos : mode == PY_ACC ? a.nsplit : 1;
+    const dim3 grid((unsigned)((nlines + a.L - 1) / a.L * many)), block((unsigned)lx_threads(a.plan, a.L));
+    const size_t lds = sizeof(float2) * (size_t)a.L * a.plan.S;
     switch (mode) {
     case PY_EMBED: k_py_rows<PY_EMBED><<<grid, block, lds, h->stream>>>(a); break;
-    case PY_PSF: k_py_rows<PY_PSF><<<grid, block, lds, h->stream>>>(a); break;
+    case PY_PSF: k_py_cols<PY_PSF><<<grid, block, lds, h->stream>>>(a); break;
     case PY_MOD: k_py_rows<PY_MOD><<<grid, block, lds, h->stream>>>(a); break;
-    case PY_ACC: k_py_rows<PY_ACC><<<grid, block, lds, h->stream>>>(a); break;
+    case PY_ACC: k_py_cols<PY_ACC><<<grid, block, lds, h->stream>>>(a); break;
     case PY_REAL: k_py_rows<PY_REAL><<<grid, block, lds, h->stream>>>(a); break;
-    case PY_DTF: k_py_rows<PY_DTF><<<grid, block, lds, h->stream>>>(a); break;
+    case PY_DTF: k_py_cols<PY_DTF><<<grid, block, lds, h->stream>>>(a); break;
     default: k_py_rows<PY_IMG><<<grid, block, lds, h->stream>>>(a); break;
     }
     return MX_OK;
-}
-
-void py_transpose(mx_pywfs_t *h, const float2 *in, float2 *out, int y0, int y1) {
-    const unsigned nt = (unsigned)((h->n + 31) / 32);
-    k_py_transpose<<<dim3(nt, nt), dim3(256), 0, h->stream>>>(PyTrArgs{in, out, (int)h->n, y0, y1});
 }
 
 // pywfs_ints and pywfs_grad on the OPD in d_opd (queued on the stream)
@@ -445,65 +384,83 @@ int py_image(mx_pywfs_t *h, double siglev) {
     const long n = h->n, nn = n * n;
     const int n2 = (int)(n / 2);
     if (h->timing) HIPCHK(hipEventRecord(h->ev[0], h->stream));
-    k_py_zero<<<dim3(1024), dim3(256), 0, h->stream>>>(h->d_pup, nn);
+    // The PSF's normalisation is applied as the power of two next to it and
+    // the weights relative to the first one's, both exact (the latter for one
+    // ring and wavelength); the rest goes into the samples' FP64 factor, so
+    // that no rounding of a factor scales every intensity alike.
+    const double psfnorm = 1. / (std::sqrt(h->ampnorm) * (double)n), psf2 = std::exp2(std::rint(std::log2(psfnorm)));
+    bool first = true;
+    double wt0 = 0;
     for (int iw = 0; iw < h->nwvl; iw++) {
         float2 *P = h->d_P + (size_t)iw * nn;
-        // field rows (band only) -> A; transpose -> B [x][y]; FFT along y,
-        // centred and scaled -> P [x][y]
-        PyRowArgs e{};
+        // field rows (band only) along x -> A [y][kx]; columns along y,
+        // centred and scaled -> P [kx][ky]
+        PyArgs e{};
         e.rowp = h->d_rowp;
         e.ent = h->d_ent;
         e.opd = h->d_opd;
         e.amp = h->d_amp;
-        e.inv_wvl = (float)(1. / h->wvl[iw]);
+        e.inv_wvl = 1. / h->wvl[iw];
         e.out = h->d_A + (size_t)h->ylo * n;
-        py_rows(h, PY_EMBED, e, h->nband);
-        py_transpose(h, h->d_A, h->d_B, h->ylo, h->ylo + h->nband);
-        PyRowArgs f{};
-        f.in = h->d_B;
+        py_pass(h, PY_EMBED, e, h->nband);
+        PyArgs f{};
+        f.in = h->d_A;
         f.out = P;
-        f.scale = (float)(1. / (std::sqrt(h->ampnorm) * (double)n));
-        py_rows(h, PY_PSF, f, (int)n);
-        // modulation positions (lib/pywfs.c:390-430)
+        f.y0 = h->ylo;
+        f.y1 = h->ylo + h->nband;
+        f.scale = (float)psf2;
+        py_pass(h, PY_PSF, f, (int)n);
+        // modulation positions (lib/pywfs.c:390-430), in batches: rows ux of
+        // the window along uy -> scratch [position][ux][y]; columns along ux,
+        // |.|^2 -> pup [split][y][x]
         const double dtheta = h->wvl[iw] / (h->dx * (double)n);
+        PyArgs m{};
+        m.in = P;
+        m.mask = h->d_mask + (size_t)iw * nn;
+        m.out = h->d_B;
+        m.nsplit = h->nsplit;
+        auto flush = [&]() {
+            if (!m.npos) return;
+            py_pass(h, PY_MOD, m, (int)n);
+            PyArgs c = m;
+            c.in = h->d_B;
+            c.outr = h->d_pup;
+            c.first = first;
+            py_pass(h, PY_ACC, c, (int)n);
+            first = false;
+            m.npos = 0;
+        };
         for (int ir = 0; ir < h->modulring; ir++) {
             const double ri = h->modulate * (ir + 1) / h->modulring;
             const int npos = h->modulpos * (ir + 1) / h->modulring;
             for (int ip = 0; ip < npos; ip++) {
                 const double th = 2. * M_PI * ((double)ip / npos);
-                PyRowArgs m{};
-                m.in = P;
-                m.mask = h->d_mask + (size_t)iw * nn;
-                m.ox = (int)std::lround(std::cos(th) * ri / dtheta);
-                m.oy = (int)std::lround(std::sin(th) * ri / dtheta);
-                m.out = h->d_B;
-                py_rows(h, PY_MOD, m, (int)n);
-                py_transpose(h, h->d_B, h->d_A, 0, (int)n);
-                PyRowArgs c{};
-                c.in = h->d_A;
-                c.outr = h->d_pup;
-                c.scale = (float)(h->wvlwts[iw] / ((double)nn * npos * h->modulring));
-                py_rows(h, PY_ACC, c, (int)n);
+                m.ox[m.npos] = (int)std::lround(std::cos(th) * ri / dtheta);
+                m.oy[m.npos] = (int)std::lround(std::sin(th) * ri / dtheta);
+                const double wt = h->wvlwts[iw] / ((double)nn * npos * h->modulring);
+                if (wt0 == 0) wt0 = wt;
+                m.wt[m.npos] = wt0 != 0 ? (float)(wt / wt0) : 0.f;
+                if (++m.npos == h->nbatch) flush();
             }
         }
+        flush();
     }
-    // detector transfer function: rows of the pupil intensity, transpose,
-    // FFT x DTF x inverse FFT along y, transpose, inverse FFT along x
-    PyRowArgs r1{};
+    // detector transfer function: rows of the pupil intensity along x, columns
+    // along y x DTF and back, rows back
+    PyArgs r1{};
     r1.inr = h->d_pup;
+    r1.nsplit = h->nsplit;
     r1.out = h->d_A;
-    py_rows(h, PY_REAL, r1, (int)n);
-    py_transpose(h, h->d_A, h->d_B, 0, (int)n);
-    PyRowArgs r2{};
-    r2.in = h->d_B;
+    py_pass(h, PY_REAL, r1, (int)n);
+    PyArgs r2{};
+    r2.in = h->d_A;
     r2.nomt = h->d_nomt;
-    r2.out = h->d_A;
-    py_rows(h, PY_DTF, r2, (int)n);
-    py_transpose(h, h->d_A, h->d_B, 0, (int)n);
-    PyRowArgs r3{};
+    r2.out = h->d_B;
+    py_pass(h, PY_DTF, r2, (int)n);
+    PyArgs r3{};
     r3.in = h->d_B;
     r3.outr = h->d_img;
-    py_rows(h, PY_IMG, r3, (int)n);
+    py_pass(h, PY_IMG, r3, (int)n);
     // samples and gradients
     PySampleArgs s{};
     s.img = h->d_img;
@@ -517,10 +474,10 @@ int py_image(mx_pywfs_t *h, double siglev) {
         s.offx[k] = h->sioff[2 * k] * n2 + n2 - 0.5;
         s.offy[k] = h->sioff[2 * k + 1] * n2 + n2 - 0.5;
     }
-    s.alpha = (float)((double)h->nsa * siglev / (double)nn);
+    s.alpha = (double)h->nsa * siglev / (double)nn * wt0 * (psfnorm / psf2) * (psfnorm / psf2);
     s.ints = h->d_ints;
     k_py_sample<<<dim3((unsigned)((h->nsa * h->nside + 255) / 256)), dim3(256), 0, h->stream>>>(s);
-    PyGradArgs g{h->d_ints, (int)h->nsa, h->nside, h->sigmatch, h->raw, (float)h->gain, (float)h->siglev,
+    PyGradArgs g{h->d_ints, (int)h->nsa, h->nside, h->sigmatch, h->raw, h->gain, h->siglev,
                  h->d_saa, h->have_gradoff ? h->d_gradoff : nullptr, h->d_grad};
     k_py_grad<<<dim3(1), dim3(256), 0, h->stream>>>(g);
     HIPCHK(hipGetLastError());
@@ -555,8 +512,8 @@ int mx_pywfs_init(mx_pywfs_t **out, const mx_pywfs_cfg_t *c) {
         return set_err(MX_EINVAL, "mx_pywfs_init: nside=%d (2, 3 or 4 pupil images)", c->nside);
     if (n % 2)
         return set_err(MX_EINVAL, "mx_pywfs_init: the FFT grid side %ld must be even", n);
-    LfPlan plan;
-    if (!py_plan(n, plan))
+    LinePlan plan;
+    if (n > MX_PY_MAXN || !lx_plan(n, plan))
         return set_err(MX_EINVAL, "mx_pywfs_init: FFT grid side %ld is not a product of 2, 3, 5 and 7 up to %d", n,
                        MX_PY_MAXN);
     if (c->nsa < 1 || !c->salocx || !c->salocy || !c->sioff || !c->mask || !c->nominal)
@@ -598,14 +555,14 @@ int mx_pywfs_init(mx_pywfs_t **out, const mx_pywfs_cfg_t *c) {
     h->plan = plan;
     PYCHK(hipSetDevice(h->device));
     {
-        // the row passes' two line buffers may exceed the default dynamic LDS limit
-        const int lds = (int)(sizeof(float2) * 2 * MX_LF_LDS);
+        // the lines of a block may exceed the default dynamic LDS limit
+        const int lds = (int)(sizeof(float2) * plan.S * (size_t)std::max(py_row_lines(n), py_col_lines(n)));
         const void *k[] = {reinterpret_cast<const void *>(&k_py_rows<PY_EMBED>),
-                           reinterpret_cast<const void *>(&k_py_rows<PY_PSF>),
+                           reinterpret_cast<const void *>(&k_py_cols<PY_PSF>),
                            reinterpret_cast<const void *>(&k_py_rows<PY_MOD>),
-                           reinterpret_cast<const void *>(&k_py_rows<PY_ACC>),
+                           reinterpret_cast<const void *>(&k_py_cols<PY_ACC>),
                            reinterpret_cast<const void *>(&k_py_rows<PY_REAL>),
-                           reinterpret_cast<const void *>(&k_py_rows<PY_DTF>),
+                           reinterpret_cast<const void *>(&k_py_cols<PY_DTF>),
                            reinterpret_cast<const void *>(&k_py_rows<PY_IMG>)};
         for (const void *f : k) PYCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     }
@@ -642,7 +599,7 @@ int mx_pywfs_init(mx_pywfs_t **out, const mx_pywfs_cfg_t *c) {
         rowp[r + 1] = (int)ent.size();
     }
     std::vector<float2> tw;
-    lf_twiddles(h->plan, tw);
+    lx_twiddles(n, tw);
     std::vector<float> amp(c->nloc);
     for (long i = 0; i < c->nloc; i++) amp[i] = (float)c->amp[i];
     std::vector<float2> mt((size_t)c->nwvl * nn);
@@ -677,9 +634,21 @@ int mx_pywfs_init(mx_pywfs_t **out, const mx_pywfs_cfg_t *c) {
     PYCHK(up(&h->d_gradoff, (const float *)nullptr, (size_t)h->ng * c->nsa));
     PYCHK(up(&h->d_opd, (const float *)nullptr, (size_t)c->nloc));
     PYCHK(up(&h->d_A, (const float2 *)nullptr, (size_t)nn));
-    PYCHK(up(&h->d_B, (const float2 *)nullptr, (size_t)nn));
+    {
+        // positions per batch, evened out; splits of a batch's positions so
+        // that the column pass has four blocks for each CU
+        int npos = 0;
+        for (int ir = 0; ir < h->modulring; ir++) npos += h->modulpos * (ir + 1) / h->modulring;
+        npos = std::max(npos, 1);
+        const int most = (int)std::max(1L, std::min({MX_PY_SCRATCH / (8 * nn), (long)MX_PY_MAXB, (long)npos}));
+        const int nlaunch = (npos + most - 1) / most;
+        h->nbatch = (npos + nlaunch - 1) / nlaunch;
+        const int groups = (int)((n + py_col_lines(n) - 1) / py_col_lines(n));
+        h->nsplit = std::max(1, std::min({h->nbatch, MX_PY_MAXSPLIT, (1024 + groups - 1) / groups}));
+    }
+    PYCHK(up(&h->d_B, (const float2 *)nullptr, (size_t)nn * h->nbatch));
     PYCHK(up(&h->d_P, (const float2 *)nullptr, (size_t)nn * c->nwvl));
-    PYCHK(up(&h->d_pup, (const float *)nullptr, (size_t)nn));
+    PYCHK(up(&h->d_pup, (const float *)nullptr, (size_t)nn * h->nsplit));
     PYCHK(up(&h->d_img, (const float *)nullptr, (size_t)nn));
     PYCHK(up(&h->d_ints, (const float *)nullptr, (size_t)c->nsa * c->nside));
     PYCHK(up(&h->d_grad, (const float *)nullptr, (size_t)h->ng * c->nsa));

@@ -2584,29 +2584,32 @@ __global__ __launch_bounds__(MX_LF_THREADS) void k_lf_sample(LfSampleArgs a) {
     // most of the gradient error of a 16 x 16 pixel detector
     double s0 = 0., s1 = 0., s2 = 0.;
     for (int p = threadIdx.x; p < a.npix; p += blockDim.x) {
-        float pv = 0.f;
+        double px = 0.; // the pixel before it is rounded to FP32
         for (int iwvl = 0; iwvl < a.nwvl; iwvl++) {
             const float *im = a.img + (((long)isa * a.nwfs + iwfs) * a.nwvl + iwvl) * a.imgstride; // (lf_chain)
             const LfWvl &SW = a.wv[iwvl];
             const int4 id = SW.si_c[isa * SW.si_sa + p];
             const float4 w = SW.si_w[isa * SW.si_sa + p];
-            pv += W.alpha[iwvl] * (w.x * im[id.x] + w.y * im[id.y] + w.z * im[id.z] + w.w * im[id.w]);
+            px += (double)W.alpha[iwvl] *
+                  ((double)w.x * im[id.x] + (double)w.y * im[id.y] + (double)w.z * im[id.z] + (double)w.w * im[id.w]);
         }
+        float pv = (float)px;
         if (!dt_frame(a.dt, ibase + p, pv)) continue; // uniform: not the exposure's last frame
         if (a.noise.on) pv = add_noise(a.noise, pv, p, iwfs, a.nsa, isa);
         a.ints[ibase + p] = pv;
+        if (a.noise.on || a.dt.phase != (MX_DT_FIRST | MX_DT_OUT)) px = pv;
         if (a.i0acc) a.i0acc[ibase + p] += (double)pv;
         dither_add(a.dith, iwfs, ibase + p, pv);
         if (a.phytype == MX_PTYPE_MF) {
             const float *mt = a.mtche + ibase * 2 + 2 * p;
-            s0 += (double)mt[0] * pv;
-            s1 += (double)mt[1] * pv;
-            s2 += pv;
+            s0 += mt[0] * px;
+            s1 += mt[1] * px;
+            s2 += px;
         } else {
-            const float iI = pv - a.cogoff;
+            const double iI = px - a.cogoff;
             if (iI > a.cogthres) {
-                s0 += (double)iI * (p % a.pixpsax);
-                s1 += (double)iI * (p / a.pixpsax);
+                s0 += iI * (p % a.pixpsax);
+                s1 += iI * (p / a.pixpsax);
                 s2 += iI;
             }
         }
@@ -3252,6 +3255,13 @@ int mx_wfsgrad_init_batch(mx_wfsgrad_t **out, const mx_powfs_t *p, const mx_wfs_
     h->lf = lf;
     std::vector<float2> lf_tw;
     if (lf) {
+        // blocks of 512 threads (an autotune candidate) may exceed the default
+        // dynamic LDS limit
+        for (int q : {0, 1, 2, 4})
+            if (hipFuncSetAttribute(lf_kernel(q), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess) {
+                mx_wfsgrad_free(h);
+                return set_err(MX_EHIP, "the large-field kernels' LDS size could not be set");
+            }
         lx_plan(h->nwvf, h->lf_pn);
         lx_plan(N, h->lf_pm);
         lx_twiddles(h->nwvf, lf_tw);
