@@ -2769,6 +2769,18 @@ struct StepPlan {
     bool llt = false;
 };
 
+// A window of consecutive WFS's results in pinned memory, as step gen left
+// them.  A program reads every WFS after a step, and a blocking copy each (to
+// pageable memory, 12 to 15 us) cost more than a small step; one copy behind
+// the step's kernels brings the window's.
+struct Fetch {
+    float *pin = nullptr;
+    size_t cap = 0; // floats
+    long gen = -1;
+    int w0 = 0, w1 = 0;
+};
+constexpr size_t MX_FETCH = 1 << 18; // most floats of a window (1 MB; one WFS if it has more)
+
 struct mx_wfsgrad_s {
     int device = 0;
     int nreal = 1; // realisations; WFS r * (nwfs / nreal) + i is realisation r's WFS i
@@ -2923,6 +2935,9 @@ struct mx_wfsgrad_s {
     bool pending_timing = false;
     // staging
     std::vector<float> hbuf;
+    // results of step step_gen on their way to the host (mx_wfsgrad_sync)
+    long step_gen = 0; // steps queued
+    Fetch f_grad, f_ints;
 };
 
 namespace {
@@ -2940,9 +2955,12 @@ DevLayer *g_dlayers = nullptr; // device [MX_MAXREAL][MX_MAXLAYER]
 // DM surfaces of one realisation
 struct DmState {
     int ndm = 0;
-    DevLayer h_layers[MX_MAXDM];
+    DevLayer h_layers[MX_MAXDM] = {};
+    bool tab_set = false; // h_layers is the device's table
     float *d_data = nullptr;
     size_t bytes = 0;
+    float *pin = nullptr; // the surfaces on their way to the GPU
+    size_t pin_len = 0;
 };
 DmState g_dm[MX_MAXREAL];
 DevLayer *g_ddms = nullptr; // device [MX_MAXREAL][MX_MAXDM]
@@ -3336,6 +3354,11 @@ int mx_wfsgrad_init_batch(mx_wfsgrad_t **out, const mx_powfs_t *p, const mx_wfs_
         if (hipMemcpy(h->d_llt_amp, la.data(), sizeof(float) * la.size(), hipMemcpyHostToDevice) != hipSuccess)
             return fail(set_err(MX_EHIP, "upload of LLT amplitude failed"));
     }
+    // the gradients' window (the intensities' is made when they are first read)
+    if (hipHostMalloc((void **)&h->f_grad.pin, sizeof(float) * std::max<size_t>(2 * nsa, std::min<size_t>(2 * nsa * nwfs, MX_FETCH))) !=
+        hipSuccess)
+        return fail(set_err(MX_EHIP, "hipHostMalloc failed"));
+    h->f_grad.cap = std::max<size_t>(2 * nsa, std::min<size_t>(2 * nsa * nwfs, MX_FETCH));
     // per-WFS constants; norm_ints of wfsints.c:111-115
     const double norm_psf = std::sqrt(p->areascale) / (double)(h->nxsa * h->nwvf);
     std::vector<DevWfs> dw(nwfs);
@@ -3416,6 +3439,8 @@ int mx_wfsgrad_free(mx_wfsgrad_t *h) {
     if (h->stream) hipStreamSynchronize(h->stream);
     if (h->stream2) hipStreamSynchronize(h->stream2);
     drop_graph(h);
+    for (Fetch *f : {&h->f_grad, &h->f_ints})
+        if (f->pin) hipHostFree(f->pin);
     void *ptrs[] = {h->d_ptsx, h->d_ptsy, h->d_amp, h->d_saa, h->d_wfs, h->d_wv, h->d_llt_amp, h->d_llt_opd, h->d_lotf,
                     h->d_lotf_t, h->d_F, h->d_F16, h->d_mwv, h->d_imcc, h->d_opdadd, h->d_ptt, h->d_lf_tw, h->d_b1, h->d_b2, h->d_b3, h->d_img,
                     h->d_lfw,
@@ -3825,16 +3850,23 @@ int mx_dm2gpu_real(int ireal, const mx_atm_layer_t *dms, int ndm) {
         D.bytes = total * sizeof(float);
     }
     if (!g_ddms) HIPCHK(hipMalloc(&g_ddms, sizeof(DevLayer) * MX_MAXREAL * MX_MAXDM));
+    // every surface in one copy from pinned memory, and the table of their
+    // geometry only where it changed (a control loop sends new shapes of the
+    // same mirrors before every step)
+    if (D.pin_len < total) {
+        if (D.pin) HIPCHK(hipHostFree(D.pin));
+        D.pin = nullptr;
+        D.pin_len = 0;
+        HIPCHK(hipHostMalloc((void **)&D.pin, total * sizeof(float)));
+        D.pin_len = total;
+    }
     size_t off = 0;
-    std::vector<float> tmp;
+    DevLayer tab[MX_MAXDM] = {};
     for (int i = 0; i < ndm; i++) {
         const mx_atm_layer_t &L = dms[i];
         const size_t n = (size_t)L.nx * L.ny;
-        tmp.resize(n);
-        for (size_t k = 0; k < n; k++) tmp[k] = (float)L.p[k];
-        HIPCHK(hipMemcpy(D.d_data + off, tmp.data(), n * sizeof(float), hipMemcpyHostToDevice));
-        DevLayer &d = D.h_layers[i];
-        d = DevLayer{};
+        for (size_t k = 0; k < n; k++) D.pin[off + k] = (float)L.p[k];
+        DevLayer &d = tab[i];
         d.p = D.d_data + off;
         d.nx = (int)L.nx;
         d.ny = (int)L.ny;
@@ -3845,8 +3877,14 @@ int mx_dm2gpu_real(int ireal, const mx_atm_layer_t *dms, int ndm) {
         d.ht = L.ht;
         off += n;
     }
-    HIPCHK(hipMemcpy(g_ddms + (size_t)ireal * MX_MAXDM, D.h_layers, sizeof(DevLayer) * MX_MAXDM,
-                     hipMemcpyHostToDevice));
+    if (total) HIPCHK(hipMemcpy(D.d_data, D.pin, total * sizeof(float), hipMemcpyHostToDevice));
+    if (!D.tab_set || std::memcmp(tab, D.h_layers, sizeof(tab)) != 0) {
+        D.tab_set = false;
+        std::memcpy(D.h_layers, tab, sizeof(tab));
+        HIPCHK(hipMemcpy(g_ddms + (size_t)ireal * MX_MAXDM, D.h_layers, sizeof(DevLayer) * MX_MAXDM,
+                         hipMemcpyHostToDevice));
+        D.tab_set = true;
+    }
     D.ndm = ndm;
     return MX_OK;
 }
@@ -4682,6 +4720,7 @@ void step_queued(mx_wfsgrad_t *h, const StepPlan &sp) {
     if (h->dith_on && h->last_out) h->dith_nframe++;
     if (h->pistat) h->pistat_nstep++; // every step, as MAOS accumulates it
     h->queued = true;
+    h->step_gen++;
 }
 } // namespace
 
@@ -4813,22 +4852,50 @@ int mx_wfsgrad_wait(mx_wfsgrad_t *h) {
     return MX_OK;
 }
 
+namespace {
+int fetch_room(Fetch &f, size_t need) {
+    if (f.cap >= need) return MX_OK;
+    if (f.pin) HIPCHK(hipHostFree(f.pin));
+    f.pin = nullptr;
+    f.cap = 0;
+    HIPCHK(hipHostMalloc((void **)&f.pin, sizeof(float) * need));
+    f.cap = need;
+    return MX_OK;
+}
+// starts the copy of WFS iwfs's n results (and the following WFS's, up to the
+// window) behind the queued work, unless the window has them
+int fetch_start(mx_wfsgrad_t *h, Fetch &f, const float *d, long n, int iwfs) {
+    if (f.gen == h->step_gen && iwfs >= f.w0 && iwfs < f.w1) return MX_OK;
+    const int k = (int)std::max<size_t>(1, std::min<size_t>(h->nwfs - iwfs, MX_FETCH / std::max(1L, n)));
+    const size_t need = (size_t)k * n;
+    f.gen = -1;
+    if (const int rc = fetch_room(f, need)) return rc;
+    HIPCHK(hipMemcpyAsync(f.pin, d + (size_t)iwfs * n, sizeof(float) * need, hipMemcpyDeviceToHost, h->stream));
+    f.w0 = iwfs;
+    f.w1 = iwfs + k;
+    f.gen = h->step_gen;
+    return MX_OK;
+}
+void fetch_read(const Fetch &f, long n, int iwfs, double *out) {
+    const float *p = f.pin + (size_t)(iwfs - f.w0) * n;
+    for (long i = 0; i < n; i++) out[i] = p[i];
+}
+} // namespace
+
 int mx_wfsgrad_sync(mx_wfsgrad_t *h, int iwfs, double *grad, double *ints) {
     if (!h || iwfs < 0 || iwfs >= h->nwfs) return set_err(MX_EINVAL, "mx_wfsgrad_sync: bad handle or iwfs");
     HIPCHK(hipSetDevice(h->device));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    const long nsa = h->nsa;
-    if (grad) {
-        h->hbuf.resize(2 * nsa);
-        HIPCHK(hipMemcpy(h->hbuf.data(), h->d_grad + iwfs * 2 * nsa, sizeof(float) * 2 * nsa, hipMemcpyDeviceToHost));
-        for (long i = 0; i < 2 * nsa; i++) grad[i] = h->hbuf[i];
+    const long ng = 2 * h->nsa, ni = h->nsa * h->npix;
+    int rc = MX_OK;
+    if (grad) rc = fetch_start(h, h->f_grad, h->d_grad, ng, iwfs);
+    if (!rc && ints) rc = fetch_start(h, h->f_ints, h->d_ints, ni, iwfs);
+    const hipError_t e = hipStreamSynchronize(h->stream);
+    if (rc || e != hipSuccess) { // nothing of an unfinished copy is handed out later
+        h->f_grad.gen = h->f_ints.gen = -1;
+        return rc ? rc : set_err(MX_EHIP, "mx_wfsgrad_sync failed: %s", hipGetErrorString(e));
     }
-    if (ints) {
-        const long n = nsa * h->npix;
-        h->hbuf.resize(n);
-        HIPCHK(hipMemcpy(h->hbuf.data(), h->d_ints + iwfs * n, sizeof(float) * n, hipMemcpyDeviceToHost));
-        for (long i = 0; i < n; i++) ints[i] = h->hbuf[i];
-    }
+    if (grad) fetch_read(h->f_grad, ng, iwfs, grad);
+    if (ints) fetch_read(h->f_ints, ni, iwfs, ints);
     return MX_OK;
 }
 
