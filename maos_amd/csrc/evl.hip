@@ -459,8 +459,11 @@ __global__ __launch_bounds__(256) void k_evl_ptt_fin(const double *part, double 
 // (prop to aper->locs with alpha = atmscale, maos/perfevl.c:275-300 and
 // gpu_atm2loc, cuda/sim/accphi.cu), then the DM surfaces subtracted
 // (alpha = -1, no wrap; a point outside a surface takes nothing from it).
-// The screen map is the one of the WFS ray trace with the point's own
-// coordinate as origin.
+// The screen map is the one of the WFS ray trace, a point's coordinate in
+// place of its index, its uniform part formed once per block.  Bound by the
+// screens' reads and the latency of the gathers: four layers' are in flight,
+// and neighbouring blocks share an XCD, so that the screen rows that two rows
+// of points read come from one L2.
 struct EvlOpdArgs {
     const DevLayer *layers; // [MX_MAXLAYER]
     const DevLayer *dms;    // [MX_MAXDM]
@@ -473,25 +476,43 @@ struct EvlOpdArgs {
 };
 
 __global__ __launch_bounds__(256) void k_evl_opd(EvlOpdArgs a) {
-    const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    const int idir = blockIdx.y;
-    if (i >= a.nloc) return;
-    const double x = a.locx[i], y = a.locy[i];
+    constexpr int G = 4; // layers in flight
+    __shared__ double map[MX_MAXLAYER][4]; // x scale, x origin, y scale, y origin of each layer
+    const int nblk = (int)((a.nloc + 255) / 256), idir = blockIdx.y, tid = (int)threadIdx.x;
     const double hs = a.hs[idir], ihs = hs != 0. ? 1. / hs : 0.;
     const double tx = a.thetax[idir], ty = a.thetay[idir];
+    if (tid < 2 * a.nps) { // (a point's coordinate is its step from the map's origin)
+        const bool ax = (tid & 1) == 0;
+        axis_map(a.layers[tid >> 1], ax, ihs, ax ? tx : ty, 0., 0., a.isim, a.dt, 1., 0., map[tid >> 1][ax ? 0 : 2],
+                 map[tid >> 1][ax ? 1 : 3]);
+    }
+    __syncthreads();
+    const long i = (long)xcd_unit((int)blockIdx.x, nblk) * 256 + tid;
+    if (i >= a.nloc) return;
+    const double x = a.locx[i], y = a.locy[i];
     float sum = 0.f;
-    for (int l = 0; l < a.nps; l++) {
-        const DevLayer &L = a.layers[l];
-        if (hs != 0. && L.ht > hs) continue;
-        int ix, iy;
-        float fx, fy;
-        screen_coord(L, true, 0, ihs, tx, 0., 0., a.isim, a.dt, 0., x, ix, fx);
-        screen_coord(L, false, 0, ihs, ty, 0., 0., a.isim, a.dt, 0., y, iy, fy);
-        const int ix1 = ix + 1 == L.nx ? 0 : ix + 1, iy1 = iy + 1 == L.ny ? 0 : iy + 1;
-        const float *r0 = L.p + (long)iy * L.nx, *r1 = L.p + (long)iy1 * L.nx;
-        const float v0 = fmaf(fx, r0[ix1] - r0[ix], r0[ix]);
-        const float v1 = fmaf(fx, r1[ix1] - r1[ix], r1[ix]);
-        sum += fmaf(fy, v1 - v0, v0);
+    for (int l0 = 0; l0 < a.nps; l0 += G) {
+        float fx[G], fy[G], q[G][4];
+#pragma unroll
+        for (int u = 0; u < G; u++) {
+            const int l = min(l0 + u, a.nps - 1); // (past the last layer: its loads again, not used)
+            const DevLayer &L = a.layers[l];
+            int ix, iy;
+            screen_wrap(L, true, x, map[l][0], map[l][1], ix, fx[u]);
+            screen_wrap(L, false, y, map[l][2], map[l][3], iy, fy[u]);
+            const int ix1 = ix + 1 == L.nx ? 0 : ix + 1, iy1 = iy + 1 == L.ny ? 0 : iy + 1;
+            const float *r0 = L.p + (long)iy * L.nx, *r1 = L.p + (long)iy1 * L.nx;
+            q[u][0] = r0[ix];
+            q[u][1] = r0[ix1];
+            q[u][2] = r1[ix];
+            q[u][3] = r1[ix1];
+        }
+#pragma unroll
+        for (int u = 0; u < G; u++) {
+            if (l0 + u >= a.nps || (hs != 0. && a.layers[l0 + u].ht > hs)) continue; // uniform
+            const float v0 = fmaf(fx[u], q[u][1] - q[u][0], q[u][0]), v1 = fmaf(fx[u], q[u][3] - q[u][2], q[u][2]);
+            sum += fmaf(fy[u], v1 - v0, v0);
+        }
     }
     float v = (float)((double)sum * a.atmscale);
     for (int d = 0; d < a.ndm; d++) {

@@ -404,10 +404,10 @@ __device__ __forceinline__ void axis_map(const DevLayer &L, bool isx, double ihs
     dout = ptsdx * d1 * scale;
     oout = orig * d1 * scale + (disp - o0) * d1;
 }
-__device__ __forceinline__ void screen_wrap(const DevLayer &L, bool isx, int i, double dout, double oout, int &ii,
+__device__ __forceinline__ void screen_wrap(const DevLayer &L, bool isx, double i, double dout, double oout, int &ii,
                                             float &ff) {
     const double nn = (double)(isx ? L.nx : L.ny);
-    double X = fma((double)i, dout, oout);
+    double X = fma(i, dout, oout);
     const double q = X * (isx ? L.inx : L.iny);
     double fq = floor(q);
     if (q - fq < 1e-9 || q - fq > 1. - 1e-9) fq = floor(X / nn);
