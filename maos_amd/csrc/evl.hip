@@ -194,36 +194,45 @@ constexpr int evl_clds() {
     return evl_cols<N>() * N + evl_cols<N>() * N / 16;
 }
 
+// One launch of a pass covers the wavelengths that share N and psfsize
+// (blockIdx.y), as many as their scratch allows: each alone leaves the chip
+// partly idle (132 row blocks for four directions of a 1024^2 grid, two uneven
+// rounds of 961 for one of 4096^2), and its tail would be waited for.
+struct PsfRowWvl {
+    const int2 *ent;  // (band position (iy - ylo) N + ix, point index), sorted by row
+    const int *rowp;  // [nband + 1] entry range of each band row
+    float2 *B;        // [ndir][P / C][nband][C]
+    int nband, ngroup;
+    double k;         // 1 / wvl
+};
 struct PsfRowArgs {
     const float *opd; // [ndir][nloc]
     const float *amp; // [nloc]
-    const int2 *ent;  // (band position (iy - ylo) N + ix, point index), sorted by row
-    const int *rowp;  // [nband + 1] entry range of each band row
     const float2 *tw; // [N]
-    float2 *B;        // [ndir][P / C][nband][C]
     long nloc;
-    int ndir, nband, ngroup, P, C;
-    double k; // 2 pi / wvl
+    int ndir, P, C;
+    PsfRowWvl w[MX_MAXWVL];
 };
 
 template <int N>
 __global__ __launch_bounds__(evl_threads<N>()) void k_psf_rows(PsfRowArgs a) {
     constexpr int R = evl_rows<N>(), T = evl_threads<N>();
     __shared__ float2 s[evl_lds<N>()];
-    const int unit = xcd_unit((int)blockIdx.x, a.ngroup * a.ndir);
-    const int idir = unit / a.ngroup, b0 = (unit % a.ngroup) * R;
-    const int nr = min(R, a.nband - b0);
+    const PsfRowWvl &w = a.w[blockIdx.y];
+    if ((int)blockIdx.x >= w.ngroup * a.ndir) return; // uniform: a wavelength with a shorter band
+    const int unit = xcd_unit((int)blockIdx.x, w.ngroup * a.ndir);
+    const int idir = unit / w.ngroup, b0 = (unit % w.ngroup) * R;
+    const int nr = min(R, w.nband - b0);
     for (int i = threadIdx.x; i < evl_lds<N>(); i += T) s[i] = make_float2(0.f, 0.f);
     __syncthreads();
-    const int e1 = a.rowp[b0 + nr];
+    const int e1 = w.rowp[b0 + nr];
     const float *op = a.opd + (long)idir * a.nloc;
-    const double twopi = 6.283185307179586476925;
     // four entries per thread per round, their loads issued together
-    for (int e0 = a.rowp[b0] + (int)threadIdx.x; e0 < e1; e0 += 4 * T) {
+    for (int e0 = w.rowp[b0] + (int)threadIdx.x; e0 < e1; e0 += 4 * T) {
         int2 en[4];
         float o[4], am[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) en[u] = e0 + u * T < e1 ? a.ent[e0 + u * T] : make_int2(-1, 0);
+        for (int u = 0; u < 4; u++) en[u] = e0 + u * T < e1 ? w.ent[e0 + u * T] : make_int2(-1, 0);
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             o[u] = op[en[u].y];
@@ -232,51 +241,56 @@ __global__ __launch_bounds__(evl_threads<N>()) void k_psf_rows(PsfRowArgs a) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             if (en[u].x < 0) continue;
-            // phase in FP64, reduced to [-pi, pi] before the FP32 sincos
-            double ph = (double)o[u] * a.k;
-            ph -= rint(ph * (1. / twopi)) * twopi;
+            // phase in revolutions, reduced to [-1/2, 1/2] in FP64
+            double ph = (double)o[u] * w.k;
+            ph -= rint(ph);
             float sn, cs;
-            sincosf((float)ph, &sn, &cs);
+            sincospif(2.f * (float)ph, &sn, &cs);
             s[lp(en[u].x - b0 * N)] = make_float2(am[u] * cs, am[u] * sn);
         }
     }
     lds_fft<N, R, T>(s, a.tw);
     // centre window columns c < P: kx = c - P/2 (mod N)
     const int ncb = a.P / a.C, C = a.C;
-    float2 *dst = a.B + (long)idir * ncb * a.nband * C;
+    float2 *dst = w.B + (long)idir * ncb * w.nband * C;
     for (int i = threadIdx.x; i < ncb * nr * C; i += T) {
         const int cc = i % C, rr = (i / C) % nr, cb = i / (C * nr);
         const int kx = (cb * C + cc - a.P / 2 + N) & (N - 1);
-        dst[((long)cb * a.nband + b0 + rr) * C + cc] = s[lp(rr * N + kx)];
+        dst[((long)cb * w.nband + b0 + rr) * C + cc] = s[lp(rr * N + kx)];
     }
 }
 
-struct PsfColArgs {
+struct PsfColWvl {
     const float2 *B;  // [ndir][P / C][nband][C]
-    const float2 *tw; // [N]
     float *acc;       // [ndir][P (x)][P (y)]
-    int ndir, nband, ylo, P, C, ncb;
+    int nband, ylo;
+};
+struct PsfColArgs {
+    const float2 *tw; // [N]
+    int ndir, P, C, ncb;
     int CK, nck; // columns per workgroup (a power of two dividing P, at most evl_cols), P / CK
+    PsfColWvl w[MX_MAXWVL];
 };
 
 template <int N>
 __global__ __launch_bounds__(evl_cthreads<N>()) void k_psf_cols(PsfColArgs a) {
     constexpr int CM = evl_cols<N>(), T = evl_cthreads<N>();
     __shared__ float2 s[evl_clds<N>()];
+    const PsfColWvl &w = a.w[blockIdx.y];
     const int unit = xcd_unit((int)blockIdx.x, a.nck * a.ndir);
     const int idir = unit / a.nck, c0 = (unit % a.nck) * a.CK;
     const int C = a.C, CK = a.CK;
     // Both HBM round trips are started early: the column values before the
     // LDS is cleared, the accumulator values before the FFT.  Each lane
     // holds at most 16 of each (nband CK <= N CK = 16 T and CK P <= 16 T).
-    const int nin = a.nband * CK, nout = CK * a.P;
+    const int nin = w.nband * CK, nout = CK * a.P;
     float2 pre[16];
 #pragma unroll
     for (int u = 0; u < 16; u++) {
         const int i = (int)threadIdx.x + u * T;
         if (i < nin) {
             const int c = c0 + i % CK, b = i / CK;
-            pre[u] = a.B[(((long)idir * a.ncb + c / C) * a.nband + b) * C + c % C];
+            pre[u] = w.B[(((long)idir * a.ncb + c / C) * w.nband + b) * C + c % C];
         }
     }
     for (int i = threadIdx.x; i < evl_clds<N>(); i += T) s[i] = make_float2(0.f, 0.f);
@@ -284,9 +298,9 @@ __global__ __launch_bounds__(evl_cthreads<N>()) void k_psf_cols(PsfColArgs a) {
 #pragma unroll
     for (int u = 0; u < 16; u++) {
         const int i = (int)threadIdx.x + u * T;
-        if (i < nin) s[lp((i % CK) * N + a.ylo + i / CK)] = pre[u];
+        if (i < nin) s[lp((i % CK) * N + w.ylo + i / CK)] = pre[u];
     }
-    float *acc = a.acc + ((long)idir * a.P + c0) * a.P; // column cc = i / P, row r = i % P
+    float *acc = w.acc + ((long)idir * a.P + c0) * a.P; // column cc = i / P, row r = i % P
     float old[16];
 #pragma unroll
     for (int u = 0; u < 16; u++) {
@@ -543,15 +557,15 @@ struct EvlWvl {
     double *d_acc1 = nullptr; // [ndir], psfsize 1
 };
 
-// the two passes of one wavelength; with ev (timing) each pass is bracketed
+// the two passes of nw wavelengths; with ev (timing) each pass is bracketed
 // by events and waited for, and its time added to ms[0] (rows) and ms[1]
 // (columns)
 template <int N>
-int psf_launch(const EvlWvl &w, PsfRowArgs &ra, PsfColArgs &ca, hipStream_t st, hipEvent_t *ev, double *ms) {
+int psf_launch(int nw, int ngroup, const PsfRowArgs &ra, const PsfColArgs &ca, hipStream_t st, hipEvent_t *ev, double *ms) {
     if (ev) HIPCHK(hipEventRecord(ev[0], st));
-    k_psf_rows<N><<<dim3((unsigned)(w.ngroup * ra.ndir)), dim3(evl_threads<N>()), 0, st>>>(ra);
+    k_psf_rows<N><<<dim3((unsigned)(ngroup * ra.ndir), (unsigned)nw), dim3(evl_threads<N>()), 0, st>>>(ra);
     if (ev) HIPCHK(hipEventRecord(ev[1], st));
-    k_psf_cols<N><<<dim3((unsigned)(w.nck * ca.ndir)), dim3(evl_cthreads<N>()), 0, st>>>(ca);
+    k_psf_cols<N><<<dim3((unsigned)(ca.nck * ca.ndir), (unsigned)nw), dim3(evl_cthreads<N>()), 0, st>>>(ca);
     if (ev) {
         HIPCHK(hipEventRecord(ev[2], st));
         HIPCHK(hipEventSynchronize(ev[2]));
@@ -579,6 +593,7 @@ struct mx_evl_s {
     double *h_tot = nullptr;                     // pinned: the p/t/t sums [ndir][4], written by the GPU
     double imcc[9] = {}, ipcc = 0;               // inverse of sum amp [1 x y]^T [1 x y], 1 / sum amp
     float2 *d_B = nullptr;
+    size_t b_len = 0; // its elements
     double *d_out = nullptr; // PSF rows on their way to the host, [out_len]
     long out_len = 0;
     EvlWvl w[MX_MAXWVL];
@@ -653,28 +668,39 @@ void evl_release(mx_evl_t *h) {
 int evl_psf_queue(mx_evl_t *h, const float *d_opd) {
     const hipStream_t st = h->stream;
     hipEvent_t *ev = h->timing ? h->ev : nullptr;
-    for (int iw = 0; iw < h->nwvl; iw++) {
+    for (int iw = 0; iw < h->nwvl;) {
         EvlWvl &w = h->w[iw];
-        const double k = 2. * M_PI / w.wvl;
         if (w.P == 1) {
-            StrehlArgs sa{d_opd, h->d_amp, h->d_part, w.d_acc1, h->nloc, k};
+            StrehlArgs sa{d_opd, h->d_amp, h->d_part, w.d_acc1, h->nloc, 2. * M_PI / w.wvl};
             k_strehl_part<<<dim3(MX_STREHL_PARTS, (unsigned)h->ndir), dim3(256), 0, st>>>(sa);
             k_strehl_fin<<<dim3((unsigned)h->ndir), dim3(64), 0, st>>>(sa);
+            iw++;
             continue;
         }
-        PsfRowArgs ra{d_opd, h->d_amp, w.d_ent, w.d_rowp, w.d_tw, h->d_B, h->nloc, h->ndir, w.nband, w.ngroup,
-                      w.P, w.C, k};
-        PsfColArgs ca{h->d_B, w.d_tw, w.d_acc, h->ndir, w.nband, w.ylo, w.P, w.C, w.ncb, w.CK, w.nck};
+        PsfRowArgs ra{d_opd, h->d_amp, w.d_tw, h->nloc, h->ndir, w.P, w.C, {}};
+        PsfColArgs ca{w.d_tw, h->ndir, w.P, w.C, w.ncb, w.CK, w.nck, {}};
+        int nw = 0, ngroup = 0;
+        size_t off = 0;
+        for (; iw < h->nwvl; iw++, nw++) { // the following wavelengths of the same sizes, while the scratch holds them
+            EvlWvl &v = h->w[iw];
+            const size_t len = (size_t)h->ndir * v.nband * v.P;
+            if (v.N != w.N || v.P != w.P || off + len > h->b_len) break;
+            float2 *B = h->d_B + off;
+            ra.w[nw] = PsfRowWvl{v.d_ent, v.d_rowp, B, v.nband, v.ngroup, 1. / v.wvl};
+            ca.w[nw] = PsfColWvl{B, v.d_acc, v.nband, v.ylo};
+            ngroup = std::max(ngroup, v.ngroup);
+            off += len;
+        }
         int rc;
         switch (w.N) {
-        case 32: rc = psf_launch<32>(w, ra, ca, st, ev, h->t_pass); break;
-        case 64: rc = psf_launch<64>(w, ra, ca, st, ev, h->t_pass); break;
-        case 128: rc = psf_launch<128>(w, ra, ca, st, ev, h->t_pass); break;
-        case 256: rc = psf_launch<256>(w, ra, ca, st, ev, h->t_pass); break;
-        case 512: rc = psf_launch<512>(w, ra, ca, st, ev, h->t_pass); break;
-        case 1024: rc = psf_launch<1024>(w, ra, ca, st, ev, h->t_pass); break;
-        case 2048: rc = psf_launch<2048>(w, ra, ca, st, ev, h->t_pass); break;
-        case 4096: rc = psf_launch<4096>(w, ra, ca, st, ev, h->t_pass); break;
+        case 32: rc = psf_launch<32>(nw, ngroup, ra, ca, st, ev, h->t_pass); break;
+        case 64: rc = psf_launch<64>(nw, ngroup, ra, ca, st, ev, h->t_pass); break;
+        case 128: rc = psf_launch<128>(nw, ngroup, ra, ca, st, ev, h->t_pass); break;
+        case 256: rc = psf_launch<256>(nw, ngroup, ra, ca, st, ev, h->t_pass); break;
+        case 512: rc = psf_launch<512>(nw, ngroup, ra, ca, st, ev, h->t_pass); break;
+        case 1024: rc = psf_launch<1024>(nw, ngroup, ra, ca, st, ev, h->t_pass); break;
+        case 2048: rc = psf_launch<2048>(nw, ngroup, ra, ca, st, ev, h->t_pass); break;
+        case 4096: rc = psf_launch<4096>(nw, ngroup, ra, ca, st, ev, h->t_pass); break;
         default: return set_err(MX_EINVAL, "internal: nembed %d", w.N);
         }
         if (rc) return rc;
@@ -770,7 +796,7 @@ int mx_evl_init(mx_evl_t **out, long nloc, const double *locx, const double *loc
         EVCHK(hipHostMalloc((void **)&h->h_tot, sizeof(double) * 4 * ndir));
         EVCHK(hipMemcpy(h->d_amp64, amp, sizeof(double) * nloc, hipMemcpyHostToDevice));
     }
-    size_t bmax = 0;
+    size_t bmax = 0, bsum = 0;
     for (int iw = 0; iw < nwvl; iw++) {
         EvlWvl &w = h->w[iw];
         w.wvl = wvl[iw];
@@ -842,9 +868,12 @@ int mx_evl_init(mx_evl_t **out, long nloc, const double *locx, const double *loc
         EVCHK(hipMemcpy(w.d_tw, tw.data(), sizeof(float2) * N, hipMemcpyHostToDevice));
         EVCHK(hipMemset(w.d_acc, 0, sizeof(float) * ndir * w.P * w.P));
         bmax = std::max(bmax, (size_t)ndir * w.nband * w.P);
+        bsum += (size_t)ndir * w.nband * w.P;
         h->out_len = std::max(h->out_len, std::min((long)w.P * w.P, std::max((long)w.P, MX_PSF_OUT)));
     }
-    if (bmax && (rc = dev_alloc(&h->d_B, bmax))) return fail(rc);
+    // the row passes' output of every wavelength, up to 256 MB of it (at least one's)
+    h->b_len = std::max(bmax, std::min(bsum, (size_t)(256 << 20) / sizeof(float2)));
+    if (bmax && (rc = dev_alloc(&h->d_B, h->b_len))) return fail(rc);
     EVCHK(hipDeviceSynchronize());
     *out = h;
     return MX_OK;

@@ -64,3 +64,35 @@ def test_wavefront_error_slices(n, ndir):
         tol = 1e3 * len(x) * 2.0 ** -53
         assert np.abs(rms[d] - [tot - pis, ptt - pis, tot - ptt]).max() <= tol * tot
         assert np.abs(coeff[d] - q).max() <= tol * np.abs(o).max() * max(1, 1 / np.abs(x).max())
+
+
+def test_wavelengths_of_several_sizes():
+    """Wavelengths that share a launch (the same sizes, other bands), that do
+    not, a Strehl-only one between them, and scratch for one at a time (134 MB
+    each of two directions) give what handles of one wavelength give."""
+    from maos_amd import engine
+    x, y = _points(9)
+    amp = np.linspace(1, 2, len(x))
+    opd = np.random.default_rng(5).normal(size=(2, len(x))) * 2e-7
+    dirs = [(0, 0, 0)] * 2
+    ix, iy = np.round((x - x.min()) * 16).astype(int), np.round((y - y.min()) * 16).astype(int)
+
+    def emb(N, sy, oy):  # rows sy apart from row oy on
+        return (ix + 3) + (iy * sy + oy) * N
+    for spec in ([(64, 32, 1, 5), (64, 32, 5, 2), (64, 1, 1, 0), (128, 32, 3, 0)],
+                 [(64, 32, 1, 5), (128, 128, 15, 0), (64, 32, 2, 5), (64, 32, 5, 2)],
+                 [(4096, 2048, 500, 0), (4096, 2048, 511, 1), (4096, 2048, 300, 9)]):
+        print("case: wavelengths of sizes %s" % (spec,), flush=True)
+        wvl = [1e-6 * (1 + 0.1 * k) for k in range(len(spec))]
+        e = [emb(N, sy, oy) for N, P, sy, oy in spec]
+        ev = engine.Evl(amp, wvl, [s[0] for s in spec], [s[1] for s in spec], np.concatenate(e), dirs=dirs)
+        ev.psf_add(opd)
+        ev.psf_add(0.5 * opd)
+        for k, (N, P, _, _) in enumerate(spec):
+            one = engine.Evl(amp, [wvl[k]], [N], [P], e[k], dirs=dirs)
+            one.psf_add(opd)
+            one.psf_add(0.5 * opd)
+            for d in range(2):
+                assert np.array_equal(ev.psf(d, k)[0], one.psf(d, 0)[0])
+            one.close()
+        ev.close()
