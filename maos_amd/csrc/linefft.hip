@@ -2,12 +2,13 @@
 // in place by one block, for the large-field Shack-Hartmann passes and the
 // pyramid WFS.
 //
-// The transform is a Stockham autosort over few, large radices (2 to 10, 12
-// and 16; at most four stages up to 4096 points where the length allows).
+// The transform is a Stockham autosort over few, large radices (2 to 10, 12,
+// 16 and 18; at most four stages up to 4096 points where the length allows).
 // What bounds such a pass is the chain of its stages: an LDS round trip, the
 // twiddle loads and barriers each.  So
-//  - the radices are large (512 = 8 8 8, 480 = 16 6 5, 2916 = 9 9 9 4 rather
-//    than 4 3 3 3 3 3 3), a thread holding up to LX_E points in registers;
+//  - the radices are large (512 = 8 8 8, 480 = 16 6 5, 2916 = 18 18 9 rather
+//    than 4 3 3 3 3 3 3; as 9 9 9 4 a pyramid step of that grid took 4.13 ms
+//    against 3.85), a thread holding up to LX_E points in registers;
 //  - the first stage reads its points through a functor (from global memory,
 //    or computed) and the last one hands its points to a functor, so a
 //    transform of s stages makes s - 1 LDS round trips and touches no LDS
@@ -178,6 +179,8 @@ struct LxRoots {
 };
 // R1 R2 points as R2 transforms of R1 (points R2 n1 + n2), the twiddles
 // w^(n2 k1) and R1 transforms of R2; output k1 + R1 k2
+template <int R, bool INV>
+__device__ __forceinline__ void lx_dft(float2 (&v)[R]);
 template <int R1, int R2, bool INV>
 __device__ __forceinline__ void comp_dft(float2 (&v)[R1 * R2]) {
     constexpr LxRoots<R1 * R2> W{};
@@ -188,7 +191,7 @@ __device__ __forceinline__ void comp_dft(float2 (&v)[R1 * R2]) {
         float2 u[R1];
 #pragma unroll
         for (int n1 = 0; n1 < R1; n1++) u[n1] = v[R2 * n1 + n2];
-        small_dft<R1>(u, t);
+        lx_dft<R1, INV>(u);
 #pragma unroll
         for (int k1 = 0; k1 < R1; k1++)
             if (n2 * k1) {
@@ -203,7 +206,7 @@ __device__ __forceinline__ void comp_dft(float2 (&v)[R1 * R2]) {
         float2 u[R2];
 #pragma unroll
         for (int n2 = 0; n2 < R2; n2++) u[n2] = a[n2][k1];
-        small_dft<R2>(u, t);
+        lx_dft<R2, INV>(u);
 #pragma unroll
         for (int k2 = 0; k2 < R2; k2++) v[k1 + R1 * k2] = u[k2];
     }
@@ -215,6 +218,7 @@ __device__ __forceinline__ void lx_dft(float2 (&v)[R]) {
     else if constexpr (R == 10) comp_dft<2, 5, INV>(v);
     else if constexpr (R == 12) comp_dft<4, 3, INV>(v);
     else if constexpr (R == 16) comp_dft<4, 4, INV>(v);
+    else if constexpr (R == 18) comp_dft<3, 6, INV>(v);
     else if constexpr (R > 1) small_dft<R>(v, INV ? 1.f : -1.f);
 }
 // which index of (line, butterfly) is fastest over the threads: the
@@ -296,7 +300,7 @@ __device__ __forceinline__ void lx_stage(float2 *s, LxPlan P, const LxLines &g, 
 // points would pass through memory)
 #define LX_INLINE __attribute__((always_inline))
 #define LX_RADIX(X)                                                                                                  \
-    X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(12) X(16)
+    X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(12) X(16) X(18)
 // FFT of the block's g.L lines (exp(-i ...); INV: exp(+i ...), not scaled):
 // points come from ld by map MI and go to st by map MO; LDSIN: ld reads LDS.
 //   Every thread of the block takes part, and
@@ -345,7 +349,7 @@ __device__ __forceinline__ void lx_outputs(LxPlan P, const LxLines &g, F &&f) {
 // single radix gets a stage of radix 1 after it, so that there are always a
 // first and a last one.  False if n does not factor so.
 inline void lx_search(long n, int most, std::vector<int> &cur, std::vector<int> &best) {
-    static const int rad[] = {16, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+    static const int rad[] = {18, 16, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
     if (n == 1) {
         auto cap = [](const std::vector<int> &v) {
             int c = LX_E;
@@ -377,7 +381,7 @@ inline bool lx_plan(long n, LinePlan &P) {
     P = LinePlan{};
     if (n < 2) return false;
     std::vector<int> cur, best;
-    lx_search(n, 16, cur, best);
+    lx_search(n, 18, cur, best);
     if (best.empty() || best.size() > (size_t)LX_MAXST - 1) return false;
     if (best.size() == 1) best.push_back(1);
     P.n = (int)n;

@@ -117,26 +117,38 @@ __global__ __launch_bounds__(1024) void k_py_rows(PyArgs a) {
         const float *inr = MODE == PY_REAL ? a.inr + (long)r0 * n : nullptr;
         const int nsplit = a.nsplit;
         const long nn = (long)n * n;
-        lx_fft<MODE == PY_IMG, LX_ROW, LX_ROW, false>(
-            pyl, plan, ln,
-            [&](int l, int j, int off) LX_INLINE {
-                const bool ok = l < nl;
-                const int i = ok ? __mul24(l, n) + j + off : 0;
-                if constexpr (MODE == PY_IMG) return lx_sel(ok, lx_at(in, i));
-                float v = 0.f;
+        auto store = [&](int l, int d, int off, float2 v, int) LX_INLINE {
+            if (l >= nl) return;
+            const int i = __mul24(l, n) + d;
+            if constexpr (MODE == PY_IMG) lx_at(a.outr + (long)r0 * n + off, i) = v.x;
+            else lx_at(a.out + (long)r0 * n + off, i) = v;
+        };
+        if (MODE == PY_IMG || nsplit == 1) {
+            lx_fft<MODE == PY_IMG, LX_ROW, LX_ROW, false>(
+                pyl, plan, ln,
+                [&](int l, int j, int off) LX_INLINE {
+                    const bool ok = l < nl;
+                    const int i = ok ? __mul24(l, n) + j + off : 0;
+                    if constexpr (MODE == PY_IMG) return lx_sel(ok, lx_at(in, i));
+                    else return lx_sel(ok, make_float2(lx_at(inr, i), 0.f));
+                },
+                store);
+        } else if constexpr (MODE == PY_REAL) {
+            lx_fft<false, LX_ROW, LX_ROW, false>(
+                pyl, plan, ln,
+                [&](int l, int j, int off) LX_INLINE {
+                    const bool ok = l < nl;
+                    const int i = ok ? __mul24(l, n) + j + off : 0;
+                    float v = 0.f;
 #pragma unroll
-                for (int q = 0; q < MX_PY_MAXSPLIT; q++) { // (loads of all at once, past the last split the first again)
-                    const float t = lx_at(inr + (q < nsplit ? q * nn : 0), i);
-                    v += q < nsplit ? t : 0.f;
-                }
-                return make_float2(ok ? v : 0.f, 0.f);
-            },
-            [&](int l, int d, int off, float2 v, int) LX_INLINE {
-                if (l >= nl) return;
-                const int i = __mul24(l, n) + d;
-                if constexpr (MODE == PY_IMG) lx_at(a.outr + (long)r0 * n + off, i) = v.x;
-                else lx_at(a.out + (long)r0 * n + off, i) = v;
-            });
+                    for (int q = 0; q < MX_PY_MAXSPLIT; q++) { // (loads of all at once, past the last split the first again)
+                        const float t = lx_at(inr + (q < nsplit ? q * nn : 0), i);
+                        v += q < nsplit ? t : 0.f;
+                    }
+                    return make_float2(ok ? v : 0.f, 0.f);
+                },
+                store);
+        }
     }
 }
 

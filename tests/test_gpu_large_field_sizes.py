@@ -14,9 +14,9 @@ INTS_TOL = 2e-5  # the parity bars of the forms
 GRAD_TOL_MAS = 0.1
 
 
-# nxsa, embfac, notf: 16 -> 48 = 12 4; 48 in 70 = 10 7; 80 = 10 8 in 84 = 12 7;
+# nxsa, embfac, notf: 16 -> 48 = 12 4 or 6 8; 70 = 10 7; 80 = 10 8; 84 = 12 7;
 # 96 in 210 (7); 96 in 250 (5 5 10) and 256 (columns of 129 points, the longest
-# of the staged sums); 128 in 270 (27 10) (columns of 136,
+# of the staged sums); 128 in 270 = 18 .. (columns of 136,
 # summed by waves); 432 in 486 = 2 3^5; 480 in 1000 (10 10 10); 448 = 64 7
 @pytest.mark.parametrize("nxsa,embfac,notf", [(16, 3, 48), (16, 3, 70), (16, 5, 84), (48, 2, 210), (48, 2, 250),
                                               (48, 2, 256), (64, 2, 270), (144, 3, 486), (240, 2, 1000),
