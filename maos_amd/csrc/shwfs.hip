@@ -3027,11 +3027,14 @@ const void *lf_kernel(int q) {
 }
 // lines per block of a pass over nlines lines of n points in each of nchain
 // chains: a power of two up to 16 of at most 16 points for each of `threads`
-// threads (4096 points at 256, about 35 KB of LDS), fewer while that leaves
+// threads (4096 points at 256, about 35 KB of LDS), fewer while the
+// last group's empty lines are more than an eighth of the pass (the 65 rows of a 128^2 OTF in groups
+// of 16: 333 us a step of the padded LGS case, of 8: 323) or while that leaves
 // less than two blocks for a CU, but at least lmin.
 int lf_lines(int n, int nlines, int nchain, int threads, int lmin) {
     int L = 16;
     while (L > lmin && L * n > 16 * threads) L /= 2;
+    while (L > std::max(lmin, 4) && ((nlines + L - 1) / L * L - nlines) * 8 > nlines) L /= 2;
     while (L > lmin && (long)((nlines + L - 1) / L) * nchain < 512) L /= 2;
     return L;
 }
