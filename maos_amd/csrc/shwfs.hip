@@ -2274,8 +2274,9 @@ __global__ __launch_bounds__(256) void k_llt_acorr(LltAcorrArgs a) {
 //   D  FFT those rows of B2 (columns padded the same way), x nominal or
 //      conj(lotf) ETF, inverse FFT, keep the columns the detector samples
 //                                                     -> B3 [nx][notf/2+1]
-//   E  the sampled rows of those columns, summed directly over uy (the other
-//      half plane is the conjugate)                  -> image [ny][nx]
+//   E  the sampled rows of those columns: few of them summed directly over uy
+//      (the other half plane is the conjugate), many of them, or the whole
+//      image, by inverse FFTs                        -> image [ny][nx]
 // then k_lf_sample applies si (maos/wfsints.c:286) and the pixel processing.
 // The |E|^2 never leaves the chip, and every factor after it is the transform
 // of a real function, so half the plane is enough.
@@ -2290,6 +2291,16 @@ constexpr int MX_LF_THREADS = 512; // most threads per block the choice of L aim
 constexpr int MX_LF_MAXS = 128;    // most sampled rows / columns kept (else the full image)
 constexpr int MX_LF_ESUB = 8;      // lanes that share one output of pass E
 constexpr int MX_LF_ESHORT = 129;  // longest column (m/2 + 1) of its staged form
+// Most sampled rows for which pass E sums its outputs directly.  The direct
+// sums cost ny terms a column and are FP64; the line FFTs cost the same for any
+// ny.  Imaging of a step in us, direct / FFT, for detectors whose pixels are two
+// samples apart:
+//                       24 rows   32 rows   48 rows   64 rows   whole image
+//   12 chains of 512^2   72 / 75   74 / 75   84 / 78   94 / 80   1393 / 124
+//   one of 1024^2        51 / 56   51 / 56   54 / 58   56 / 59    851 / 93
+//   12 of 128^2          48 / 39   52 / 39   62 / 41   71 / 42
+constexpr int MX_LF_EROWS = 32;
+constexpr long MX_LF_EWAVES = 1L << 21; // most blocks of the direct sums of long columns (a launch has 2^24)
 // complex elements of pass E's column buffer
 constexpr int MX_LF_ECOL = 2080;
 // columns per block of pass E: as many as the buffer holds, at most 16
@@ -2490,8 +2501,8 @@ __global__ __launch_bounds__(1024) void k_lf_d(LfArgs a) {
 
 // pass E: the inverse transform along y of the sampled columns at the sampled
 // rows, real part: I[ys][xs] = Re sum_{uy <= m/2} w(uy) B3[xs][uy]
-// exp(+2 pi i uy ys / m), w = 1 at 0 and m/2, else 2.  A few tens of outputs
-// per column, so they are summed directly, in FP64, rather than transformed.
+// exp(+2 pi i uy ys / m), w = 1 at 0 and m/2, else 2.  Up to MX_LF_EROWS rows
+// are summed directly, in FP64, rather than transformed (k_lf_e_fft).
 // Short columns (mh <= MX_LF_ESHORT): XG columns staged in LDS, MX_LF_ESUB
 // lanes an output (k_lf_e).  Long ones, of which there are few: a wave per
 // output straight from L2 (k_lf_e_wave), since the staged form leaves too few
@@ -2553,6 +2564,42 @@ __global__ __launch_bounds__(256) void k_lf_e(LfArgs a) {
 #pragma unroll
         for (int d = 1; d < MX_LF_ESUB; d <<= 1) acc += __shfl_xor(acc, d);
         if (on && sub == 0) out[(long)iyy * W.nx + xs0 + xl] = (float)acc;
+    }
+}
+
+// Many sampled rows, above all the whole image: the columns' inverse line
+// FFTs, two columns a and b per complex line as a + i b (their values are
+// real: the imaginary parts at 0 and m/2 do not count), the part past m/2 by
+// conjugation; the sampled rows are picked from LDS.
+__global__ __launch_bounds__(1024) void k_lf_e_fft(LfArgs a) {
+    const int m = a.notf, h = m / 2, mh = h + 1, L = a.L, S = a.pm.S;
+    const LxLines ln{L, a.lgL};
+    int g, c, iwfs, isa, iwvl;
+    lf_unit(a, ((a.maxnx + 1) / 2 + L - 1) / L, g, c);
+    lf_chain(a, c, iwfs, isa, iwvl);
+    const LfWvl &W = a.wv[iwvl];
+    const int x0 = 2 * L * g, nx = W.nx - x0; // sampled columns from this group on
+    if (nx <= 0) return; // uniform: no sampled column in this group
+    const float2 *in = a.b3 + ((long)c * a.maxnx + x0) * mh;
+    lx_fft<true, LX_ROW, LX_ROW, false>(
+        lfs, LX_PLAN(LfArgs, pm), ln,
+        [&](int l, int j, int off) LX_INLINE {
+            const int e = j + off, k = e <= h ? e : m - e;
+            const bool ok0 = 2 * l < nx, ok1 = 2 * l + 1 < nx;
+            const float2 p = lx_sel(ok0, lx_at(in, ok0 ? __mul24(2 * l, mh) + k : 0));
+            const float2 q = lx_sel(ok1, lx_at(in, ok1 ? __mul24(2 * l + 1, mh) + k : 0));
+            const bool edge = k == 0 || k == h;
+            const float py = edge ? 0.f : (e <= h ? p.y : -p.y), qy = edge ? 0.f : (e <= h ? q.y : -q.y);
+            return make_float2(p.x - qy, py + q.x);
+        },
+        [&](int l, int d, int off, float2 v, int) LX_INLINE { lfs[__mul24(l, S) + d + off] = v; });
+    __syncthreads();
+    float *out = a.img + (long)c * a.maxny * a.maxnx + x0;
+    for (int e = threadIdx.x; e < 2 * L * W.ny; e += blockDim.x) {
+        const int x = e & (2 * L - 1), iyy = e >> (a.lgL + 1);
+        if (x >= nx) continue;
+        const float2 v = lfs[__mul24(x >> 1, S) + W.rows[iyy]];
+        out[(long)iyy * W.nx + x] = x & 1 ? v.y : v.x;
     }
 }
 
@@ -3018,11 +3065,13 @@ bool supported(long notf, long nxsa, long embfac) {
     return (notf == 64 && nxsa == 32 && embfac == 2) || (notf == 32 && nxsa == 16 && embfac == 2);
 }
 
-// pass q of the large-field form (0..3: A, B, D, E; 4: the uplink's D; 5: E of long columns)
+// pass q of the large-field form (0..3: A, B, D, E; 4: the uplink's D; 5: E of
+// long columns, 6: of many rows)
 const void *lf_kernel(int q) {
-    const void *k[6] = {reinterpret_cast<const void *>(&k_lf_a), reinterpret_cast<const void *>(&k_lf_b),
+    const void *k[7] = {reinterpret_cast<const void *>(&k_lf_a), reinterpret_cast<const void *>(&k_lf_b),
                         reinterpret_cast<const void *>(&k_lf_d<false>), reinterpret_cast<const void *>(&k_lf_e),
-                        reinterpret_cast<const void *>(&k_lf_d<true>), reinterpret_cast<const void *>(&k_lf_e_wave)};
+                        reinterpret_cast<const void *>(&k_lf_d<true>), reinterpret_cast<const void *>(&k_lf_e_wave),
+                        reinterpret_cast<const void *>(&k_lf_e_fft)};
     return k[q];
 }
 // lines per block of a pass over nlines lines of n points in each of nchain
@@ -3278,7 +3327,7 @@ int mx_wfsgrad_init_batch(mx_wfsgrad_t **out, const mx_powfs_t *p, const mx_wfs_
     if (lf) {
         // blocks of 512 threads (an autotune candidate) may exceed the default
         // dynamic LDS limit
-        for (int q : {0, 1, 2, 4})
+        for (int q : {0, 1, 2, 4, 6})
             if (hipFuncSetAttribute(lf_kernel(q), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess) {
                 mx_wfsgrad_free(h);
                 return set_err(MX_EHIP, "the large-field kernels' LDS size could not be set");
@@ -3900,11 +3949,22 @@ int mx_dm2gpu(const mx_atm_layer_t *dms, int ndm) { return mx_dm2gpu_real(0, dms
 // its lines per block set in u
 StepLaunch lf_launch(const mx_wfsgrad_t *h, LfArgs &u, int q, bool up) {
     const int n = u.nwvf, m = u.notf, mh = m / 2 + 1, T = h->lf_threads;
-    if (q == 3 && mh > MX_LF_ESHORT) {
-        StepLaunch e{lf_kernel(5), dim3((unsigned)((u.maxny * u.maxnx + 3) / 4 * u.nchain)), dim3(256), &u};
-        return e;
-    }
     if (q == 3) {
+        const long outs = (long)u.maxny * u.maxnx, waves = (outs + 3) / 4 * u.nchain; // blocks of four waves
+        const bool fft = u.maxny > MX_LF_EROWS || (mh > MX_LF_ESHORT && waves > MX_LF_EWAVES);
+        if (fft) {
+            const int npair = (u.maxnx + 1) / 2;
+            u.L = lf_lines(m, npair, u.nchain, T, 1);
+            u.lgL = ilog2c(u.L);
+            StepLaunch e{lf_kernel(6), dim3((unsigned)((npair + u.L - 1) / u.L * u.nchain)),
+                         dim3((unsigned)lx_threads(u.pm, u.L)), &u};
+            e.lds = (unsigned)(sizeof(float2) * u.L * u.pm.S);
+            return e;
+        }
+        if (mh > MX_LF_ESHORT) {
+            StepLaunch e{lf_kernel(5), dim3((unsigned)waves), dim3(256), &u};
+            return e;
+        }
         const int XG = lf_ecols(mh);
         StepLaunch e{lf_kernel(3), dim3((unsigned)((u.maxnx + XG - 1) / XG * u.nchain)), dim3(256), &u};
         return e;
