@@ -31,6 +31,7 @@
 // bound by the 16-byte runs that it reads of each row).
 constexpr int MX_PY_MAXN = 4096;
 constexpr int MX_PY_MAXSIDE = 4;
+constexpr int MX_PY_LDS = 96 * 1024;        // most LDS of a block's lines (71,216 bytes for two columns of 4050 points)
 constexpr int MX_PY_MAXB = 32;              // most positions of a batch
 // bytes of scratch planes that a batch aims at (at least one plane): the
 // rows' mask and PSF reads and the sum's update are shared by a batch (784^2:
@@ -381,7 +382,7 @@ int py_pass(mx_pywfs_t *h, int mode, PyArgs a, int nlines) {
     a.nlines = nlines;
     const int many = mode == PY_MOD ? a.npos : mode == PY_ACC ? a.nsplit : 1;
     const dim3 grid((unsigned)((nlines + a.L - 1) / a.L * many)), block((unsigned)lx_threads(a.plan, a.L));
-    const size_t lds = sizeof(float2) * (size_t)a.L * a.plan.S;
+    const size_t lds = sizeof(float2) * (size_t)a.L * a.plan.S; // (at most MX_PY_LDS)
     switch (mode) {
     case PY_EMBED: k_py_rows<PY_EMBED><<<grid, block, lds, h->stream>>>(a); break;
     case PY_PSF: k_py_cols<PY_PSF><<<grid, block, lds, h->stream>>>(a); break;
@@ -570,8 +571,9 @@ int mx_pywfs_init(mx_pywfs_t **out, const mx_pywfs_cfg_t *c) {
     h->plan = plan;
     PYCHK(hipSetDevice(h->device));
     {
-        // the lines of a block may exceed the default dynamic LDS limit
-        const int lds = (int)(sizeof(float2) * plan.S * (size_t)std::max(py_row_lines(n), py_col_lines(n)));
+        // the lines of a block may exceed the default dynamic LDS limit; the
+        // limit belongs to the kernel, not to this handle, so it is the one that
+        // every grid side fits
         const void *k[] = {reinterpret_cast<const void *>(&k_py_rows<PY_EMBED>),
                            reinterpret_cast<const void *>(&k_py_cols<PY_PSF>),
                            reinterpret_cast<const void *>(&k_py_rows<PY_MOD>),
@@ -579,7 +581,7 @@ int mx_pywfs_init(mx_pywfs_t **out, const mx_pywfs_cfg_t *c) {
                            reinterpret_cast<const void *>(&k_py_rows<PY_REAL>),
                            reinterpret_cast<const void *>(&k_py_cols<PY_DTF>),
                            reinterpret_cast<const void *>(&k_py_rows<PY_IMG>)};
-        for (const void *f : k) PYCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        for (const void *f : k) PYCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, MX_PY_LDS));
     }
     PYCHK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
     PYCHK(hipEventCreate(&h->ev[0]));
