@@ -404,24 +404,27 @@ __device__ __forceinline__ void axis_map(const DevLayer &L, bool isx, double ihs
     dout = ptsdx * d1 * scale;
     oout = orig * d1 * scale + (disp - o0) * d1;
 }
-__device__ __forceinline__ void screen_wrap(const DevLayer &L, bool isx, double i, double dout, double oout, int &ii,
-                                            float &ff) {
-    const double nn = (double)(isx ? L.nx : L.ny);
+// (n, in: the axis's length and its inverse)
+__device__ __forceinline__ void axis_wrap(int n, double in, double i, double dout, double oout, int &ii, float &ff) {
+    const double nn = (double)n;
     double X = fma(i, dout, oout);
-    const double q = X * (isx ? L.inx : L.iny);
+    const double q = X * in;
     double fq = floor(q);
     if (q - fq < 1e-9 || q - fq > 1. - 1e-9) fq = floor(X / nn);
     X -= fq * nn;
     const double fl = floor(X);
     ii = (int)fl;
     double fr = X - fl;
-    const int n = isx ? L.nx : L.ny;
     if (ii >= n) ii -= n;
     if (ii < 0) {
         ii += n;
         fr = 0.;
     }
     ff = (float)fr;
+}
+__device__ __forceinline__ void screen_wrap(const DevLayer &L, bool isx, double i, double dout, double oout, int &ii,
+                                            float &ff) {
+    axis_wrap(isx ? L.nx : L.ny, isx ? L.inx : L.iny, i, dout, oout, ii, ff);
 }
 __device__ __forceinline__ void screen_coord(const DevLayer &L, bool isx, int i, double ihs, double theta,
                                              double misreg, double shift0, long isim, double dt,
@@ -1057,17 +1060,112 @@ __global__ __launch_bounds__(64) void k_dm_opd(DmArgs a) {
     }
 }
 
+// ------------------------------------------------------------ gathers
+// acc plus the bilinear values of layers l0 .. l0 + G - 1 (periodic) at one
+// point; at(u, L, c, fx, r, fy) gives its column, row and fractions on layer l0 +
+// u.  The loads of the G layers are issued together; a layer above the source
+// (at range hs, 0: at infinity) is loaded and not added.
+template <int G, class AT>
+__device__ __forceinline__ float add_layers(const DevLayer *layers, double hs, int l0, float acc, AT &&at) {
+    float fx[G], fy[G], q[G][4];
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+        const DevLayer &L = layers[l0 + u];
+        int c0, r0;
+        at(u, L, c0, fx[u], r0, fy[u]);
+        const int c1 = c0 + 1 == L.nx ? 0 : c0 + 1, r1 = r0 + 1 == L.ny ? 0 : r0 + 1;
+        const float *p0 = L.p + (long)r0 * L.nx, *p1 = L.p + (long)r1 * L.nx;
+        q[u][0] = p0[c0];
+        q[u][1] = p0[c1];
+        q[u][2] = p1[c0];
+        q[u][3] = p1[c1];
+    }
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+        if (hs != 0. && layers[l0 + u].ht > hs) continue; // uniform
+        const float v0 = fmaf(fx[u], q[u][1] - q[u][0], q[u][0]), v1 = fmaf(fx[u], q[u][3] - q[u][2], q[u][2]);
+        acc += fmaf(fy[u], v1 - v0, v0);
+    }
+    return acc;
+}
+
 // ------------------------------------------------------------ coarse grids
 // OPD of grids coarser than a screen (the low-order NGS grids at 1/16 m over
 // 1/64 m screens, or a screen under 40 pixels), whose screen footprint the
-// staged tiles of k_wfs_opd do not hold: one point per thread gathers its
-// four neighbours from every layer, and the DM surfaces and the OPD inputs
-// are applied before the one store.  Bound by the latency of the gathers, so
-// the chip is filled with points (900 blocks for one 480^2 grid) and four
-// layers' gathers are in flight per lane; the grid-uniform FP64 maps are
-// formed once per block.  One wave per 32^2 or 16^2 tile with one layer after
-// another, as the staged form has it, left most of the chip idle: 77 us for
-// the 480^2 tip-tilt grid and seven layers, whose step fell from 191 to 120 us.
+// staged tiles of k_wfs_opd do not hold: a point gathers its four neighbours
+// from every layer, and the DM surfaces and the OPD inputs are applied before
+// the one store.  Two forms with the same numbers (opd_points decides):
+//  - k_wfs_opd_pt, one point per thread, four layers' gathers in flight, the
+//    grid-uniform FP64 maps formed once per block.  It fills the chip with the
+//    points of few grids (900 blocks for one 480^2 grid) and is bound by the
+//    latency of the gathers there, by its FP64 coordinates (two per point and
+//    layer) on many.
+//  - k_wfs_opd_tile, one wave per tile of NX^2 points, NX^2 / 64 consecutive
+//    rows of a column per lane, the FP64 coordinates once per column and row of
+//    the tile; 64 gathers of a lane in flight (one layer at 16 points, four at
+//    4).  Bound by the gathers' rate on many grids: 17,000 of 32^2 points and
+//    one layer take 45 us (0.39 Gpoint/ms), 119 one point per thread.
+struct CoarseGrid { // one WFS's subaperture (or LLT) grid of n^2 points
+    int iwfs, isa, n;
+    bool llt;
+    double x0, y0, ihs;              // first point; 1 / range (0: at infinity)
+    double tx, ty, mx, my, sx, sy;   // direction, misregistration, shift
+};
+__device__ __forceinline__ void coarse_init(const OpdArgs &a, const DevWfs &W, CoarseGrid &g) {
+    g.ihs = W.hs != 0. ? 1. / W.hs : 0.;
+    g.tx = W.thetax;
+    g.ty = W.thetay;
+    if (g.llt) {
+        g.x0 = a.llt_origx;
+        g.y0 = a.llt_origy;
+        g.tx -= a.llt_ox / W.hs;
+        g.ty -= a.llt_oy / W.hs;
+        g.mx = g.my = 0.;
+        g.sx = a.llt_ox;
+        g.sy = a.llt_oy;
+    } else {
+        g.x0 = a.ptsx[g.isa];
+        g.y0 = a.ptsy[g.isa];
+        g.mx = W.misregx;
+        g.my = W.misregy;
+        g.sx = g.sy = 0.;
+    }
+}
+// map of axis ax of layer L for that grid, from its first point
+__device__ __forceinline__ void coarse_map(const OpdArgs &a, const CoarseGrid &g, const DevLayer &L, bool ax,
+                                           double &dout, double &oout) {
+    axis_map(L, ax, g.ihs, ax ? g.tx : g.ty, ax ? g.mx : g.my, ax ? g.sx : g.sy, a.isim, a.dt, a.ptsdx, ax ? g.x0 : g.y0,
+             dout, oout);
+}
+// the traced values of P points (ix, iy ..), scaled, with the DM surfaces and
+// inputs, to their places
+template <int P>
+__device__ __forceinline__ void coarse_store(const OpdArgs &a, const DevWfs &W, const CoarseGrid &g, const DmMap *dmap,
+                                             float atmscale, float (&v)[P], int ix, int iy) {
+#pragma unroll
+    for (int j = 0; j < P; j++) v[j] *= atmscale;
+    const int pt = iy * g.n + ix;
+    float *out;
+    if (g.llt) {
+        out = a.llt_opd + (long)g.iwfs * g.n * g.n + pt;
+    } else {
+        const long first = (long)g.isa * g.n * g.n;
+        out = a.opd + (long)g.iwfs * a.nsa * g.n * g.n + first + pt;
+        for (int d = 0; d < a.ndm; d++) {
+            const DevLayer &L = a.dms[W.ireal * MX_MAXDM + d];
+            if (W.hs != 0. && L.ht > W.hs) continue;
+#pragma unroll
+            for (int j = 0; j < P; j++) v[j] = dm_sub(L, dmap[d], v[j], ix, iy + j);
+        }
+        if (a.opdadd || a.ptt) {
+            const OpdIn in = opd_in(a.opdadd, a.opdadd_ws, a.ptt, g.iwfs, first, g.x0, g.y0, a.ptsdx);
+#pragma unroll
+            for (int j = 0; j < P; j++) v[j] = opd_add(in, v[j], ix, iy + j, pt + j * g.n);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < P; j++) out[j * g.n] = v[j];
+}
 constexpr int MX_OPD_PT_THREADS = 256;
 // blocks of one grid of side n
 constexpr int pt_blocks(int n) { return (n * n + MX_OPD_PT_THREADS - 1) / MX_OPD_PT_THREADS; }
@@ -1076,73 +1174,147 @@ __global__ __launch_bounds__(MX_OPD_PT_THREADS) void k_wfs_opd_pt(OpdArgs a) {
     __shared__ double map[MX_MAXLAYER][4]; // x step, x origin, y step, y origin of each traced layer
     __shared__ DmMap dmap[MX_MAXDM];
     const int b = (int)blockIdx.x, tid = (int)threadIdx.x;
-    const bool llt = b < a.nllt; // the LLT uplink grids come first
-    const int n = llt ? a.llt_side : a.nxsa, nb = pt_blocks(n);
-    int iwfs, isa = 0, blk;
-    if (llt) {
-        iwfs = b / nb;
+    CoarseGrid g;
+    g.llt = b < a.nllt; // the LLT uplink grids come first
+    g.n = g.llt ? a.llt_side : a.nxsa;
+    g.isa = 0;
+    const int nb = pt_blocks(g.n);
+    int blk;
+    if (g.llt) {
+        g.iwfs = b / nb;
         blk = b % nb;
     } else {
         const int unit = xcd_unit(b - a.nllt, a.nsa * a.nwfs * nb), rest = unit / a.nwfs;
-        iwfs = unit % a.nwfs;
-        isa = rest / nb;
+        g.iwfs = unit % a.nwfs;
+        g.isa = rest / nb;
         blk = rest % nb;
     }
-    const DevWfs &W = a.wfs[iwfs];
+    const DevWfs &W = a.wfs[g.iwfs];
     const DevLayer *layers = a.layers + W.ireal * MX_MAXLAYER;
-    const double ihs = W.hs != 0. ? 1. / W.hs : 0.;
-    const double x0 = llt ? a.llt_origx : a.ptsx[isa], y0 = llt ? a.llt_origy : a.ptsy[isa];
+    coarse_init(a, W, g);
+    const float sc = (float)a.atmscale[W.ireal]; // (here: its load is waited for with the others)
     if (tid < 2 * a.nps) {
-        const DevLayer &L = layers[tid >> 1];
         const bool ax = (tid & 1) == 0;
-        const double th = ax ? W.thetax : W.thetay, lo = ax ? a.llt_ox : a.llt_oy;
-        axis_map(L, ax, ihs, llt ? th - lo / W.hs : th, llt ? 0. : (ax ? W.misregx : W.misregy), llt ? lo : 0., a.isim,
-                 a.dt, a.ptsdx, ax ? x0 : y0, map[tid >> 1][ax ? 0 : 2], map[tid >> 1][ax ? 1 : 3]);
+        coarse_map(a, g, layers[tid >> 1], ax, map[tid >> 1][ax ? 0 : 2], map[tid >> 1][ax ? 1 : 3]);
     }
-    const int ndm = llt ? 0 : a.ndm;
-    if (tid >= 64 && tid < 64 + ndm) dmap[tid - 64] = dm_map(a.dms[W.ireal * MX_MAXDM + tid - 64], W, a.ptsdx, x0, y0);
+    if (tid >= 64 && tid < 64 + a.ndm)
+        dmap[tid - 64] = dm_map(a.dms[W.ireal * MX_MAXDM + tid - 64], W, a.ptsdx, g.x0, g.y0);
     __syncthreads();
     const int pt = blk * MX_OPD_PT_THREADS + tid;
-    if (pt >= n * n) return;
-    const int ix = pt % n, iy = pt / n;
-    float acc = 0.f;
+    if (pt >= g.n * g.n) return;
+    const int iy = (int)((unsigned)pt / (unsigned)g.n), ix = pt - iy * g.n;
+    float acc[1] = {0.f};
     for (int l0 = 0; l0 < a.nps; l0 += G) {
-        float fx[G], fy[G], q[G][4];
-#pragma unroll
-        for (int u = 0; u < G; u++) {
-            const int l = min(l0 + u, a.nps - 1); // (past the last layer: its loads again, not used)
-            const DevLayer &L = layers[l];
-            int c0, r0;
-            screen_wrap(L, true, ix, map[l][0], map[l][1], c0, fx[u]);
-            screen_wrap(L, false, iy, map[l][2], map[l][3], r0, fy[u]);
-            const int c1 = c0 + 1 == L.nx ? 0 : c0 + 1, r1 = r0 + 1 == L.ny ? 0 : r0 + 1;
-            const float *p0 = L.p + (long)r0 * L.nx, *p1 = L.p + (long)r1 * L.nx;
-            q[u][0] = p0[c0];
-            q[u][1] = p0[c1];
-            q[u][2] = p1[c0];
-            q[u][3] = p1[c1];
-        }
-#pragma unroll
-        for (int u = 0; u < G; u++) {
-            if (l0 + u >= a.nps || (W.hs != 0. && layers[l0 + u].ht > W.hs)) continue; // uniform; layers above the source
-            const float r0 = fmaf(fx[u], q[u][1] - q[u][0], q[u][0]), r1 = fmaf(fx[u], q[u][3] - q[u][2], q[u][2]);
-            acc += fmaf(fy[u], r1 - r0, r0);
+        auto at = [&](int u, const DevLayer &L, int &c, float &fx, int &r, float &fy) {
+            const double *m = map[l0 + u];
+            screen_wrap(L, true, ix, m[0], m[1], c, fx);
+            screen_wrap(L, false, iy, m[2], m[3], r, fy);
+        };
+        switch (a.nps - l0) {
+        case 1: acc[0] = add_layers<1>(layers, W.hs, l0, acc[0], at); break;
+        case 2: acc[0] = add_layers<2>(layers, W.hs, l0, acc[0], at); break;
+        case 3: acc[0] = add_layers<3>(layers, W.hs, l0, acc[0], at); break;
+        default: acc[0] = add_layers<G>(layers, W.hs, l0, acc[0], at); break;
         }
     }
-    float v = (float)a.atmscale[W.ireal] * acc;
-    const long first = (long)isa * n * n;
-    if (llt) {
-        a.llt_opd[(long)iwfs * n * n + pt] = v;
-        return;
-    }
-    for (int d = 0; d < ndm; d++) {
-        const DevLayer &L = a.dms[W.ireal * MX_MAXDM + d];
-        if (W.hs != 0. && L.ht > W.hs) continue;
-        v = dm_sub(L, dmap[d], v, ix, iy);
-    }
-    v = opd_add(opd_in(a.opdadd, a.opdadd_ws, a.ptt, iwfs, first, x0, y0, a.ptsdx), v, ix, iy, pt);
-    a.opd[((long)iwfs * a.nsa) * n * n + first + pt] = v;
+    coarse_store(a, W, g, dmap, sc, acc, ix, iy);
 }
+
+// (four waves a SIMD, which the tables' LDS allows: the loads of 16 points in
+// flight; ONE: a grid is one tile, and the wave is short of instructions to
+// spend on finding its tile)
+template <int NX, bool ONE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_wfs_opd_tile(OpdArgs a) {
+    constexpr int PPT = NX * NX / 64, G = 16 / PPT; // points of a lane; layers in flight
+    __shared__ double map[MX_MAXLAYER][2][3]; // of each layer's axes: step, origin, 1 / length
+    __shared__ int len[MX_MAXLAYER][2];
+    __shared__ DmMap dmap[MX_MAXDM];
+    __shared__ int cell[MX_MAXLAYER][2 * NX]; // the tile's columns, then its rows
+    __shared__ float frac[MX_MAXLAYER][2 * NX];
+    const int b = (int)blockIdx.x, line = (int)threadIdx.x;
+    CoarseGrid g;
+    g.llt = b < a.nllt; // the LLT uplink grids come first
+    g.isa = 0;
+    const int tiles = ONE ? 1 : g.llt ? a.llt_tiles : a.tiles, T2 = tiles * tiles;
+    g.n = tiles * NX;
+    int it;
+    if (g.llt) {
+        g.iwfs = b / T2;
+        it = b % T2;
+    } else {
+        const int unit = xcd_unit(b - a.nllt, a.nsa * a.nwfs * T2), rest = unit / a.nwfs;
+        g.iwfs = unit % a.nwfs;
+        g.isa = rest / T2;
+        it = rest % T2;
+    }
+    const DevWfs &W = a.wfs[g.iwfs];
+    const DevLayer *layers = a.layers + W.ireal * MX_MAXLAYER;
+    coarse_init(a, W, g);
+    const float sc = (float)a.atmscale[W.ireal]; // (here: its load is waited for with the others)
+    if (line >= 64 - a.ndm)
+        dmap[63 - line] = dm_map(a.dms[W.ireal * MX_MAXDM + 63 - line], W, a.ptsdx, g.x0, g.y0);
+    if (line < 2 * a.nps) {
+        const bool ax = (line & 1) == 0;
+        const DevLayer &L = layers[line >> 1];
+        double *m = map[line >> 1][line & 1];
+        coarse_map(a, g, L, ax, m[0], m[1]);
+        m[2] = ax ? L.inx : L.iny;
+        len[line >> 1][line & 1] = ax ? L.nx : L.ny;
+    }
+    __syncthreads();
+    const int cx = NX * (it % tiles), cy = NX * (it / tiles), ix = line % NX, jb = line / NX * PPT;
+    for (int e = line; e < 2 * NX * a.nps; e += 64) {
+        const int l = e / (2 * NX), k = e % (2 * NX), ay = k / NX;
+        const double *m = map[l][ay];
+        axis_wrap(len[l][ay], m[2], ay ? cy + k - NX : cx + k, m[0], m[1], cell[l][k], frac[l][k]);
+    }
+    __syncthreads();
+    float acc[PPT];
+#pragma unroll
+    for (int j = 0; j < PPT; j++) acc[j] = 0.f;
+    if constexpr (G == 1) {
+        for (int l = 0; l < a.nps; l++) {
+            const DevLayer L = layers[l];
+            if (W.hs != 0. && L.ht > W.hs) continue; // uniform: a layer above the source
+            const int c0 = cell[l][ix], c1 = c0 + 1 == L.nx ? 0 : c0 + 1;
+            const float fx = frac[l][ix];
+#pragma unroll
+            for (int j = 0; j < PPT; j++) {
+                const int r0 = cell[l][NX + jb + j], r1 = r0 + 1 == L.ny ? 0 : r0 + 1;
+                const float *p0 = L.p + (long)r0 * L.nx, *p1 = L.p + (long)r1 * L.nx;
+                const float v0 = fmaf(fx, p0[c1] - p0[c0], p0[c0]), v1 = fmaf(fx, p1[c1] - p1[c0], p1[c0]);
+                acc[j] += fmaf(frac[l][NX + jb + j], v1 - v0, v0);
+            }
+        }
+    } else {
+        for (int l0 = 0; l0 < a.nps; l0 += G) {
+            auto layers_at = [&](auto N) {
+#pragma unroll
+                for (int j = 0; j < PPT; j++)
+                    acc[j] = add_layers<decltype(N)::value>(
+                        layers, W.hs, l0, acc[j], [&](int u, const DevLayer &, int &c, float &fx, int &r, float &fy) {
+                            c = cell[l0 + u][ix];
+                            fx = frac[l0 + u][ix];
+                            r = cell[l0 + u][NX + jb + j];
+                            fy = frac[l0 + u][NX + jb + j];
+                        });
+            };
+            switch (a.nps - l0) {
+            case 1: layers_at(std::integral_constant<int, 1>{}); break;
+            case 2: layers_at(std::integral_constant<int, 2>{}); break;
+            case 3: layers_at(std::integral_constant<int, 3>{}); break;
+            default: layers_at(std::integral_constant<int, G>{}); break;
+            }
+        }
+    }
+    coarse_store(a, W, g, dmap, sc, acc, cx + ix, cy + jb);
+}
+// The coarse grids go one point per thread: fewer tiles than four waves a CU.
+// Trace in us, points / tiles, 1 and 7 layers: 52 tiles of 32^2 6.1 / 6.2 and
+// 7.7 / 13, 675 (three 480^2 grids) 12 / 11 and 25 / 29, 1,200 14 / 8.7 and 29 /
+// 26, 17,000 119 / 45 and 282 / 221; 800 of 16^2 6.4 / 6.2 and 9.9 / 10, 3,400
+// 11 / 8.1 and 22 / 20.
+constexpr bool opd_points(long tiles) { return tiles < 1024; }
 
 // ------------------------------------------------------------ dither fold
 // At each PLL output of the TT dither (maos/wfsgrad.c:709-731): the folded
@@ -4096,7 +4268,8 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
     o.tiles = (int)(h->nxsa / opd_nx);
     o.llt_tiles = (int)((h->cfg.llt_nx + opd_nx - 1) / opd_nx);
     o.llt_side = o.llt_tiles * opd_nx;
-    const int llt_blocks = direct ? pt_blocks(o.llt_side) : o.llt_tiles * o.llt_tiles; // per LLT grid
+    const bool points = direct && opd_points(h->nsa * h->nwfs * o.tiles * o.tiles);
+    const int llt_blocks = points ? pt_blocks(o.llt_side) : o.llt_tiles * o.llt_tiles; // per LLT grid
     o.nllt = llt ? h->nwfs * llt_blocks : 0;
     KArgs &a = h->arg_step;
     a = KArgs{};
@@ -4256,7 +4429,12 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
     const void *kopd_t[2][2] = {
         {reinterpret_cast<const void *>(&k_wfs_opd<16, false>), reinterpret_cast<const void *>(&k_wfs_opd<16, true>)},
         {reinterpret_cast<const void *>(&k_wfs_opd<32, false>), reinterpret_cast<const void *>(&k_wfs_opd<32, true>)}};
-    const void *kopd = direct ? reinterpret_cast<const void *>(&k_wfs_opd_pt) : kopd_t[opd_nx == 32][o.tiles > 1];
+    const void *kcoarse_t[2][2] = {
+        {reinterpret_cast<const void *>(&k_wfs_opd_tile<16, true>), reinterpret_cast<const void *>(&k_wfs_opd_tile<16, false>)},
+        {reinterpret_cast<const void *>(&k_wfs_opd_tile<32, true>), reinterpret_cast<const void *>(&k_wfs_opd_tile<32, false>)}};
+    const void *kopd = points             ? reinterpret_cast<const void *>(&k_wfs_opd_pt)
+                       : direct ? kcoarse_t[opd_nx == 32][o.tiles > 1 || o.llt_tiles > 1]
+                                : kopd_t[opd_nx == 32][o.tiles > 1];
     // MX_FUSED=1 in the environment: the MFMA imaging and uplink kernels trace
     // their own grids (no ray-trace launch, the OPD staged in LDS), for the
     // MFMA forms on the 32-point grid without DM surfaces or OPD inputs.
@@ -4274,9 +4452,9 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
         m.opd_out = h->d_opd;
         m.llt_opd_out = h->d_llt_opd;
     } else {
-        const long nblk = direct ? pt_blocks((int)h->nxsa) : o.tiles * o.tiles; // per subaperture grid
+        const long nblk = points ? pt_blocks((int)h->nxsa) : o.tiles * o.tiles; // per subaperture grid
         L[nl++] = {kopd, dim3((unsigned)(h->nsa * h->nwfs * nblk + o.nllt)),
-                   dim3(direct ? MX_OPD_PT_THREADS : MX_OPD_THREADS), &o};
+                   dim3(points ? MX_OPD_PT_THREADS : MX_OPD_THREADS), &o};
     }
     if (ndm > 0 && !direct) {
         DmArgs &dm = h->arg_dm;
@@ -4585,7 +4763,7 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
         q.isim = isim + 1;
         q.llt_opd = h->d_llt_opd2;
         q.nllt = h->nwfs * llt_blocks;
-        L[nl] = {kopd, dim3((unsigned)q.nllt), dim3(direct ? MX_OPD_PT_THREADS : MX_OPD_THREADS), &q};
+        L[nl] = {kopd, dim3((unsigned)q.nllt), dim3(points ? MX_OPD_PT_THREADS : MX_OPD_THREADS), &q};
         L[nl++].dep = -1;
         if (uplink_direct) {
             LltAcorrArgs &u = h->arg_lltac_pre;
