@@ -475,9 +475,11 @@ __global__ __launch_bounds__(256) void k_evl_ptt_fin(const double *part, double 
 // (alpha = -1, no wrap; a point outside a surface takes nothing from it).
 // The screen map is the one of the WFS ray trace, a point's coordinate in
 // place of its index, its uniform part formed once per block.  Bound by the
-// screens' reads and the latency of the gathers: four layers' are in flight,
-// and neighbouring blocks share an XCD, so that the screen rows that two rows
-// of points read come from one L2.
+// screens' reads and the latency of the gathers: four layers' are in flight (no
+// more than there are: a remainder of one layer made one of 2.85 M points and
+// one layer 29 us, now 20, and one of seven 52, now 47), and neighbouring blocks
+// share an XCD, so that the screen rows that two rows of points read come from
+// one L2.
 struct EvlOpdArgs {
     const DevLayer *layers; // [MX_MAXLAYER]
     const DevLayer *dms;    // [MX_MAXDM]
@@ -506,26 +508,16 @@ __global__ __launch_bounds__(256) void k_evl_opd(EvlOpdArgs a) {
     const double x = a.locx[i], y = a.locy[i];
     float sum = 0.f;
     for (int l0 = 0; l0 < a.nps; l0 += G) {
-        float fx[G], fy[G], q[G][4];
-#pragma unroll
-        for (int u = 0; u < G; u++) {
-            const int l = min(l0 + u, a.nps - 1); // (past the last layer: its loads again, not used)
-            const DevLayer &L = a.layers[l];
-            int ix, iy;
-            screen_wrap(L, true, x, map[l][0], map[l][1], ix, fx[u]);
-            screen_wrap(L, false, y, map[l][2], map[l][3], iy, fy[u]);
-            const int ix1 = ix + 1 == L.nx ? 0 : ix + 1, iy1 = iy + 1 == L.ny ? 0 : iy + 1;
-            const float *r0 = L.p + (long)iy * L.nx, *r1 = L.p + (long)iy1 * L.nx;
-            q[u][0] = r0[ix];
-            q[u][1] = r0[ix1];
-            q[u][2] = r1[ix];
-            q[u][3] = r1[ix1];
-        }
-#pragma unroll
-        for (int u = 0; u < G; u++) {
-            if (l0 + u >= a.nps || (hs != 0. && a.layers[l0 + u].ht > hs)) continue; // uniform
-            const float v0 = fmaf(fx[u], q[u][1] - q[u][0], q[u][0]), v1 = fmaf(fx[u], q[u][3] - q[u][2], q[u][2]);
-            sum += fmaf(fy[u], v1 - v0, v0);
+        auto at = [&](int u, const DevLayer &L, int &c, float &fx, int &r, float &fy) {
+            const double *m = map[l0 + u];
+            screen_wrap(L, true, x, m[0], m[1], c, fx);
+            screen_wrap(L, false, y, m[2], m[3], r, fy);
+        };
+        switch (a.nps - l0) {
+        case 1: sum = add_layers<1>(a.layers, hs, l0, sum, at); break;
+        case 2: sum = add_layers<2>(a.layers, hs, l0, sum, at); break;
+        case 3: sum = add_layers<3>(a.layers, hs, l0, sum, at); break;
+        default: sum = add_layers<G>(a.layers, hs, l0, sum, at); break;
         }
     }
     float v = (float)((double)sum * a.atmscale);
