@@ -586,7 +586,10 @@ struct mx_evl_s {
     double imcc[9] = {}, ipcc = 0;               // inverse of sum amp [1 x y]^T [1 x y], 1 / sum amp
     float2 *d_B = nullptr;
     size_t b_len = 0; // its elements
-    double *d_out = nullptr; // PSF rows on their way to the host, [out_len]
+    // PSF rows and p/t/t sums on their way to the host, one read-out at a time:
+    // several threads may read a handle that no call steps
+    std::mutex out_mx;
+    double *d_out = nullptr; // [out_len]
     long out_len = 0;
     EvlWvl w[MX_MAXWVL];
     long nacc = 0;
@@ -952,6 +955,7 @@ int mx_evl_wfe(mx_evl_t *h, double *rms, double *coeff) {
     if (!h || (!rms && !coeff)) return set_err(MX_EINVAL, "mx_evl_wfe: null argument");
     if (!h->d_ptt) return set_err(MX_ESTATE, "mx_evl_wfe: the handle was made without point coordinates");
     HIPCHK(hipSetDevice(h->device));
+    std::lock_guard<std::mutex> lock(h->out_mx);
     const int np = ptt_parts(h->nloc, h->ndir);
     PttArgs a{h->d_opd, h->d_amp64, h->d_locx, h->d_locy, h->d_ptt, h->nloc, np};
     k_evl_ptt<<<dim3((unsigned)np, (unsigned)h->ndir), dim3(256), 0, h->stream>>>(a);
@@ -1003,6 +1007,7 @@ int mx_evl_psf_get(mx_evl_t *h, int idir, int iwvl, double *psf, long *nacc) {
         return MX_OK;
     }
     // strips of rows through the handle's output buffer
+    std::lock_guard<std::mutex> lock(h->out_mx);
     const long P = w.P, rows = std::min(P, std::max(1L, MX_PSF_OUT / P));
     if (const int rc = dev_alloc(&h->d_out, (size_t)h->out_len)) return rc;
     for (long y0 = 0; y0 < P; y0 += rows) {
