@@ -330,6 +330,11 @@ struct PsfOutArgs {
     double sc;
 };
 constexpr long MX_PSF_OUT = 1L << 21; // most values of one strip (16 MB, kept by the handle)
+// Most values of a window that the kernel writes to pinned host memory (2 MB,
+// kept by the handle): a copy to pageable memory costs some 15 us however
+// small.  In us with the copy / pinned: 32^2 28 / 16, 128^2 32 / 21, 250^2 50 /
+// 41, 512^2 180 / 154, 724^2 305 / 305.
+constexpr long MX_PSF_PIN = 1L << 18;
 __global__ __launch_bounds__(256) void k_psf_out(PsfOutArgs a) {
     __shared__ float t[32][33];
     const int x0 = (int)blockIdx.x * 32, r0 = (int)blockIdx.y * 32, tx = threadIdx.x % 32, ty = threadIdx.x / 32;
@@ -591,6 +596,8 @@ struct mx_evl_s {
     std::mutex out_mx;
     double *d_out = nullptr; // [out_len]
     long out_len = 0;
+    double *h_out = nullptr; // pinned [pin_len], for the windows of at most MX_PSF_PIN values
+    long pin_len = 0;
     EvlWvl w[MX_MAXWVL];
     long nacc = 0;
     int ireal = 0; // realisation whose screens and DM surfaces mx_evl_trace reads
@@ -654,6 +661,7 @@ void evl_release(mx_evl_t *h) {
             if (p) hipFree(p);
     }
     if (h->h_tot) hipHostFree(h->h_tot);
+    if (h->h_out) hipHostFree(h->h_out);
     for (hipEvent_t e : h->ev)
         if (e) hipEventDestroy(e);
     if (h->stream) hipStreamDestroy(h->stream);
@@ -864,11 +872,14 @@ int mx_evl_init(mx_evl_t **out, long nloc, const double *locx, const double *loc
         EVCHK(hipMemset(w.d_acc, 0, sizeof(float) * ndir * w.P * w.P));
         bmax = std::max(bmax, (size_t)ndir * w.nband * w.P);
         bsum += (size_t)ndir * w.nband * w.P;
-        h->out_len = std::max(h->out_len, std::min((long)w.P * w.P, std::max((long)w.P, MX_PSF_OUT)));
+        const long np2 = (long)w.P * w.P;
+        if (np2 <= MX_PSF_PIN) h->pin_len = std::max(h->pin_len, np2);
+        else h->out_len = std::max(h->out_len, std::min(np2, std::max((long)w.P, MX_PSF_OUT)));
     }
     // the row passes' output of every wavelength, up to 256 MB of it (at least one's)
     h->b_len = std::max(bmax, std::min(bsum, (size_t)(256 << 20) / sizeof(float2)));
     if (bmax && (rc = dev_alloc(&h->d_B, h->b_len))) return fail(rc);
+    if (h->pin_len) EVCHK(hipHostMalloc((void **)&h->h_out, sizeof(double) * h->pin_len));
     EVCHK(hipDeviceSynchronize());
     *out = h;
     return MX_OK;
@@ -1009,10 +1020,20 @@ int mx_evl_psf_get(mx_evl_t *h, int idir, int iwvl, double *psf, long *nacc) {
     // strips of rows through the handle's output buffer
     std::lock_guard<std::mutex> lock(h->out_mx);
     const long P = w.P, rows = std::min(P, std::max(1L, MX_PSF_OUT / P));
+    const float *acc = w.d_acc + (size_t)idir * P * P;
+    if (P * P <= MX_PSF_PIN) {
+        PsfOutArgs a{acc, h->h_out, (int)P, 0, (int)P, sc};
+        const unsigned nt = (unsigned)((P + 31) / 32);
+        k_psf_out<<<dim3(nt, nt), dim3(256), 0, h->stream>>>(a);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(h->stream));
+        std::memcpy(psf, h->h_out, sizeof(double) * P * P);
+        return MX_OK;
+    }
     if (const int rc = dev_alloc(&h->d_out, (size_t)h->out_len)) return rc;
     for (long y0 = 0; y0 < P; y0 += rows) {
         const long ny = std::min(rows, P - y0);
-        PsfOutArgs a{w.d_acc + (size_t)idir * P * P, h->d_out, (int)P, (int)y0, (int)ny, sc};
+        PsfOutArgs a{acc, h->d_out, (int)P, (int)y0, (int)ny, sc};
         k_psf_out<<<dim3((unsigned)((P + 31) / 32), (unsigned)((ny + 31) / 32)), dim3(256), 0, h->stream>>>(a);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(psf + y0 * P, h->d_out, sizeof(double) * ny * P, hipMemcpyDeviceToHost, h->stream));

@@ -14,9 +14,11 @@ def _points(n):
     return X[m].copy(), Y[m].copy()
 
 
-# P = 2 and 34: less than a tile and its remainder; 1448: the widest window of
-# one strip (1448^2 < 2^21); 1450: the first of two; 2050: three, the last short
-@pytest.mark.parametrize("N,P", [(64, 2), (64, 34), (2048, 1448), (2048, 1450), (4096, 2050)])
+# P = 2 and 34: less than a tile and its remainder; 512: the widest window that
+# is written to host memory (2^18 values), 514 the first that is copied; 1448: the
+# widest of one strip (1448^2 < 2^21); 1450: the first of two; 2050: three, the
+# last short
+@pytest.mark.parametrize("N,P", [(64, 2), (64, 34), (512, 512), (1024, 514), (2048, 1448), (2048, 1450), (4096, 2050)])
 def test_psf_readout_strips(N, P):
     from maos_amd import engine
     x, y = _points(25)
