@@ -14,11 +14,12 @@ INTS_TOL = 2e-5  # the parity bars of the forms
 GRAD_TOL_MAS = 0.1
 
 
-# nxsa, embfac, notf: 16 -> 48 = 12 4 or 6 8; 70 = 10 7; 80 = 10 8; 84 = 12 7;
-# 96 in 210 (7); 96 in 250 (5 5 10) and 256 (columns of 129 points, the longest
-# of the staged sums); 128 in 270 = 18 .. (columns of 136,
-# summed by waves); 432 in 486 = 2 3^5; 480 in 1000 (10 10 10); 448 = 64 7
-@pytest.mark.parametrize("nxsa,embfac,notf", [(16, 3, 48), (16, 3, 70), (16, 5, 84), (48, 2, 210), (48, 2, 250),
+# nxsa, embfac, notf: 16 = 4 4 and 18 = 6 3 (one radix, split); 48 = 8 6; 70 = 10 7;
+# 80 = 16 5; 84 = 12 7; 96 = 16 6 in 210 = 7 6 5, in 250 = 10 5 5 and in 256 = 16 16
+# (columns of 129 points, the longest of the staged sums); 128 = 16 8 in 270 = 9 6 5
+# (columns of 136, summed by waves); 432 = 9 8 6 in 486 = 9 9 6; 480 = 16 6 5 in
+# 1000 = 10 10 10; 448 = 8 8 7
+@pytest.mark.parametrize("nxsa,embfac,notf", [(16, 1, 16), (16, 1, 18), (16, 3, 48), (16, 3, 70), (16, 5, 84), (48, 2, 210), (48, 2, 250),
                                               (48, 2, 256), (64, 2, 270), (144, 3, 486), (240, 2, 1000),
                                               (224, 2, 448)])
 @pytest.mark.parametrize("nwvl", [1, 2])
