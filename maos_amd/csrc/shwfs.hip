@@ -426,14 +426,6 @@ __device__ __forceinline__ void screen_wrap(const DevLayer &L, bool isx, double 
                                             float &ff) {
     axis_wrap(isx ? L.nx : L.ny, isx ? L.inx : L.iny, i, dout, oout, ii, ff);
 }
-__device__ __forceinline__ void screen_coord(const DevLayer &L, bool isx, int i, double ihs, double theta,
-                                             double misreg, double shift0, long isim, double dt,
-                                             double ptsdx, double orig, int &ii, float &ff) {
-    double dout, oout;
-    axis_map(L, isx, ihs, theta, misreg, shift0, isim, dt, ptsdx, orig, dout, oout);
-    screen_wrap(L, isx, i, dout, oout, ii, ff);
-}
-
 // Static surface OPD (powfs.opdadd, maos/wfsgrad.c:228-230) and per-step
 // piston/tip/tilt (loc_add_ptt, maos/wfsgrad.c:243-256: TTM/FSM commands) of
 // one subaperture grid with origin (x0, y0):
@@ -2519,7 +2511,7 @@ __device__ __forceinline__ void lf_chain(const LfArgs &a, int c, int &iwfs, int 
     iwfs = (c / a.nwvl) % a.nwfs;
     isa = c / (a.nwvl * a.nwfs);
 }
-// the passes run in dynamic LDS of lf_lds() bytes
+// the passes run in dynamic LDS (lf_launch sets its bytes)
 extern __shared__ float2 lfs[];
 
 // pass A: embed the field-band rows and FFT them along x
