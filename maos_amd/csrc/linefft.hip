@@ -26,13 +26,64 @@
 constexpr int LX_MAXST = 12; // most stages
 constexpr int LX_E = 18;     // most points a thread holds in a stage
 struct LinePlan {
-    int n, nst, cap;         // cap: fewest points per thread of any stage
+    int n, nst, cap;         // cap: points per thread that set the block (at most any stage's)
     int S;                   // LDS stride of a line (odd): its most padded form
     // of stage i: radix, n / radix, n / (span radix); pad of its output and
     // the step between the points of a butterfly of its input in LDS
     int rad[LX_MAXST], nb[LX_MAXST], ts[LX_MAXST], pad[LX_MAXST], rstep[LX_MAXST];
     const float2 *tw;        // exp(-2 pi i t / n), t < n
 };
+
+// butterflies of radix R that a thread holds
+__host__ __device__ constexpr int lx_per(int R) { return LX_E / R; }
+// LDS cycles of the 64 lanes (8 bytes each, 64 banks of 4) that reach the
+// elements at(lane): the most lanes on one pair of banks, counted per 32
+template <class F>
+constexpr int lx_conflicts(int lanes, F at) {
+    int worst = 0, cnt[32] = {};
+    for (int i = 0; i < lanes; i++) {
+        const int c = ++cnt[at(i) % 32];
+        worst = c > worst ? c : worst;
+    }
+    return worst;
+}
+constexpr int lx_min(int a, int b) { return a < b ? a : b; }
+// the plan of the radices rad[0 .. nst)
+constexpr void lx_fill(LinePlan &P, const int *rad, int nst) {
+    int n = 1;
+    for (int i = 0; i < nst; i++) n *= rad[i];
+    P.n = n;
+    P.nst = nst;
+    P.cap = LX_E;
+    int Ns = 1, S = n;
+    for (int i = 0; i < nst; i++) {
+        const int R = rad[i];
+        P.rad[i] = R;
+        P.nb[i] = n / R;
+        P.ts[i] = n / (Ns * R);
+        P.cap = lx_min(P.cap, R * lx_per(R));
+        if (i > 0) P.rstep[i] = P.nb[i] + P.pad[i - 1] * (P.nb[i] / Ns);
+        if (i + 1 < nst) {
+            // the pad with the fewest conflicts of the stage's writes and the
+            // next one's reads (lanes at consecutive butterflies)
+            const int Nx = Ns * R, nbx = n / rad[i + 1];
+            int least = 1 << 30;
+            for (int p = 0; p <= 17; p++) {
+                const int c =
+                    lx_conflicts(lx_min(64, P.nb[i]), [=](int j) { return j / Ns * (Nx + p) + j % Ns; }) +
+                    lx_conflicts(lx_min(64, nbx), [=](int j) { return j + j / Nx * p; });
+                if (c < least) {
+                    least = c;
+                    P.pad[i] = p;
+                }
+            }
+            const int padded = n + P.pad[i] * (n / Nx);
+            S = padded > S ? padded : S;
+        }
+        Ns *= R;
+    }
+    P.S = S | 1;
+}
 
 // a plan in constant memory: its run-time indexed arrays are scalar loads
 typedef const __attribute__((address_space(4))) LinePlan *LxPlan;
@@ -41,8 +92,6 @@ typedef const __attribute__((address_space(4))) LinePlan *LxPlan;
     ((LxPlan)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() +    \
               offsetof(ARGS, MEMBER)))
 
-// butterflies of radix R that a thread holds
-__host__ __device__ constexpr int lx_per(int R) { return LX_E / R; }
 // element i of a uniform base (32-bit offset, the base in scalar registers)
 template <class T>
 __device__ __forceinline__ const T &lx_at(const T *base, int i) {
@@ -228,25 +277,77 @@ enum LxMap { LX_ROW = 0, LX_COL };
 struct LxLines {
     int L, lgL; // lines, log2 L (LX_COL)
 };
-template <int MAP>
+// a / b: by the compiler where b is a constant of the plan (CT), else from its
+// reciprocal
+template <bool CT>
+__device__ __forceinline__ int lx_div(int a, int b, float rb) {
+    if constexpr (CT) return (int)((unsigned)a / (unsigned)b);
+    else return qdiv(a, b, rb);
+}
+template <int MAP, bool CT>
 __device__ __forceinline__ void lx_item(int it, int nb, float rnb, const LxLines &g, int &l, int &j) {
     if constexpr (MAP == LX_COL) {
         l = it & (g.L - 1);
         j = it >> g.lgL;
     } else {
-        l = qdiv(it, nb, rnb);
+        l = lx_div<CT>(it, nb, rnb);
         j = it - __mul24(l, nb);
     }
 }
-// Stage i (radix R, span Ns).  FIRST reads ld(l, j, off): point j + off of
+// What a stage reads of its plan: at run time, stage i of span Ns ...
+struct LxRtStage {
+    LxPlan P;
+    int i, Ns;
+    static constexpr bool CT = false;
+    __device__ int nb() const { return P->nb[i]; }
+    __device__ int S() const { return P->S; }
+    __device__ int pad() const { return P->pad[i]; }
+    __device__ int prev_pad() const { return P->pad[i - 1]; }
+    __device__ int rstep() const { return P->rstep[i]; }
+    __device__ int ts() const { return P->ts[i]; }
+    __device__ const float2 *tw() const { return P->tw; }
+};
+// ... or constants: the plan of radices R..., of a length that kernels are
+// compiled for (tw: its twiddles)
+template <int... R>
+struct LxCt {
+    static constexpr LinePlan make() {
+        LinePlan P{};
+        const int r[] = {R...};
+        lx_fill(P, r, (int)sizeof...(R));
+        P.cap = (P.cap + 1) / 2; // (twice the threads: their stages are short, and few lines leave the chip idle)
+        return P;
+    }
+    static constexpr LinePlan P = make();
+    const float2 *tw;
+};
+template <class CP, int I>
+struct LxCtStage {
+    static constexpr int span() {
+        int s = 1;
+        for (int i = 0; i < I; i++) s *= CP::P.rad[i];
+        return s;
+    }
+    const float2 *tw_;
+    static constexpr int Ns = span();
+    static constexpr bool CT = true;
+    __device__ static constexpr int nb() { return CP::P.nb[I]; }
+    __device__ static constexpr int S() { return CP::P.S; }
+    __device__ static constexpr int pad() { return CP::P.pad[I]; }
+    __device__ static constexpr int prev_pad() { return CP::P.pad[I > 0 ? I - 1 : 0]; }
+    __device__ static constexpr int rstep() { return CP::P.rstep[I]; }
+    __device__ static constexpr int ts() { return CP::P.ts[I]; }
+    __device__ const float2 *tw() const { return tw_; }
+};
+// Stage V (radix R, span Ns).  FIRST reads ld(l, j, off): point j + off of
 // line l, off uniform; LAST hands st(l, d, off, v, slot) point d + off, off
 // uniform (slot: the thread's register slot, a constant after unrolling); the
 // others use the padded LDS lines s.  BAR: ld reads LDS that the stage
 // overwrites.
-template <int R, bool INV, bool FIRST, bool LAST, int MAP, bool BAR, class LD, class ST>
-__device__ __forceinline__ void lx_stage(float2 *s, LxPlan P, const LxLines &g, int i, int Ns, LD &ld, ST &st) {
+template <int R, bool INV, bool FIRST, bool LAST, int MAP, bool BAR, class V, class LD, class ST>
+__device__ __forceinline__ void lx_stage(float2 *s, const V P, const LxLines &g, LD &ld, ST &st) {
     constexpr int PER = lx_per(R);
-    const int nb = P->nb[i], total = g.L * nb, T = (int)blockDim.x;
+    const int nb = P.nb(), Ns = P.Ns, total = g.L * nb, T = (int)blockDim.x;
     const float rnb = 1.f / (float)nb, rns = 1.f / (float)Ns;
     float2 v[PER][R];
 #pragma unroll
@@ -254,15 +355,15 @@ __device__ __forceinline__ void lx_stage(float2 *s, LxPlan P, const LxLines &g, 
         const int it = (int)threadIdx.x + p * T;
         if (it < total) {
             int l, j;
-            lx_item<MAP>(it, nb, rnb, g, l, j);
+            lx_item<MAP, V::CT>(it, nb, rnb, g, l, j);
             if constexpr (FIRST) {
 #pragma unroll
                 for (int r = 0; r < R; r++) v[p][r] = ld(l, j, r * nb);
             } else {
-                const int q = qdiv(j, Ns, rns);
-                const float2 *x = s + __mul24(l, P->S) + j + __mul24(q, P->pad[i - 1]);
+                const int q = lx_div<V::CT>(j, Ns, rns);
+                const float2 *x = s + __mul24(l, P.S()) + j + __mul24(q, P.prev_pad());
 #pragma unroll
-                for (int r = 0; r < R; r++) v[p][r] = x[r * P->rstep[i]];
+                for (int r = 0; r < R; r++) v[p][r] = x[r * P.rstep()];
             }
         }
     }
@@ -272,14 +373,14 @@ __device__ __forceinline__ void lx_stage(float2 *s, LxPlan P, const LxLines &g, 
         const int it = (int)threadIdx.x + p * T;
         if (it < total) {
             int l, j;
-            lx_item<MAP>(it, nb, rnb, g, l, j);
-            const int q = FIRST ? j : qdiv(j, Ns, rns), k = FIRST ? 0 : j - __mul24(q, Ns);
+            lx_item<MAP, V::CT>(it, nb, rnb, g, l, j);
+            const int q = FIRST ? j : lx_div<V::CT>(j, Ns, rns), k = FIRST ? 0 : j - __mul24(q, Ns);
             if constexpr (!FIRST) {
-                const int t = __mul24(k, P->ts[i]);
+                const int t = __mul24(k, P.ts());
                 int tm = t;
 #pragma unroll
                 for (int m = 1; m < R; m++, tm += t) {
-                    const float2 w = lx_at(P->tw, tm);
+                    const float2 w = lx_at(P.tw(), tm);
                     v[p][m] = cmul(v[p][m], make_float2(w.x, INV ? -w.y : w.y));
                 }
             }
@@ -288,7 +389,7 @@ __device__ __forceinline__ void lx_stage(float2 *s, LxPlan P, const LxLines &g, 
 #pragma unroll
                 for (int r = 0; r < R; r++) st(l, __mul24(q, Ns * R) + k, r * Ns, v[p][r], p * R + r);
             } else {
-                float2 *y = s + __mul24(l, P->S) + __mul24(q, Ns * R + P->pad[i]) + k;
+                float2 *y = s + __mul24(l, P.S()) + __mul24(q, Ns * R + P.pad()) + k;
 #pragma unroll
                 for (int r = 0; r < R; r++) y[r * Ns] = v[p][r];
             }
@@ -308,19 +409,39 @@ __device__ __forceinline__ void lx_stage(float2 *s, LxPlan P, const LxLines &g, 
 // barrier only.
 template <bool INV, int MI, int MO, bool LDSIN, class LD, class ST>
 __device__ __forceinline__ void lx_fft(float2 *s, LxPlan P, const LxLines &g, LD &&ld, ST &&st) {
-#define LX_CASE(R) case R: lx_stage<R, INV, true, false, MI, LDSIN>(s, P, g, 0, 1, ld, st); break;
+#define LX_CASE(R) case R: lx_stage<R, INV, true, false, MI, LDSIN>(s, LxRtStage{P, 0, 1}, g, ld, st); break;
     switch (P->rad[0]) { LX_RADIX(LX_CASE) default: break; }
 #undef LX_CASE
     int Ns = P->rad[0], i = 1;
     for (; i < P->nst - 1; i++) {
-#define LX_CASE(R) case R: lx_stage<R, INV, false, false, LX_ROW, false>(s, P, g, i, Ns, ld, st); break;
+#define LX_CASE(R) case R: lx_stage<R, INV, false, false, LX_ROW, false>(s, LxRtStage{P, i, Ns}, g, ld, st); break;
         switch (P->rad[i]) { LX_RADIX(LX_CASE) default: break; }
 #undef LX_CASE
         Ns *= P->rad[i];
     }
-#define LX_CASE(R) case R: lx_stage<R, INV, false, true, MO, false>(s, P, g, i, Ns, ld, st); break;
+#define LX_CASE(R) case R: lx_stage<R, INV, false, true, MO, false>(s, LxRtStage{P, i, Ns}, g, ld, st); break;
     switch (P->rad[i]) { LX_CASE(1) LX_RADIX(LX_CASE) default: break; }
 #undef LX_CASE
+}
+
+// the same for a plan of constants
+template <bool INV, int MI, int MO, bool LDSIN, int I, class CP, class LD, class ST>
+__device__ __forceinline__ void lx_stages(float2 *s, const CP &P, const LxLines &g, LD &ld, ST &st) {
+    constexpr bool first = I == 0, last = I == CP::P.nst - 1;
+    lx_stage<CP::P.rad[I], INV, first, last, first ? MI : last ? MO : LX_ROW, first && LDSIN>(
+        s, LxCtStage<CP, I>{P.tw}, g, ld, st);
+    if constexpr (!last) lx_stages<INV, MI, MO, LDSIN, I + 1>(s, P, g, ld, st);
+}
+template <bool INV, int MI, int MO, bool LDSIN, int... R, class LD, class ST>
+__device__ __forceinline__ void lx_fft(float2 *s, const LxCt<R...> &P, const LxLines &g, LD &&ld, ST &&st) {
+    lx_stages<INV, MI, MO, LDSIN, 0>(s, P, g, ld, st);
+}
+// a kernel's plan: constants (T an LxCt) or p
+struct LxRt {};
+template <class T>
+__device__ __forceinline__ auto lx_pick(LxPlan p) {
+    if constexpr (std::is_same<T, LxRt>::value) return p;
+    else return T{p->tw};
 }
 
 // f(l, d, off, slot) for every point that lx_fft's last stage hands this
@@ -335,7 +456,7 @@ __device__ __forceinline__ void lx_outputs(LxPlan P, const LxLines &g, F &&f) {
             const int it = (int)threadIdx.x + p * (int)blockDim.x;                                                   \
             if (it < total) {                                                                                        \
                 int l, j;                                                                                            \
-                lx_item<MO>(it, nb, rnb, g, l, j);                                                                   \
+                lx_item<MO, false>(it, nb, rnb, g, l, j);                                                            \
                 _Pragma("unroll") for (int r = 0; r < R; r++) f(l, j, r * nb, p * R + r);                            \
             }                                                                                                        \
         }                                                                                                            \
@@ -371,14 +492,6 @@ inline void lx_search(long n, int most, std::vector<int> &cur, std::vector<int> 
             cur.pop_back();
         }
 }
-// LDS cycles of the 64 lanes (8 bytes each, 64 banks of 4) that reach the
-// elements at(lane): the most lanes on one pair of banks, counted per 32
-template <class F>
-inline int lx_conflicts(int lanes, F at) {
-    int worst = 0, cnt[32] = {};
-    for (int i = 0; i < lanes; i++) worst = std::max(worst, ++cnt[at(i) % 32]);
-    return worst;
-}
 inline bool lx_plan(long n, LinePlan &P) {
     P = LinePlan{};
     if (n < 2) return false;
@@ -391,36 +504,7 @@ inline bool lx_plan(long n, LinePlan &P) {
             if (n % k == 0) r = k;
         best = {(int)n / r, r};
     }
-    P.n = (int)n;
-    P.nst = (int)best.size();
-    P.cap = LX_E;
-    int Ns = 1, S = (int)n;
-    for (int i = 0; i < P.nst; i++) {
-        const int R = best[i];
-        P.rad[i] = R;
-        P.nb[i] = (int)n / R;
-        P.ts[i] = (int)n / (Ns * R);
-        P.cap = std::min(P.cap, R * lx_per(R));
-        if (i > 0) P.rstep[i] = P.nb[i] + P.pad[i - 1] * (P.nb[i] / Ns);
-        if (i + 1 < P.nst) {
-            // the pad with the fewest conflicts of the stage's writes and the
-            // next one's reads (lanes at consecutive butterflies)
-            const int Nx = Ns * R, nbx = (int)n / best[i + 1];
-            int least = 1 << 30;
-            for (int p = 0; p <= 17; p++) {
-                const int c = lx_conflicts(std::min(64, P.nb[i]),
-                                           [&](int j) { return j / Ns * (Nx + p) + j % Ns; }) +
-                              lx_conflicts(std::min(64, nbx), [&](int j) { return j + j / Nx * p; });
-                if (c < least) {
-                    least = c;
-                    P.pad[i] = p;
-                }
-            }
-            S = std::max(S, (int)n + P.pad[i] * ((int)n / Nx));
-        }
-        Ns *= R;
-    }
-    P.S = S | 1;
+    lx_fill(P, best.data(), (int)best.size());
     return true;
 }
 inline void lx_twiddles(long n, std::vector<float2> &tw) {
@@ -429,5 +513,8 @@ inline void lx_twiddles(long n, std::vector<float2> &tw) {
         tw.push_back(make_float2((float)std::cos(a), (float)std::sin(a)));
     }
 }
-// threads of a block of L lines (a multiple of 64)
-inline int lx_threads(const LinePlan &P, int L) { return (int)(((long)L * P.n + P.cap - 1) / P.cap + 63) / 64 * 64; }
+// threads of a block of L lines: a multiple of 64, at most 1024 (8192 points,
+// the most of a block, take 820 at the fewest points of any stage, 10)
+inline int lx_threads(const LinePlan &P, int L) {
+    return std::min(1024, (int)(((long)L * P.n + P.cap - 1) / P.cap + 63) / 64 * 64);
+}

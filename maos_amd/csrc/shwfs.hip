@@ -2515,6 +2515,7 @@ __device__ __forceinline__ void lf_chain(const LfArgs &a, int c, int &iwfs, int 
 extern __shared__ float2 lfs[];
 
 // pass A: embed the field-band rows and FFT them along x
+template <class PN>
 __global__ __launch_bounds__(1024) void k_lf_a(LfArgs a) {
     const int n = a.nwvf, nxsa = a.nxsa, skip = (n - nxsa) / 2, L = a.L, S = a.pn.S;
     const LxLines ln{L, a.lgL};
@@ -2541,7 +2542,7 @@ __global__ __launch_bounds__(1024) void k_lf_a(LfArgs a) {
     __syncthreads();
     float2 *out = a.b1 + ((long)c * nxsa + g * L) * n;
     lx_fft<false, LX_ROW, LX_ROW, true>(
-        lfs, LX_PLAN(LfArgs, pn), ln,
+        lfs, lx_pick<PN>(LX_PLAN(LfArgs, pn)), ln,
         [&](int l, int j, int off) LX_INLINE {
             const int e = j + off;
             return lx_sel(l < nrow && e >= skip && e < skip + nxsa, lfs[__mul24(l, S) + j + off]);
@@ -2555,6 +2556,7 @@ __global__ __launch_bounds__(1024) void k_lf_a(LfArgs a) {
 // PSF is real, so columns 2q and 2q+1 go through one complex FFT as z = a + i
 // b, and A[k] = (Z[k] + conj Z[m-k]) / 2, B[k] = (Z[k] - conj Z[m-k]) / 2i are
 // kept for k <= m/2 only.
+template <class PN, class PM>
 __global__ __launch_bounds__(1024) void k_lf_b(LfArgs a) {
     const int n = a.nwvf, m = a.notf, nxsa = a.nxsa, skip = (n - nxsa) / 2, L = a.L, mh = m / 2 + 1, h = n / 2;
     const LxLines ln{L, a.lgL}, l2{L / 2, a.lgL - 1};
@@ -2566,7 +2568,7 @@ __global__ __launch_bounds__(1024) void k_lf_b(LfArgs a) {
     const float sc = a.psf_scale;
     float *psf = reinterpret_cast<float *>(lfs);
     lx_fft<false, LX_COL, LX_COL, false>(
-        lfs, LX_PLAN(LfArgs, pn), ln,
+        lfs, lx_pick<PN>(LX_PLAN(LfArgs, pn)), ln,
         [&](int l, int j, int off) LX_INLINE {
             const int e = j + off;
             const bool ok = x0 + l < n && e >= skip && e < skip + nxsa;
@@ -2578,7 +2580,7 @@ __global__ __launch_bounds__(1024) void k_lf_b(LfArgs a) {
         });
     __syncthreads();
     lx_fft<false, LX_COL, LX_COL, true>(
-        lfs, LX_PLAN(LfArgs, pm), l2,
+        lfs, lx_pick<PM>(LX_PLAN(LfArgs, pm)), l2,
         [&](int l, int j, int off) LX_INLINE {
             const int e = j + off;
             return lx_sel(e < h || e >= m - h, lfs[__mul24(l, S2) + j + off]);
@@ -2601,7 +2603,7 @@ __global__ __launch_bounds__(1024) void k_lf_b(LfArgs a) {
 // columns: B3 is [nx][m/2+1].  UPLINK: the chains are (WFS, wavelength) LLT
 // fields and the row FFT is conj-stored as the uplink OTF lotfc over
 // uy <= m/2 (maos/wfsints.c:149-199).
-template <bool UPLINK>
+template <bool UPLINK, class PM>
 __global__ __launch_bounds__(1024) void k_lf_d(LfArgs a) {
     const int n = a.nwvf, m = a.notf, mh = m / 2 + 1, L = a.L, S = a.pm.S, h = n / 2;
     const LxLines ln{L, a.lgL};
@@ -2617,7 +2619,7 @@ __global__ __launch_bounds__(1024) void k_lf_d(LfArgs a) {
     };
     if constexpr (UPLINK) {
         float2 *lo = a.lotf + (long)c * m * m + (long)y0 * m;
-        lx_fft<false, LX_ROW, LX_ROW, false>(lfs, LX_PLAN(LfArgs, pm), ln, load, [&](int l, int d, int off, float2 v, int) LX_INLINE {
+        lx_fft<false, LX_ROW, LX_ROW, false>(lfs, lx_pick<PM>(LX_PLAN(LfArgs, pm)), ln, load, [&](int l, int d, int off, float2 v, int) LX_INLINE {
             if (l < nrow) lx_at(lo + off, __mul24(l, m) + d) = make_float2(v.x, -v.y);
         });
         return;
@@ -2634,7 +2636,7 @@ __global__ __launch_bounds__(1024) void k_lf_d(LfArgs a) {
     } else if (W.nominal) {
         nm = W.nominal + (long)isa * W.nom_sa + (long)y0 * m;
     }
-    lx_fft<false, LX_ROW, LX_ROW, false>(lfs, LX_PLAN(LfArgs, pm), ln, load, [&](int l, int d, int off, float2 v, int) LX_INLINE {
+    lx_fft<false, LX_ROW, LX_ROW, false>(lfs, lx_pick<PM>(LX_PLAN(LfArgs, pm)), ln, load, [&](int l, int d, int off, float2 v, int) LX_INLINE {
         const int i = __mul24(l, m) + d;
         if (l < nrow) {
             if (lo) {
@@ -2653,7 +2655,7 @@ __global__ __launch_bounds__(1024) void k_lf_d(LfArgs a) {
     });
     __syncthreads();
     lx_fft<true, LX_ROW, LX_ROW, true>(
-        lfs, LX_PLAN(LfArgs, pm), ln, [&](int l, int j, int off) LX_INLINE { return lfs[__mul24(l, S) + j + off]; },
+        lfs, lx_pick<PM>(LX_PLAN(LfArgs, pm)), ln, [&](int l, int j, int off) LX_INLINE { return lfs[__mul24(l, S) + j + off]; },
         [&](int l, int d, int off, float2 v, int) LX_INLINE { lfs[__mul24(l, S) + d + off] = v; });
     __syncthreads();
     float2 *out = a.b3 + (long)c * a.maxnx * mh + y0;
@@ -2735,6 +2737,7 @@ __global__ __launch_bounds__(256) void k_lf_e(LfArgs a) {
 // FFTs, two columns a and b per complex line as a + i b (their values are
 // real: the imaginary parts at 0 and m/2 do not count), the part past m/2 by
 // conjugation; the sampled rows are picked from LDS.
+template <class PM>
 __global__ __launch_bounds__(1024) void k_lf_e_fft(LfArgs a) {
     const int m = a.notf, h = m / 2, mh = h + 1, L = a.L, S = a.pm.S;
     const LxLines ln{L, a.lgL};
@@ -2746,7 +2749,7 @@ __global__ __launch_bounds__(1024) void k_lf_e_fft(LfArgs a) {
     if (nx <= 0) return; // uniform: no sampled column in this group
     const float2 *in = a.b3 + ((long)c * a.maxnx + x0) * mh;
     lx_fft<true, LX_ROW, LX_ROW, false>(
-        lfs, LX_PLAN(LfArgs, pm), ln,
+        lfs, lx_pick<PM>(LX_PLAN(LfArgs, pm)), ln,
         [&](int l, int j, int off) LX_INLINE {
             const int e = j + off, k = e <= h ? e : m - e;
             const bool ok0 = 2 * l < nx, ok1 = 2 * l + 1 < nx;
@@ -3235,14 +3238,55 @@ bool supported(long notf, long nxsa, long embfac) {
     return (notf == 64 && nxsa == 32 && embfac == 2) || (notf == 32 && nxsa == 16 && embfac == 2);
 }
 
-// pass q of the large-field form (0..3: A, B, D, E; 4: the uplink's D; 5: E of
-// long columns, 6: of many rows)
-const void *lf_kernel(int q) {
-    const void *k[7] = {reinterpret_cast<const void *>(&k_lf_a), reinterpret_cast<const void *>(&k_lf_b),
-                        reinterpret_cast<const void *>(&k_lf_d<false>), reinterpret_cast<const void *>(&k_lf_e),
-                        reinterpret_cast<const void *>(&k_lf_d<true>), reinterpret_cast<const void *>(&k_lf_e_wave),
-                        reinterpret_cast<const void *>(&k_lf_e_fft)};
+// Lengths that the large-field passes are compiled for: the fields (PN) and
+// OTFs (PM) of the configured low-order NGS, tip-tilt and padded LGS powfs.
+// Constants take the plan's loads, the choice of each stage's radix and half of
+// the index arithmetic out of a pass, which is what bounds one of few lines (the
+// chip has one or two waves of it a SIMD): a step of one chain of 960^2 in
+// 1024^2 79 -> 57 us, of 24 of 480^2 in 512^2 121 -> 102, of 1,968 of 128^2 248
+// -> 216, and with twice the threads (LxCt) 53, 95 and 205.
+#define LF_LENGTHS(X)                                                                                                \
+    X(LF_CT(16, 6), LF_CT(12, 10))                                                                                   \
+    X(LF_CT(16, 8), LF_CT(16, 8))                                                                                    \
+    X(LF_CT(16, 6, 5), LF_CT(8, 8, 8))                                                                               \
+    X(LF_CT(10, 12, 8), LF_CT(16, 8, 8))
+#define LF_CT(...) LxCt<__VA_ARGS__>
+template <class PN, class PM>
+const void *lf_kernel_t(int q) {
+    const void *k[7] = {reinterpret_cast<const void *>(&k_lf_a<PN>),        reinterpret_cast<const void *>(&k_lf_b<PN, PM>),
+                        reinterpret_cast<const void *>(&k_lf_d<false, PM>), reinterpret_cast<const void *>(&k_lf_e),
+                        reinterpret_cast<const void *>(&k_lf_d<true, PM>),  reinterpret_cast<const void *>(&k_lf_e_wave),
+                        reinterpret_cast<const void *>(&k_lf_e_fft<PM>)};
     return k[q];
+}
+// pass q of the large-field form (0..3: A, B, D, E; 4: the uplink's D; 5: E of
+// long columns, 6: of many rows) for a field of n and an OTF of m points
+template <class PN, class PM>
+bool lf_compiled(int q, int n, int m, const void *&k) { // pass q of these lengths is this one (A: of n, B: both, others: of m)
+    const bool is = (q > 1 || n == PN::P.n) && (q == 0 || m == PM::P.n);
+    if (is) k = lf_kernel_t<PN, PM>(q);
+    return is;
+}
+const void *lf_kernel(int q, int n, int m) {
+    const void *k = nullptr;
+#define LF_KERNEL(...) if (lf_compiled<__VA_ARGS__>(q, n, m, k)) return k;
+    LF_LENGTHS(LF_KERNEL)
+#undef LF_KERNEL
+    return lf_kernel_t<LxRt, LxRt>(q);
+}
+// the passes' plan of length n
+template <class PN, class PM>
+bool lf_compiled_plan(long n, LinePlan &P) {
+    if (n == PN::P.n) P = PN::P;
+    else if (n == PM::P.n) P = PM::P;
+    else return false;
+    return true;
+}
+bool lf_plan(long n, LinePlan &P) {
+#define LF_PLAN(...) if (lf_compiled_plan<__VA_ARGS__>(n, P)) return true;
+    LF_LENGTHS(LF_PLAN)
+#undef LF_PLAN
+    return lx_plan(n, P);
 }
 // lines per block of a pass over nlines lines of n points in each of nchain
 // chains: a power of two up to 16 of at most 16 points for each of `threads`
@@ -3264,7 +3308,7 @@ bool lf_supported(long notf, long nxsa, long embfac) {
     LinePlan a, b;
     const long nwvf = nxsa * embfac;
     return nxsa >= 16 && nxsa % 16 == 0 && embfac >= 1 && nwvf % 2 == 0 && notf % 2 == 0 && notf >= nwvf &&
-           notf <= MX_LF_MAXN && lx_plan(nwvf, a) && lx_plan(notf, b);
+           notf <= MX_LF_MAXN && lf_plan(nwvf, a) && lf_plan(notf, b);
 }
 
 // FP32 -> BF16 with round-to-nearest-even (finite inputs)
@@ -3498,12 +3542,12 @@ int mx_wfsgrad_init_batch(mx_wfsgrad_t **out, const mx_powfs_t *p, const mx_wfs_
         // blocks of 512 threads (an autotune candidate) may exceed the default
         // dynamic LDS limit
         for (int q : {0, 1, 2, 4, 6})
-            if (hipFuncSetAttribute(lf_kernel(q), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess) {
+            if (hipFuncSetAttribute(lf_kernel(q, (int)h->nwvf, (int)N), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess) {
                 mx_wfsgrad_free(h);
                 return set_err(MX_EHIP, "the large-field kernels' LDS size could not be set");
             }
-        lx_plan(h->nwvf, h->lf_pn);
-        lx_plan(N, h->lf_pm);
+        lf_plan(h->nwvf, h->lf_pn);
+        lf_plan(N, h->lf_pm);
         lx_twiddles(h->nwvf, lf_tw);
         const size_t nt_n = lf_tw.size();
         lx_twiddles(N, lf_tw);
@@ -4126,17 +4170,17 @@ StepLaunch lf_launch(const mx_wfsgrad_t *h, LfArgs &u, int q, bool up) {
             const int npair = (u.maxnx + 1) / 2;
             u.L = lf_lines(m, npair, u.nchain, T, 1);
             u.lgL = ilog2c(u.L);
-            StepLaunch e{lf_kernel(6), dim3((unsigned)((npair + u.L - 1) / u.L * u.nchain)),
+            StepLaunch e{lf_kernel(6, n, m), dim3((unsigned)((npair + u.L - 1) / u.L * u.nchain)),
                          dim3((unsigned)lx_threads(u.pm, u.L)), &u};
             e.lds = (unsigned)(sizeof(float2) * u.L * u.pm.S);
             return e;
         }
         if (mh > MX_LF_ESHORT) {
-            StepLaunch e{lf_kernel(5), dim3((unsigned)waves), dim3(256), &u};
+            StepLaunch e{lf_kernel(5, n, m), dim3((unsigned)waves), dim3(256), &u};
             return e;
         }
         const int XG = lf_ecols(mh);
-        StepLaunch e{lf_kernel(3), dim3((unsigned)((u.maxnx + XG - 1) / XG * u.nchain)), dim3(256), &u};
+        StepLaunch e{lf_kernel(3, n, m), dim3((unsigned)((u.maxnx + XG - 1) / XG * u.nchain)), dim3(256), &u};
         return e;
     }
     const int nlines = q == 0 ? u.nxsa : q == 1 ? n : mh;
@@ -4148,7 +4192,7 @@ StepLaunch lf_launch(const mx_wfsgrad_t *h, LfArgs &u, int q, bool up) {
         threads = std::max(threads, lx_threads(u.pm, u.L / 2));
         elems = std::max(elems, u.L / 2 * u.pm.S);
     }
-    StepLaunch e{lf_kernel(up ? 4 : q), dim3((unsigned)((nlines + u.L - 1) / u.L * u.nchain)), dim3((unsigned)threads), &u};
+    StepLaunch e{lf_kernel(up ? 4 : q, n, m), dim3((unsigned)((nlines + u.L - 1) / u.L * u.nchain)), dim3((unsigned)threads), &u};
     e.lds = (unsigned)(sizeof(float2) * elems);
     return e;
 }
