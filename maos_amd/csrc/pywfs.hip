@@ -26,17 +26,23 @@
 // time, with a transpose between the passes, the three launches of a 784^2
 // grid took 26 us a position, mostly latency (196 blocks), and those of a
 // 2916^2 grid 191 us, a seventh of them in the transpose.  In batches a step of
-// the 784^2 grid (32 positions) takes 290 us against 960, one of the 2916^2 grid
-// 4.1 ms against 6.6 (rows 2.9 TB/s of PSF, mask and scratch; the column pass is
-// bound by the 16-byte runs that it reads of each row).
+// the 784^2 grid (32 positions) takes 295 us with its read-out against 960, one
+// of the 2916^2 grid 3.8 ms against 6.6.  Three positions of 2916^2: the rows 121
+// us (131 MB read, 189 MB written: 2.6 TB/s; VALU issue 62%, waits 46% of the
+// wave cycles), the columns 197 us (239 MB read where the planes hold 204, 37 MB
+// written: 1.3 TB/s; VALU issue 33%): not the bytes, but the chain of each
+// position's loads, stages and barriers at the three blocks of six waves a CU
+// that its lines leave.
 constexpr int MX_PY_MAXN = 4096;
 constexpr int MX_PY_MAXSIDE = 4;
 constexpr int MX_PY_LDS = 96 * 1024;        // most LDS of a block's lines (71,216 bytes for two columns of 4050 points)
 constexpr int MX_PY_MAXB = 32;              // most positions of a batch
 // bytes of scratch planes that a batch aims at (at least one plane): the
-// rows' mask and PSF reads and the sum's update are shared by a batch (784^2:
-// 32 MB 384 us a step, 64 MB 336, 160 MB 297; 2916^2: 64 MB 4293, 140 MB 4061,
-// 280 MB 3981)
+// rows' mask and PSF reads and the sum's update are shared by a batch.  Queued
+// steps in us: 784^2: 32 MB 321, 64 MB 264, 140 MB 246, 205 MB and more (all 32
+// positions) 227; 2916^2: one plane 3,940, two to four (140, 205, 280 MB) 3,690,
+// 3,710 and 3,650, eight (560 MB) 3,360: kept at what one sensor may hold, not at
+// the fastest
 constexpr long MX_PY_SCRATCH = 256L << 20;
 constexpr int MX_PY_MAXSPLIT = 8;           // most partial pupil intensities
 
@@ -64,7 +70,8 @@ struct PyArgs {
 };
 extern __shared__ float2 pyl[];
 
-// (four waves a SIMD: the 18 points a thread holds and their twiddles)
+// (the 18 points a thread holds and their twiddles: five to seven waves a SIMD;
+// PY_REAL, once a step, four, with the splits' loads all in flight)
 template <int MODE>
 __global__ __launch_bounds__(1024) void k_py_rows(PyArgs a) {
     const int n = a.n, L = a.L, S = a.plan.S, tid = threadIdx.x;
@@ -358,9 +365,9 @@ void pywfs_release(mx_pywfs_t *h) {
 
 // Lines per block: as many as 4096 points hold (a power of two, at most 16), so
 // that a block has about 256 threads and a CU several blocks; columns at least
-// two, since a run of L columns is what the pass reads of a row.  (784^2: 4
-// columns 305 us a step, 8 336, 16 377; 2916^2: 2 columns 4293, 1 4344, 4
-// 4299.)
+// two, since a run of L columns is what the pass reads of a row.  (Queued steps
+// of 784^2: 2 columns 252 us, 4 227, 8 243, 16 257; of 2916^2: 1 column 3,810, 2
+// 3,690, 4 4,360.)
 int py_row_lines(long n) {
     int L = 16;
     while (L > 1 && L * n > 4096) L /= 2;

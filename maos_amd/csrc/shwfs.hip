@@ -2446,10 +2446,11 @@ __global__ __launch_bounds__(256) void k_llt_acorr(LltAcorrArgs a) {
 // of a real function, so half the plane is enough.
 //
 // Measured against five passes that wrote the PSF out and transformed it back
-// in (ping-pong Stockham stages of radix 8 at most, the plan read at run
-// time): 24 chains of 480^2 in 512^2 165 -> 85 us (1.1 TB/s of B1 and B2),
-// one chain of 960^2 in 1024^2 61 -> 55 us (latency of the passes, one or two
-// blocks a CU), 1,968 chains of 128^2 with their uplink 808 -> 220 us.
+// in (ping-pong Stockham stages of radix 8 at most): 24 chains of 480^2 in 512^2
+// 165 -> 78 us (pass A 1.3 TB/s, B 1.3, D 0.9, at 23 to 44% VALU issue: latency),
+// one chain of 960^2 in 1024^2 61 -> 37 us (latency of the passes, one or two
+// blocks a CU), 1,968 chains of 128^2 with their uplink 808 -> 196 us (D reads 151
+// MB and B writes 63 at 2.3 to 2.5 TB/s and 62 to 72% VALU issue).
 constexpr int MX_LF_MAXN = 1024;
 constexpr int MX_LF_THREADS = 512; // most threads per block the choice of L aims at (128, 256 or 512)
 constexpr int MX_LF_MAXS = 128;    // most sampled rows / columns kept (else the full image)

@@ -16,8 +16,8 @@ GRAD_TOL_MAS = 0.1
 # positions: one; fewer than the splits; one batch exactly (32); one more than
 # a batch; two rings (17 + 34 positions) and two wavelengths, whose weights differ
 @pytest.mark.parametrize("pos,ring,nwvl", [(1, 1, 1), (5, 1, 1), (32, 1, 1), (33, 1, 1), (34, 2, 1), (6, 2, 2)])
-# grids of 100 = 10 10, 126 = 14 9 (126 columns in groups of 16), 196 = 14 14 and 490 = 10 7 7
-@pytest.mark.parametrize("D,dx,N", [(2.0, 1 / 16, 100), (2.56, 1 / 16, 126), (4.0, 1 / 16, 196), (5.0, 1 / 32, 490)])
+# grids of 100 = 10 10, 126 = 18 7 (126 columns in groups of 16), 196 = 7 7 4 and 486 = 9 9 6
+@pytest.mark.parametrize("D,dx,N", [(2.0, 1 / 16, 100), (2.56, 1 / 16, 126), (4.0, 1 / 16, 196), (5.0, 1 / 32, 486)])
 def test_pywfs_batches(D, dx, N, pos, ring, nwvl):
     from maos_amd import engine
     from maos_amd.pywfs import Pywfs, PywfsCfg
