@@ -4160,14 +4160,17 @@ int mx_dm2gpu(const mx_atm_layer_t *dms, int ndm) { return mx_dm2gpu_real(0, dms
 
 } // extern "C"
 
+// blocks of pass E's wave form (four waves each), and whether it goes by line FFTs
+long lf_ewaves(const LfArgs &u) { return ((long)u.maxny * u.maxnx + 3) / 4 * u.nchain; }
+bool lf_efft(const LfArgs &u) {
+    return u.maxny > MX_LF_EROWS || (u.notf / 2 + 1 > MX_LF_ESHORT && lf_ewaves(u) > MX_LF_EWAVES);
+}
 // launch of pass q (0..3: A, B, D, E; up: the uplink's D) over u's chains,
 // its lines per block set in u
 StepLaunch lf_launch(const mx_wfsgrad_t *h, LfArgs &u, int q, bool up) {
     const int n = u.nwvf, m = u.notf, mh = m / 2 + 1, T = h->lf_threads;
     if (q == 3) {
-        const long outs = (long)u.maxny * u.maxnx, waves = (outs + 3) / 4 * u.nchain; // blocks of four waves
-        const bool fft = u.maxny > MX_LF_EROWS || (mh > MX_LF_ESHORT && waves > MX_LF_EWAVES);
-        if (fft) {
+        if (lf_efft(u)) {
             const int npair = (u.maxnx + 1) / 2;
             u.L = lf_lines(m, npair, u.nchain, T, 1);
             u.lgL = ilog2c(u.L);
@@ -4177,7 +4180,7 @@ StepLaunch lf_launch(const mx_wfsgrad_t *h, LfArgs &u, int q, bool up) {
             return e;
         }
         if (mh > MX_LF_ESHORT) {
-            StepLaunch e{lf_kernel(5, n, m), dim3((unsigned)waves), dim3(256), &u};
+            StepLaunch e{lf_kernel(5, n, m), dim3((unsigned)lf_ewaves(u)), dim3(256), &u};
             return e;
         }
         const int XG = lf_ecols(mh);
@@ -4852,7 +4855,7 @@ int plan_step(mx_wfsgrad_t *h, long isim, double dt, StepPlan &sp) {
     h->lotf_last = cur;
     if (nl > MX_MAXLAUNCH) return set_err(MX_EINVAL, "internal: %d kernels in a step", nl);
     sp.nl = nl;
-    sp.key = (1 << 30) | (ndm ? 1 << 27 : 0) | (N == 64 ? 1 : 0) | (llt ? 2 : 0) | (h->lf ? 4 : 0) |
+    sp.key = (1 << 30) | (h->lf && lf_efft(h->arg_lf[3]) ? 1 << 28 : 0) | (ndm ? 1 << 27 : 0) | (N == 64 ? 1 : 0) | (llt ? 2 : 0) | (h->lf ? 4 : 0) |
              (direct ? 8 : 0) | (variant << 4) | (o.tiles > 1 ? 1 << 7 : 0) | (opd_nx << 8) |
              (h->lf ? h->lf_threads << 14 : 0) | (h->cfg.sigmatch == 2 ? 1 << 25 : 0) |
              ((mf || fftform) && h->d_etf2_t[0] ? 1 << 24 : 0) | (fftform ? 1 << 6 : 0) |

@@ -64,3 +64,42 @@ def test_wide_detectors(nxsa, embfac, notf, pixpsa, spacing, wvls, order, nwfs):
         print("wfs %d ints %.2e grad %.2e mas" % (i, e_int, e_g), flush=True)
         assert e_int <= INTS_TOL and e_g <= GRAD_TOL_MAS
     eng.close()
+
+
+@pytest.mark.parametrize("notf", [128, 270])
+def test_detector_tables_change_between_graph_steps(notf):
+    """An engine that steps as a graph and is given the tables of a wider
+    detector (18 sampled rows, then 34, transformed instead of summed) gives
+    what an engine made for that detector gives."""
+    from maos_amd import _lib, configs, engine
+    from maos_amd._lib import check, dptr, lptr
+    from maos_amd.powfs import PTYPE_COG, AS2RAD, AperCfg, AtmCfg, Powfs, PowfsCfg, SimCfg, genatm
+    print("case: OTF %d, detector tables replaced" % notf, flush=True)
+    nxsa, dsa, wvl = 64, 1.0, 1.25e-6
+
+    def powfs(spacing):
+        pcfg = PowfsCfg(order=2, dsa=dsa, dx=dsa / nxsa, saat=0.3, hs=math.inf, embfac=2, wvl=[wvl], wvlwts=[1.0],
+                        pixpsa=17, pixtheta=spacing * wvl * nxsa / (dsa * notf) / AS2RAD, pixblur=0.3, notf=notf,
+                        phytype=PTYPE_COG, sigmatch=1, siglev=1000.0)
+        return Powfs(AperCfg(2.0, 0.2), pcfg, SimCfg(dt=1.0 / 800))
+    near, far = powfs(1.0), powfs(2.1)
+    engine.init(0)
+    engine.dm2gpu([])
+    engine.atm2gpu(genatm(AtmCfg(r0=0.15, L0=30.0, ht=[0.0], wt=[1.0], ws=[8.0], wddeg=[30.0], dx=1.0 / 64, nx=256,
+                                 seeds=[3])))
+    wfs = configs.wfs_specs(dict(powfs=near.cfg, wfs=[dict(thetax=4e-5, thetay=0.0)]), near)
+    eng, ref = engine.WfsGrad(near, wfs), engine.WfsGrad(far, wfs)
+    eng.set_graph(True)
+    for i in range(3):
+        eng.queue(i, 1.0 / 800)
+    before = eng.sync(0)[1]
+    check(_lib.hip().mx_wfsgrad_set_dtf(eng.h, 0, dptr(far.nominal[0]), far.npix, notf * notf, lptr(far.si_pp[0]),
+                                        lptr(far.si_pi[0]), dptr(far.si_px[0])))
+    for i in (7, 8):
+        eng.queue(i, 1.0 / 800)
+        ref.queue(i, 1.0 / 800)
+        got, want = eng.sync(0)[1], ref.sync(0)[1]
+        assert np.array_equal(got, want)
+    assert not np.array_equal(before, want)
+    eng.close()
+    ref.close()
