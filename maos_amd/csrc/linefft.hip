@@ -26,7 +26,7 @@
 constexpr int LX_MAXST = 12; // most stages
 constexpr int LX_E = 18;     // most points a thread holds in a stage
 struct LinePlan {
-    int n, nst, cap;         // cap: points per thread that set the block (at most any stage's)
+    int n, nst, cap;         // cap: fewest points per thread of any stage
     int S;                   // LDS stride of a line (odd): its most padded form
     // of stage i: radix, n / radix, n / (span radix); pad of its output and
     // the step between the points of a butterfly of its input in LDS
@@ -315,7 +315,6 @@ struct LxCt {
         LinePlan P{};
         const int r[] = {R...};
         lx_fill(P, r, (int)sizeof...(R));
-        P.cap = (P.cap + 1) / 2; // (twice the threads: their stages are short, and few lines leave the chip idle)
         return P;
     }
     static constexpr LinePlan P = make();
@@ -443,6 +442,12 @@ __device__ __forceinline__ auto lx_pick(LxPlan p) {
     if constexpr (std::is_same<T, LxRt>::value) return p;
     else return T{p->tw};
 }
+// and its LDS stride of a line
+template <class T>
+__device__ __forceinline__ int lx_stride(const LinePlan &p) {
+    if constexpr (std::is_same<T, LxRt>::value) return p.S;
+    else return T::P.S;
+}
 
 // f(l, d, off, slot) for every point that lx_fft's last stage hands this
 // thread by map MO (the last span is the line, so d is the butterfly)
@@ -513,8 +518,9 @@ inline void lx_twiddles(long n, std::vector<float2> &tw) {
         tw.push_back(make_float2((float)std::cos(a), (float)std::sin(a)));
     }
 }
-// threads of a block of L lines: a multiple of 64, at most 1024 (8192 points,
-// the most of a block, take 820 at the fewest points of any stage, 10)
-inline int lx_threads(const LinePlan &P, int L) {
-    return std::min(1024, (int)(((long)L * P.n + P.cap - 1) / P.cap + 63) / 64 * 64);
+// threads of a block of L lines: a multiple of 64 (8192 points, the most of a
+// block, take 820 at the fewest points of any stage, 10), mul times as many if
+// they fit a block
+inline int lx_threads(const LinePlan &P, int L, int mul = 1) {
+    return std::min(1024, mul * ((int)(((long)L * P.n + P.cap - 1) / P.cap + 63) / 64 * 64));
 }

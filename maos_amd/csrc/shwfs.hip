@@ -2518,7 +2518,7 @@ extern __shared__ float2 lfs[];
 // pass A: embed the field-band rows and FFT them along x
 template <class PN>
 __global__ __launch_bounds__(1024) void k_lf_a(LfArgs a) {
-    const int n = a.nwvf, nxsa = a.nxsa, skip = (n - nxsa) / 2, L = a.L, S = a.pn.S;
+    const int n = a.nwvf, nxsa = a.nxsa, skip = (n - nxsa) / 2, L = a.L, S = lx_stride<PN>(a.pn);
     const LxLines ln{L, a.lgL};
     int g, c, iwfs, isa, iwvl;
     lf_unit(a, (nxsa + L - 1) / L, g, c);
@@ -2561,7 +2561,7 @@ template <class PN, class PM>
 __global__ __launch_bounds__(1024) void k_lf_b(LfArgs a) {
     const int n = a.nwvf, m = a.notf, nxsa = a.nxsa, skip = (n - nxsa) / 2, L = a.L, mh = m / 2 + 1, h = n / 2;
     const LxLines ln{L, a.lgL}, l2{L / 2, a.lgL - 1};
-    const int S2 = a.pm.S;
+    const int S2 = lx_stride<PM>(a.pm);
     int g, c;
     lf_unit(a, (n + L - 1) / L, g, c);
     const int x0 = g * L;
@@ -2606,7 +2606,7 @@ __global__ __launch_bounds__(1024) void k_lf_b(LfArgs a) {
 // uy <= m/2 (maos/wfsints.c:149-199).
 template <bool UPLINK, class PM>
 __global__ __launch_bounds__(1024) void k_lf_d(LfArgs a) {
-    const int n = a.nwvf, m = a.notf, mh = m / 2 + 1, L = a.L, S = a.pm.S, h = n / 2;
+    const int n = a.nwvf, m = a.notf, mh = m / 2 + 1, L = a.L, S = lx_stride<PM>(a.pm), h = n / 2;
     const LxLines ln{L, a.lgL};
     int g, c, iwfs, isa, iwvl;
     lf_unit(a, (mh + L - 1) / L, g, c);
@@ -2740,7 +2740,7 @@ __global__ __launch_bounds__(256) void k_lf_e(LfArgs a) {
 // conjugation; the sampled rows are picked from LDS.
 template <class PM>
 __global__ __launch_bounds__(1024) void k_lf_e_fft(LfArgs a) {
-    const int m = a.notf, h = m / 2, mh = h + 1, L = a.L, S = a.pm.S;
+    const int m = a.notf, h = m / 2, mh = h + 1, L = a.L, S = lx_stride<PM>(a.pm);
     const LxLines ln{L, a.lgL};
     int g, c, iwfs, isa, iwvl;
     lf_unit(a, ((a.maxnx + 1) / 2 + L - 1) / L, g, c);
@@ -3245,13 +3245,23 @@ bool supported(long notf, long nxsa, long embfac) {
 // the index arithmetic out of a pass, which is what bounds one of few lines (the
 // chip has one or two waves of it a SIMD): a step of one chain of 960^2 in
 // 1024^2 79 -> 57 us, of 24 of 480^2 in 512^2 121 -> 102, of 1,968 of 128^2 248
-// -> 216, and with twice the threads (LxCt) 53, 95 and 205.
+// -> 216, and with twice the threads (their stages are short, and few lines leave
+// the chip idle) 53, 95 and 205.  Passes whose plan is read at run time are
+// slower with twice the threads (24 chains of 480^2 121 -> 124 us).
 #define LF_LENGTHS(X)                                                                                                \
     X(LF_CT(16, 6), LF_CT(12, 10))                                                                                   \
     X(LF_CT(16, 8), LF_CT(16, 8))                                                                                    \
     X(LF_CT(16, 6, 5), LF_CT(8, 8, 8))                                                                               \
     X(LF_CT(10, 12, 8), LF_CT(16, 8, 8))
 #define LF_CT(...) LxCt<__VA_ARGS__>
+// pass q of the large-field form (0..3: A, B, D, E; 4: the uplink's D; 5: E of
+// long columns, 6: of many rows): its kernel, the plans that it runs and how many
+// times the threads that they need it gets
+struct LfPass {
+    const void *k;
+    LinePlan pn, pm;
+    int mul;
+};
 template <class PN, class PM>
 const void *lf_kernel_t(int q) {
     const void *k[7] = {reinterpret_cast<const void *>(&k_lf_a<PN>),        reinterpret_cast<const void *>(&k_lf_b<PN, PM>),
@@ -3260,34 +3270,18 @@ const void *lf_kernel_t(int q) {
                         reinterpret_cast<const void *>(&k_lf_e_fft<PM>)};
     return k[q];
 }
-// pass q of the large-field form (0..3: A, B, D, E; 4: the uplink's D; 5: E of
-// long columns, 6: of many rows) for a field of n and an OTF of m points
 template <class PN, class PM>
-bool lf_compiled(int q, int n, int m, const void *&k) { // pass q of these lengths is this one (A: of n, B: both, others: of m)
+bool lf_compiled(int q, int n, int m, LfPass &p) { // pass q of these lengths is this one (A: of n, B: both, others: of m)
     const bool is = (q > 1 || n == PN::P.n) && (q == 0 || m == PM::P.n);
-    if (is) k = lf_kernel_t<PN, PM>(q);
+    if (is) p = {lf_kernel_t<PN, PM>(q), PN::P, PM::P, 2};
     return is;
 }
-const void *lf_kernel(int q, int n, int m) {
-    const void *k = nullptr;
-#define LF_KERNEL(...) if (lf_compiled<__VA_ARGS__>(q, n, m, k)) return k;
-    LF_LENGTHS(LF_KERNEL)
-#undef LF_KERNEL
-    return lf_kernel_t<LxRt, LxRt>(q);
-}
-// the passes' plan of length n
-template <class PN, class PM>
-bool lf_compiled_plan(long n, LinePlan &P) {
-    if (n == PN::P.n) P = PN::P;
-    else if (n == PM::P.n) P = PM::P;
-    else return false;
-    return true;
-}
-bool lf_plan(long n, LinePlan &P) {
-#define LF_PLAN(...) if (lf_compiled_plan<__VA_ARGS__>(n, P)) return true;
-    LF_LENGTHS(LF_PLAN)
-#undef LF_PLAN
-    return lx_plan(n, P);
+LfPass lf_pass(int q, const LinePlan &pn, const LinePlan &pm) {
+    LfPass p;
+#define LF_PASS(...) if (lf_compiled<__VA_ARGS__>(q, pn.n, pm.n, p)) return p;
+    LF_LENGTHS(LF_PASS)
+#undef LF_PASS
+    return {lf_kernel_t<LxRt, LxRt>(q), pn, pm, 1};
 }
 // lines per block of a pass over nlines lines of n points in each of nchain
 // chains: a power of two up to 16 of at most 16 points for each of `threads`
@@ -3309,7 +3303,7 @@ bool lf_supported(long notf, long nxsa, long embfac) {
     LinePlan a, b;
     const long nwvf = nxsa * embfac;
     return nxsa >= 16 && nxsa % 16 == 0 && embfac >= 1 && nwvf % 2 == 0 && notf % 2 == 0 && notf >= nwvf &&
-           notf <= MX_LF_MAXN && lf_plan(nwvf, a) && lf_plan(notf, b);
+           notf <= MX_LF_MAXN && lx_plan(nwvf, a) && lx_plan(notf, b);
 }
 
 // FP32 -> BF16 with round-to-nearest-even (finite inputs)
@@ -3540,15 +3534,16 @@ int mx_wfsgrad_init_batch(mx_wfsgrad_t **out, const mx_powfs_t *p, const mx_wfs_
     h->lf = lf;
     std::vector<float2> lf_tw;
     if (lf) {
+        lx_plan(h->nwvf, h->lf_pn);
+        lx_plan(N, h->lf_pm);
         // blocks of 512 threads (an autotune candidate) may exceed the default
         // dynamic LDS limit
         for (int q : {0, 1, 2, 4, 6})
-            if (hipFuncSetAttribute(lf_kernel(q, (int)h->nwvf, (int)N), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) != hipSuccess) {
+            if (hipFuncSetAttribute(lf_pass(q, h->lf_pn, h->lf_pm).k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    96 * 1024) != hipSuccess) {
                 mx_wfsgrad_free(h);
                 return set_err(MX_EHIP, "the large-field kernels' LDS size could not be set");
             }
-        lf_plan(h->nwvf, h->lf_pn);
-        lf_plan(N, h->lf_pm);
         lx_twiddles(h->nwvf, lf_tw);
         const size_t nt_n = lf_tw.size();
         lx_twiddles(N, lf_tw);
@@ -4169,34 +4164,24 @@ bool lf_efft(const LfArgs &u) {
 // its lines per block set in u
 StepLaunch lf_launch(const mx_wfsgrad_t *h, LfArgs &u, int q, bool up) {
     const int n = u.nwvf, m = u.notf, mh = m / 2 + 1, T = h->lf_threads;
-    if (q == 3) {
-        if (lf_efft(u)) {
-            const int npair = (u.maxnx + 1) / 2;
-            u.L = lf_lines(m, npair, u.nchain, T, 1);
-            u.lgL = ilog2c(u.L);
-            StepLaunch e{lf_kernel(6, n, m), dim3((unsigned)((npair + u.L - 1) / u.L * u.nchain)),
-                         dim3((unsigned)lx_threads(u.pm, u.L)), &u};
-            e.lds = (unsigned)(sizeof(float2) * u.L * u.pm.S);
-            return e;
-        }
-        if (mh > MX_LF_ESHORT) {
-            StepLaunch e{lf_kernel(5, n, m), dim3((unsigned)lf_ewaves(u)), dim3(256), &u};
-            return e;
-        }
+    const bool efft = q == 3 && lf_efft(u);
+    const LfPass p = lf_pass(q < 3 ? (up ? 4 : q) : efft ? 6 : mh > MX_LF_ESHORT ? 5 : 3, u.pn, u.pm);
+    if (q == 3 && !efft) {
         const int XG = lf_ecols(mh);
-        StepLaunch e{lf_kernel(3, n, m), dim3((unsigned)((u.maxnx + XG - 1) / XG * u.nchain)), dim3(256), &u};
-        return e;
+        const long blocks = mh > MX_LF_ESHORT ? lf_ewaves(u) : (u.maxnx + XG - 1) / XG * u.nchain;
+        return StepLaunch{p.k, dim3((unsigned)blocks), dim3(256), &u};
     }
-    const int nlines = q == 0 ? u.nxsa : q == 1 ? n : mh;
+    const int nlines = q == 0 ? u.nxsa : q == 1 ? n : q == 2 ? mh : (u.maxnx + 1) / 2;
     // (pass B pairs columns; pass D writes runs of L along uy)
-    u.L = lf_lines(q == 2 ? m : n, nlines, u.nchain, T, q == 0 ? 1 : 2);
+    u.L = lf_lines(q < 2 ? n : m, nlines, u.nchain, T, q == 0 || q == 3 ? 1 : 2);
     u.lgL = ilog2c(u.L);
-    int threads = lx_threads(q == 2 ? u.pm : u.pn, u.L), elems = u.L * (q == 2 ? u.pm.S : u.pn.S);
+    const LinePlan &P = q < 2 ? p.pn : p.pm;
+    int threads = lx_threads(P, u.L, p.mul), elems = u.L * P.S;
     if (q == 1) {
-        threads = std::max(threads, lx_threads(u.pm, u.L / 2));
-        elems = std::max(elems, u.L / 2 * u.pm.S);
+        threads = std::max(threads, lx_threads(p.pm, u.L / 2, p.mul));
+        elems = std::max(elems, u.L / 2 * p.pm.S);
     }
-    StepLaunch e{lf_kernel(up ? 4 : q, n, m), dim3((unsigned)((nlines + u.L - 1) / u.L * u.nchain)), dim3((unsigned)threads), &u};
+    StepLaunch e{p.k, dim3((unsigned)((nlines + u.L - 1) / u.L * u.nchain)), dim3((unsigned)threads), &u};
     e.lds = (unsigned)(sizeof(float2) * elems);
     return e;
 }
