@@ -2457,13 +2457,14 @@ constexpr int MX_LF_MAXS = 128;    // most sampled rows / columns kept (else the
 constexpr int MX_LF_ESUB = 8;      // lanes that share one output of pass E
 constexpr int MX_LF_ESHORT = 129;  // longest column (m/2 + 1) of its staged form
 // Most sampled rows for which pass E sums its outputs directly.  The direct
-// sums cost ny terms a column and are FP64; the line FFTs cost the same for any
-// ny.  Imaging of a step in us, direct / FFT, for detectors whose pixels are two
-// samples apart:
-//                       24 rows   32 rows   48 rows   64 rows   whole image
-//   12 chains of 512^2   72 / 75   74 / 75   84 / 78   94 / 80   1393 / 124
-//   one of 1024^2        51 / 56   51 / 56   54 / 58   56 / 59    851 / 93
-//   12 of 128^2          48 / 39   52 / 39   62 / 41   71 / 42
+// sums cost ny terms a column; the line FFTs cost the same for any ny.  Imaging
+// of a step in us, direct / FFT, for detectors whose pixels are two samples apart:
+//                       16 rows   24 rows   32 rows   48 rows   64 rows   whole image
+//   12 chains of 512^2   50 / 50   52 / 51   55 / 51   63 / 53   73 / 54   1364 / 88
+//   one of 1024^2        38 / 39   38 / 39   38 / 40   41 / 41   43 / 42    835 / 69
+//   12 of 128^2          35 / 28   40 / 28   44 / 28   54 / 30   63 / 31
+// The line lies past the detectors of the configured sensors (12 to 17 rows),
+// whose images keep the FP64 sums: short columns would gain up to 16 us there.
 constexpr int MX_LF_EROWS = 32;
 constexpr long MX_LF_EWAVES = 1L << 21; // most blocks of the direct sums of long columns (a launch has 2^24)
 // complex elements of pass E's column buffer
